@@ -12,7 +12,7 @@
 // VGPRs) of one row and one 32-block, which is exactly one MX block, and the
 // byte of its scale register selected by op_sel.
 //
-// Two kernels share one design: a 256 x 256 macro tile per workgroup of 8
+// Two large-tile kernels share one design: a 256 x 256 macro tile per workgroup of 8
 // waves (4 x 2, each 64 x 128, two waves per SIMD) with fp32 accumulators;
 // a persistent schedule, one workgroup per CU walking tiles pid, pid + grid,
 // ...; and a ring of LDS stage slots filled by direct-to-LDS loads
@@ -23,15 +23,17 @@
 // compiler cannot prove that ring slots do not alias and would otherwise
 // wait for every outstanding load before each LDS read.
 //
-//  * gemm_f4f4_mx16_kernel (K-major E8M0 scales, K % 256 == 0; the fast
-//    path): v_mfma_scale_f32_16x16x128_f8f6f4 on 128-byte stage rows in a
+//  * gemm_f4f4_mx16_kernel (K-major E8M0 scales; the fast path):
+//    v_mfma_scale_f32_16x16x128_f8f6f4 on 128-byte stage rows in a
 //    2-slot ring of 64 KiB stages.  Whole 128-byte rows matter: the
 //    direct-to-LDS path is limited by the number of L2 requests (measured:
 //    19 B/clk per CU for 16 rows x 64 B per load instruction, 36 B/clk for
 //    8 rows x 128 B).
-//  * gemm_f4f4_kernel (fp32 or row-major E8M0 scales, or K % 256 != 0):
-//    v_mfma_scale_f32_32x32x64_f8f6f4 on 64-byte stage rows in a 3- or
-//    4-slot ring.
+//  * gemm_f4f4_kernel (fp32 or row-major E8M0 scales, or rows of 2^19 bytes
+//    and more): v_mfma_scale_f32_32x32x64_f8f6f4 on 64-byte stage rows in a
+//    3- or 4-slot ring.
+// Outputs with too few 256 x 256 tiles for the CUs run gemm_f4f4_tile_kernel
+// (K-major E8M0 scales), the same instruction on smaller tiles.
 //
 // Per stage and wave the MFMAs of one K-step run while the fragments of the
 // next are read from LDS between them.  Once the slot has been read, one
@@ -697,7 +699,7 @@ __global__ __launch_bounds__(512, 1) void gemm_f4f4_mx16_kernel(GemmArgs g) {
     const int tiles_m = (int)((g.M + BM - 1) / BM), tiles_n = (int)((g.N + BN - 1) / BN);
     const int tiles = tiles_m * tiles_n;
     const int my_tiles = (tiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
-    const int nk = (int)(g.K / (2 * BKB));
+    const int nk = (int)((g.K + 2 * BKB - 1) / (2 * BKB));  // the last stage may hold 128 codes (see Panel)
 
     const int t = threadIdx.x;
     const int lane = t & 63;
@@ -726,6 +728,10 @@ __global__ __launch_bounds__(512, 1) void gemm_f4f4_mx16_kernel(GemmArgs g) {
         m0 = (int64_t)tm * BM;
         n0 = (int64_t)tn * BN;
     };
+    // K % 256 == 128: the last stage's second half lies past K.  Its scale
+    // slice lies past the scale array, so A's and B's scales there are loaded
+    // as byte 0 (2^-127 each) and the codes under them -- the next row's, or
+    // zeros past the panel's last byte -- add at most 2^-240.
     struct Panel {
         const uint8_t *p;
         int64_t n;
@@ -733,8 +739,8 @@ __global__ __launch_bounds__(512, 1) void gemm_f4f4_mx16_kernel(GemmArgs g) {
     Panel pA, pB, pS;
     const int64_t sstep = NSL * s_ld * 4;            // scale bytes one stage advances
     auto set_refill_origin = [&](int64_t m0, int64_t n0) {
-        pA = Panel{g.a + m0 * g.lda, min(g.M - m0, (int64_t)BM) * g.lda};
-        pB = Panel{g.b + n0 * g.ldb, min(g.N - n0, (int64_t)BN) * g.ldb};
+        pA = Panel{g.a + m0 * g.lda, (min(g.M - m0, (int64_t)BM) - 1) * g.lda + g.K / 2};
+        pB = Panel{g.b + n0 * g.ldb, (min(g.N - n0, (int64_t)BN) - 1) * g.ldb + g.K / 2};
         // rows past the operand read other scales or zeros: their products
         // only reach outputs that are not stored
         const int64_t sb0 = (s_j * s_ld + (s_b ? n0 : m0)) * 4;
@@ -756,7 +762,7 @@ __global__ __launch_bounds__(512, 1) void gemm_f4f4_mx16_kernel(GemmArgs g) {
     };
     auto make_desc_s = [&](int kt) {
         const int64_t so = (int64_t)kt * sstep;
-        rsS = buf_rsrc(pS.p + so, (uint64_t)(pS.n - so));
+        rsS = buf_rsrc(pS.p + so, (uint64_t)max(pS.n - so, (int64_t)0));
     };
     auto issue_op = [&](int s, int q) {
         if (q < 2 * XA) {
@@ -1023,6 +1029,259 @@ __global__ __launch_bounds__(512, 1) void gemm_f4f4_mx16_kernel(GemmArgs g) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
+// ---------------------------------------------------------------------------
+// The 16 x 16 x 128 pipeline on smaller tiles, one tile per workgroup of 4
+// waves (2 x 2), for outputs whose 256 x 256 tiles leave compute units idle.
+// A tile is 32 TM x 32 TN; per wave TM x TN accumulator tiles of 16 x 16.
+// Each output sums the same 32-blocks in the same order as in
+// gemm_f4f4_mx16_kernel, so the tile size does not change its bits.
+//
+// What bounds it: with one or two waves per SIMD and a few hundred KiB of
+// operands per tile it waits on the loads of a stage (a stage of a 128 x 128
+// tile is 512 matrix-core cycles, an L2 or HBM round trip two to four times
+// that), so the ring is as deep as the LDS allows for one workgroup per CU
+// (two where the tile is small): S - 1 stages of loads are in flight while
+// one is multiplied.  Four more waves issue the loads: a wave's instructions
+// issue in order, so an MFMA behind a load that waits for a place in the
+// memory pipeline waits too (3000x2048x8192 on 192 x 128 tiles: 35.2 us with
+// the MFMA waves loading, 30.1 with loader waves).
+//
+// Schedule per stage: the MFMAs of K-step 0 run with the reads of K-step 1's
+// fragments between them; then the wave's reads of the slot are complete, one
+// barrier frees it and publishes the next stage; the MFMAs of K-step 1 run
+// with the reads of the next stage's scales and first fragments between
+// them, while the loader waves refill the slot.
+//
+// K % 256 == 128: the last stage's second half is handled as in
+// gemm_f4f4_mx16_kernel.  Refills past the last stage use an empty descriptor
+// (zeros, no memory traffic), which keeps the outstanding-load count constant.
+constexpr int f4_tile_lds(int tm, int tn, int s) {
+    return s * ((tm + tn) * 32 * 128 + 2 * (((tm + 1) / 2) * 256 + 64 + ((tn + 1) / 2) * 256 + 64));
+}
+template <int TM, int TN, int S, int CT>
+__global__ __launch_bounds__(512, 2) void gemm_f4f4_tile_kernel(GemmArgs g) {
+    using namespace f4;
+    constexpr int BM_ = 32 * TM, BN_ = 32 * TN;      // tile: 2 x 2 waves of 16 TM x 16 TN
+    constexpr int BKB = 128, CPR = 8, RPI = 64 / CPR;
+    constexpr int NWV = 4;
+    constexpr int XA = BM_ / (NWV * RPI), XB = BN_ / (NWV * RPI);  // 16-byte DMA slots per lane and operand
+    static_assert(XA * NWV * RPI == BM_ && XB * NWV * RPI == BN_, "whole DMA instructions");
+    // scales: 64 rows of one slice per 4-byte DMA, shared out over the waves
+    // (the last ones repeat a load when the count is not a multiple of 4)
+    constexpr int SGA = (BM_ + 63) / 64, SGB = (BN_ + 63) / 64, NSG = 2 * (SGA + SGB);
+    constexpr int XS = (NSG + NWV - 1) / NWV;
+    constexpr int L = XA + XB + XS;                  // loads per lane per stage
+    constexpr int SLA = SGA * 256 + 64, SLB = SGB * 256 + 64;  // slice strides: +64 B, other banks for lane groups 2-3
+    constexpr int OFF_B = BM_ * BKB, OFF_SA = OFF_B + BN_ * BKB, OFF_SB = OFF_SA + 2 * SLA;
+    constexpr int SLOT = OFF_SB + 2 * SLB;
+    static_assert(SLOT % 16 == 0 && S * SLOT <= 160 * 1024 && S * SLOT == f4_tile_lds(TM, TN, S), "LDS");
+    static_assert((S - 1) * L < 64, "vmcnt is 6 bits");
+    constexpr int NMF = TM * TN, NRD = TM + TN;
+    // LDS reads go out over the first NRM MFMAs of a K-step: the rest cover
+    // their latency
+    constexpr int NRM = NMF * 3 / 4;
+    __shared__ __attribute__((aligned(16))) uint8_t ring[S * SLOT];
+
+    const int tiles_m = (int)((g.M + BM_ - 1) / BM_), tiles_n = (int)((g.N + BN_ - 1) / BN_);
+    const int t = threadIdx.x;
+    const int lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wm = (wave >> 1) & 1, wn = wave & 1;
+    const int r16 = lane & 15, grp = lane >> 4;
+    int tm, tn;
+    tile_coords((int)blockIdx.x, make_tile_map(tiles_m, tiles_n, GROUP_M), tm, tn);
+    const int64_t m0 = (int64_t)tm * BM_, n0 = (int64_t)tn * BN_;
+    const int nk = (int)((g.K + 255) / 256);
+
+    // ---- DMA: load i of this lane reads row (i * 4 + wave) * 8 + lane / 8 of
+    // the panel; the chunk swizzle of those rows does not depend on i
+    const int lw = wave & 3;  // loader wave
+    const int drow0 = lw * RPI + lane / CPR;
+    const int chunk = (lane % CPR) ^ f4_swz<CPR>(drow0);
+    const uint32_t offA0 = (uint32_t)(drow0 * g.lda + chunk * 16), offB0 = (uint32_t)(drow0 * g.ldb + chunk * 16);
+    const uint32_t stepA = (uint32_t)(NWV * RPI * g.lda), stepB = (uint32_t)(NWV * RPI * g.ldb);
+    const uint8_t *pA = g.a + m0 * g.lda, *pB = g.b + n0 * g.ldb;
+    const int64_t nA = (min(g.M - m0, (int64_t)BM_) - 1) * g.lda + g.K / 2;
+    const int64_t nB = (min(g.N - n0, (int64_t)BN_) - 1) * g.ldb + g.K / 2;
+    const uint64_t sbytes_a = (uint64_t)((g.K / 128 - 1) * g.ld_sa + g.M) * 4;
+    const uint64_t sbytes_b = (uint64_t)((g.K / 128 - 1) * g.ld_sb + g.N) * 4;
+    const uint32_t ring0 = lds_u32(&ring[0]);
+
+    v4i_rsrc rsA, rsB;
+    int kt_load = 0;
+    auto make_desc = [&](int kt) {
+        const int64_t ko = (int64_t)kt * BKB;
+        const bool past = kt >= nk;
+        rsA = buf_rsrc(pA + (past ? 0 : ko), past ? 0 : (uint64_t)(nA - ko));
+        rsB = buf_rsrc(pB + (past ? 0 : ko), past ? 0 : (uint64_t)(nB - ko));
+        kt_load = kt;
+    };
+    // one load (q = 0 .. L-1) of stage kt_load into the slot at byte offset so
+    auto issue_op = [&](uint32_t so, int q) {
+        if (q < XA) {
+            dma_x4_at(offA0, q, stepA, rsA, ring0 + so + (q * NWV + lw) * 1024);
+        } else if (q < XA + XB) {
+            const int i = q - XA;
+            dma_x4_at(offB0, i, stepB, rsB, ring0 + so + OFF_B + (i * NWV + lw) * 1024);
+        } else {
+            // 64-row group e of (A slice 0, A slice 1, B slice 0, B slice 1)
+            int e = (q - XA - XB) * NWV + lw;
+            e = e < NSG ? e : NSG - 1;
+            const bool to_b = e >= 2 * SGA;
+            e = to_b ? e - 2 * SGA : e;
+            const int per = to_b ? SGB : SGA;
+            const int sl = e >= per ? 1 : 0, gi = e - sl * per;
+            const int64_t row0 = (to_b ? n0 : m0) + gi * 64, ld = to_b ? g.ld_sb : g.ld_sa;
+            const int64_t b0 = (((int64_t)kt_load * 2 + sl) * ld + row0) * 4;
+            const int64_t left = (int64_t)(to_b ? sbytes_b : sbytes_a) - b0;
+            const bool past = left <= 0 || kt_load >= nk;
+            const uint8_t *base = reinterpret_cast<const uint8_t *>(to_b ? g.sb : g.sa);
+            dma_x1((uint32_t)lane * 4, buf_rsrc(base + (past ? 0 : b0), past ? 0 : (uint64_t)left),
+                   ring0 + so + (to_b ? OFF_SB + sl * SLB : OFF_SA + sl * SLA) + gi * 256);
+        }
+    };
+
+    // ---- fragment and scale reads, as in gemm_f4f4_mx16_kernel
+    uint32_t loff[2];
+    for (int st = 0; st < 2; ++st) loff[st] = (uint32_t)(r16 * BKB + (((2 * grp + st) ^ ((r16 >> 1) & 7)) << 4));
+    const uint32_t soffA = (uint32_t)(OFF_SA + (grp >> 1) * SLA + (wm * 16 * TM + r16) * 4 + 2 * (grp & 1));
+    const uint32_t soffB = (uint32_t)(OFF_SB + (grp >> 1) * SLB + (wn * 16 * TN + r16) * 4 + 2 * (grp & 1));
+    v4f acc[TM][TN];
+    v4i fa[2][TM], fb[2][TN];
+    uint32_t scA[TM], scB[TN], nxA[TM], nxB[TN];
+    auto rd_frag = [&](uint32_t so, int st, int q) {
+        const uint32_t base = q < TM ? (uint32_t)(wm * 16 * TM + q * 16) * BKB
+                                     : (uint32_t)OFF_B + (uint32_t)(wn * 16 * TN + (q - TM) * 16) * BKB;
+        const u32x4 v = *reinterpret_cast<const u32x4 *>(&ring[0] + so + base + loff[st]);
+        const v4i f = v4i{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
+        if (q < TM) fa[st][q] = f;
+        else fb[st][q - TM] = f;
+    };
+    auto rd_scale = [&](uint32_t so, int q) {
+        if (q < TM) nxA[q] = *reinterpret_cast<const uint16_t *>(&ring[0] + so + soffA + q * 64);
+        else nxB[q - TM] = *reinterpret_cast<const uint16_t *>(&ring[0] + so + soffB + (q - TM) * 64);
+    };
+
+    // ---- loader waves: fill the ring, then refill each slot after the
+    // barrier that frees it
+    if (wave >= NWV) {
+        __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+        for (int p = 0; p < S; ++p) {
+            make_desc(p);
+#pragma unroll
+            for (int q = 0; q < L; ++q) issue_op(p * SLOT, q);
+        }
+        wait_vm_barrier<(S - 1) * L>();
+        uint32_t so = 0;
+        for (int kt = 0; kt < nk; ++kt) {
+            make_desc(kt + S);
+            wait_vm_barrier<(S - 2) * L>();
+#pragma unroll
+            for (int q = 0; q < L; ++q) issue_op(so, q);
+            so = so + SLOT == S * SLOT ? 0 : so + SLOT;
+        }
+        // no load may still be writing this workgroup's LDS when it exits
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        return;
+    }
+
+    // ---- MFMA waves
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    asm volatile("s_barrier" ::: "memory");
+#pragma unroll
+    for (int q = 0; q < NRD; ++q) rd_scale(0, q);
+#pragma unroll
+    for (int q = 0; q < NRD; ++q) rd_frag(0, 0, q);
+
+    uint32_t so = 0;
+    for (int kt = 0; kt < nk; ++kt) {
+        const uint32_t sn = so + SLOT == S * SLOT ? 0 : so + SLOT;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) scA[i] = nxA[i];
+#pragma unroll
+        for (int j = 0; j < TN; ++j) scB[j] = nxB[j];
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+            if (st == 1) {
+                // this wave's reads of the slot are complete; past the
+                // barrier the slot may be refilled and stage kt + 1 has landed
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int idx = 0; idx < NMF; ++idx) {
+                const int i = idx / TN, j = idx % TN;
+                acc[i][j] = mfma_scale_f4_16(fa[st][i], fb[st][j], acc[i][j], 4, 4, st, (int)scA[i], st, (int)scB[j]);
+                if (st == 0) {
+#pragma unroll
+                    for (int r = idx * NRD / NRM; r < (idx + 1) * NRD / NRM; ++r)
+                        if (r < NRD) rd_frag(so, 1, r);
+                } else {
+#pragma unroll
+                    for (int r = idx * 2 * NRD / NRM; r < (idx + 1) * 2 * NRD / NRM; ++r) {
+                        if (r < NRD) rd_scale(sn, r);
+                        else if (r < 2 * NRD) rd_frag(sn, 0, r - NRD);
+                    }
+                }
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        so = sn;
+    }
+
+    // ---- epilogue: as in gemm_f4f4_mx16_kernel, whole 16-byte stores where
+    // the rows are aligned and the columns inside C
+    const bool vec_c = ((reinterpret_cast<uintptr_t>(g.c) & 15) == 0) && (g.ldc % 8 == 0);
+    const int q = lane & 3;
+    const int64_t rb = m0 + wm * 16 * TM, cb = n0 + wn * 16 * TN;
+    if constexpr (CT != LSMX_F32 && TN % 2 == 0) {
+        if (vec_c) {
+            const bool odd = (lane & 4) != 0;
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                const int64_t row = rb + 16 * i + 4 * grp + q;
+#pragma unroll
+                for (int jp = 0; jp < TN / 2; ++jp) {
+                    const float x0[4] = {acc[i][2 * jp][0], acc[i][2 * jp][1], acc[i][2 * jp][2], acc[i][2 * jp][3]};
+                    const float x1[4] = {acc[i][2 * jp + 1][0], acc[i][2 * jp + 1][1], acc[i][2 * jp + 1][2],
+                                         acc[i][2 * jp + 1][3]};
+                    const u32x4 v = pack16_rows8<CT>(x0, x1, q, odd);
+                    const int64_t col = cb + 32 * jp + (odd ? 16 : 0) + 8 * ((lane >> 3) & 1);
+                    if (row < g.M && col < g.N) {
+                        uint16_t *p = reinterpret_cast<uint16_t *>(g.c) + row * g.ldc + col;
+                        if (col + 8 <= g.N) *reinterpret_cast<u32x4 *>(p) = v;
+                        else
+#pragma unroll
+                            for (int c = 0; c < 8; ++c)
+                                if (col + c < g.N) p[c] = (uint16_t)(v[c >> 1] >> (16 * (c & 1)));
+                    }
+                }
+            }
+            return;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            float x[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+            quad_transpose(x, q);
+            const int64_t row = rb + 16 * i + 4 * grp + q, col = cb + 16 * j + (r16 & ~3);
+            if (row < g.M) {
+                if (CT == LSMX_F32 && vec_c && col + 4 <= g.N) store_c4<CT>(g.c, row * g.ldc + col, x[0], x[1], x[2], x[3]);
+                else
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        if (col + c < g.N) store_c<CT>(g.c, row * g.ldc + col + c, x[c]);
+            }
+        }
+}
+
 static int num_cus() {
     static int cus = 0;
     if (cus == 0) {
@@ -1036,7 +1295,72 @@ static int num_cus() {
     return cus;
 }
 
+template <int TM, int TN, int S>
+static hipError_t launch_tile(const GemmArgs &g, hipStream_t s) {
+    const int64_t grid = ((g.M + 32 * TM - 1) / (32 * TM)) * ((g.N + 32 * TN - 1) / (32 * TN));
+    if (g.c_dtype == LSMX_F32) hipLaunchKernelGGL((gemm_f4f4_tile_kernel<TM, TN, S, LSMX_F32>), (int)grid, 512, 0, s, g);
+    else if (g.c_dtype == LSMX_BF16) hipLaunchKernelGGL((gemm_f4f4_tile_kernel<TM, TN, S, LSMX_BF16>), (int)grid, 512, 0, s, g);
+    else hipLaunchKernelGGL((gemm_f4f4_tile_kernel<TM, TN, S, LSMX_F16>), (int)grid, 512, 0, s, g);
+    return hipGetLastError();
+}
+
+// Tile of the K-major path.  A launch costs about
+//   2 us + rounds * fix + stages * (t of every full round + t of the last one)
+// with stages of 256 codes and rounds of (CUs * workgroups per CU) tiles; a
+// last round that leaves CUs idle runs its stages faster (lo) than a full one
+// (hi), since the loads share the L2s and the fabric.  The constants (us) are
+// fits of graph-replayed launches at 28 shapes, M and N 64 .. 8192, K 512 ..
+// 8192, every tile at every shape, and pick the fastest tile or one within
+// 6% of it there.  Largest tiles are the most economical with loads and win
+// once they fill the CUs; before that the smaller ones do:
+//   M x N x K         256x256  256x128  192x128  128x128  64x128  64x64
+//   200x8192x2048        20.4     11.9     10.2      9.0     7.7    8.3 us
+//   256x2048x8192        40.5     26.4     21.7     18.3    15.0   11.7
+//   2048x2048x2048       17.7     13.2     11.6     10.9    11.6   14.6
+//   3000x2048x8192       47.9     30.2     30.1     43.8    40.2   50.2
+//   4096x2048x8192       43.2     35.4     46.0     42.7    50.6   67.3
+//   4096x4096x4096       37.4     44.1     49.0     52.5    60.0   75.6
+struct TileCost {
+    int bm, bn, per_cu;
+    float fix, lo, hi;
+};
+static const TileCost kTiles[] = {
+    {256, 256, 1, 8.5f, 1.00f, 1.60f}, {256, 128, 1, 6.0f, 0.62f, 0.86f}, {192, 128, 1, 4.2f, 0.50f, 0.72f},
+    {128, 128, 1, 3.5f, 0.43f, 0.58f}, {64, 128, 2, 2.6f, 0.36f, 0.665f}, {64, 64, 2, 2.0f, 0.27f, 0.45f},
+};
+static int pick_tile(int64_t M, int64_t N, int64_t K) {
+    const int cus = num_cus();
+    const float nk = (float)((K + 255) / 256);
+    int best = 0;
+    float tbest = 0.0f;
+    for (int i = 0; i < (int)(sizeof(kTiles) / sizeof(kTiles[0])); ++i) {
+        const TileCost &c = kTiles[i];
+        const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+        const int64_t cap = (int64_t)cus * c.per_cu, full = (tiles - 1) / cap, last = tiles - full * cap;
+        const float tl = c.per_cu == 1 ? c.lo + (c.hi - c.lo) * (float)last / (float)cap : last <= cus ? c.lo : c.hi;
+        const float t = (float)(full + 1) * c.fix + nk * ((float)full * c.hi + tl);
+        if (i == 0 || t < tbest) best = i, tbest = t;
+    }
+    return best;
+}
+
 hipError_t launch_gemm_f4f4(const GemmArgs &g, hipStream_t s) {
+    // the 16 x 16 x 128 kernels form 32 * ld * i in 24-bit multiplies
+    const bool kmajor = g.scale_fmt == LSMX_SCALE_E8M0_KMAJOR && g.lda < (1 << 19) && g.ldb < (1 << 19);
+    if (kmajor) {
+        int tile = pick_tile(g.M, g.N, g.K);
+#ifdef SWEEP
+        if (const char *e = getenv("LSMX_TILE")) tile = atoi(e);
+#endif
+        switch (tile) {
+        case 1: return launch_tile<8, 4, 3>(g, s);
+        case 2: return launch_tile<6, 4, 3>(g, s);
+        case 3: return launch_tile<4, 4, 4>(g, s);
+        case 4: return launch_tile<2, 4, 3>(g, s);
+        case 5: return launch_tile<2, 2, 4>(g, s);
+        default: break;
+        }
+    }
     const int tiles = (int)(((g.M + f4::BM - 1) / f4::BM) * ((g.N + f4::BN - 1) / f4::BN));
     const int grid = tiles < num_cus() ? tiles : num_cus();
 #define LSMX_GC(K, ...)                                                                        \
@@ -1045,14 +1369,13 @@ hipError_t launch_gemm_f4f4(const GemmArgs &g, hipStream_t s) {
         else if (g.c_dtype == LSMX_BF16) hipLaunchKernelGGL((K<__VA_ARGS__, LSMX_BF16>), grid, 512, 0, s, g); \
         else hipLaunchKernelGGL((K<__VA_ARGS__, LSMX_F16>), grid, 512, 0, s, g);                 \
     } while (0)
-    // K-major E8M0 scales and whole 256-code stages: the 16 x 16 x 128
-    // kernel, with the stage barrier before column block 4 of its second
-    // K-step.  Row-major E8M0 (one scale request per row), fp32 scales (16
-    // bytes per row per 128 codes) and K % 256 != 0 run the 32 x 32 x 64
-    // kernel on 64-byte stages in a 3- or 4-slot ring; the Python layer
-    // regroups scales to K-major before it calls, so it always takes the
-    // first path when K allows.
-    if (g.K % 256 == 0 && g.scale_fmt == LSMX_SCALE_E8M0_KMAJOR) LSMX_GC(gemm_f4f4_mx16_kernel, 4);
+    // K-major E8M0 scales: the 16 x 16 x 128 kernel, with the stage barrier
+    // before column block 4 of its second K-step.  Row-major E8M0 (one scale
+    // request per row), fp32 scales (16 bytes per row per 128 codes) and rows
+    // too long for the 16 x 16 x 128 kernels' load offsets run the 32 x 32 x
+    // 64 kernel on 64-byte stages in a 3- or 4-slot ring; the Python layer
+    // regroups scales to K-major before it calls.
+    if (kmajor) LSMX_GC(gemm_f4f4_mx16_kernel, 4);
     else if (g.scale_fmt == LSMX_SCALE_F32) LSMX_GC(gemm_f4f4_kernel, LSMX_SCALE_F32, 3);
     else if (g.scale_fmt == LSMX_SCALE_E8M0_KMAJOR) LSMX_GC(gemm_f4f4_kernel, LSMX_SCALE_E8M0_KMAJOR, 4);
     else LSMX_GC(gemm_f4f4_kernel, LSMX_SCALE_E8M0, 4);

@@ -19,7 +19,7 @@ import torch
 from . import _capi as C
 from . import fp4 as _fp4
 
-# Tile configuration of the f4 x f4 kernel that runs at K % 256 == 0
+# Tile configuration of the f4 x f4 kernel that runs large outputs
 # (csrc/gemm_f4f4.hip, gemm_f4f4_mx16_kernel), under the reference's CFG
 # keys: 256 x 256 tiles, SUB*32 = 256 K codes (two 128-code MFMA K-steps)
 # per stage, 4-row tile groups, 8 waves of 64 lanes, a 2-slot LDS ring.
