@@ -20,6 +20,7 @@
 // buffer_load ... lds from waves 0-3 only, one barrier per stage, refill
 // panels set once per tile phase, stages in pairs with compile-time slots,
 // epilogue of 16-byte fp32 stores after an in-quad transpose.
+#include <stdlib.h>
 #include "lsmx_dma.h"
 #include "lsmx_internal.h"
 #include "lsmx_sched.h"
@@ -386,6 +387,194 @@ __global__ __launch_bounds__(dr::NT, 1) void gemm_dense_ring_kernel(DenseArgs g)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
+// ---------------------------------------------------------------------------
+// The same products on smaller tiles, for outputs whose 256 x 256 tiles leave
+// compute units idle (1024 x 1024: 16 tiles a problem on 256 CUs).  One tile
+// of 64 TM x 64 TN per workgroup: 4 MFMA waves (2 x 2, TM x TN tiles of
+// 32 x 32 each) and 4 loader waves.  Each output sums the same K-steps in the
+// same order as in gemm_dense_ring_kernel, so the tile size does not change
+// its bits.
+//
+// What bounds it: a 128 x 128 stage is 32 KiB of loads for 512 matrix-core
+// cycles, less than one L2 round trip, so the ring is as deep as the LDS
+// allows (S - 1 stages in flight) and the loads come from waves of their own:
+// an MFMA never queues behind a load that waits for a place in the memory
+// pipeline.  Per stage one barrier, before the last K-step: the reads of the
+// slot are complete there, the loader waves refill it while the last K-step's
+// MFMAs run with the reads of the next stage's first fragments between them.
+// 1024 x 1024 x 4096, two products in one launch: 70 -> 25.7 us.
+template <int DT, int MODE, bool BNC, int TM, int TN, int S>
+__global__ __launch_bounds__(512, 2) void gemm_dense_tile_kernel(DenseArgs g) {
+    constexpr int P = MODE == 2 ? 2 : 1, KC = MODE == 1 ? 2 : 1;
+    constexpr int BM = 64 * TM, BN = 64 * TN, BKB = dr::BKB, CPR = dr::CPR, RPI = dr::RPI, KS = dr::KS;
+    constexpr int NLW = 4;
+    constexpr int XA = BM / (NLW * RPI), XB = BN / (NLW * RPI), L = XA + XB;  // 16-byte loads per loader lane per stage
+    // N-contiguous B: stage rows of BN columns, RPB rows per DMA instruction
+    constexpr int ROWB = BN * 2, CPB = ROWB / 16, RPB = 64 / CPB;
+    static_assert(64 / (RPB * NLW) == XB, "a stage of B is the same bytes in both layouts");
+    constexpr int OFF_B = BM * BKB, SLOT = OFF_B + BN * BKB;
+    static_assert(S * SLOT <= 160 * 1024 && (S - 1) * L < 64, "LDS, vmcnt");
+    constexpr int NMF = TM * TN, NRD = TM + TN;
+    __shared__ __attribute__((aligned(16))) uint8_t ring[S * SLOT];
+
+    const int tiles_m = (int)((g.M + BM - 1) / BM), tiles_n = (int)((g.N + BN - 1) / BN);
+    const int nkh = (int)(g.K * 2 / BKB), nk = KC * nkh;
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+
+    // tile of this workgroup, as in gemm_dense_ring_kernel's tile_of
+    int id = (int)blockIdx.x;
+    if ((gridDim.x & 7) == 0) id = (id & 7) * ((int)gridDim.x >> 3) + (id >> 3);
+    const int p = P == 2 ? (id & 1) : 0;
+    int tm, tn;
+    group_coords(P == 2 ? id >> 1 : id, make_tile_map(tiles_m, tiles_n, dr::GROUP_M), tm, tn);
+    const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
+
+    if (wave >= NLW) {
+        // ---- loader waves
+        __builtin_amdgcn_s_setprio(3);
+        const int lw = wave - NLW;
+        const int64_t lda_b = g.lda * 2, ldb_b = g.ldb * 2;
+        const int drow0 = lw * RPI + lane / CPR;
+        const uint32_t offA0 = (uint32_t)(drow0 * lda_b + ((lane % CPR) ^ dr::swz(drow0)) * 16);
+        // BNC: LDS position c of K-row r holds source chunk c ^ 4 (r & 3)
+        // (128-byte rows: ^ 4 ((r >> 1) & 1)); r's low bits do not depend on
+        // the load index
+        const int brow0 = RPB * lw + lane / CPB;
+        const int bsw = BN == 64 ? 4 * ((brow0 >> 1) & 1) : 4 * (brow0 & 3);
+        const uint32_t offB0 = BNC ? (uint32_t)(brow0 * ldb_b + (((lane % CPB) ^ bsw) << 4))
+                                   : (uint32_t)(drow0 * ldb_b + ((lane % CPR) ^ dr::swz(drow0)) * 16);
+        const uint32_t stepA = (uint32_t)(NLW * RPI * lda_b);
+        const uint32_t stepB = BNC ? (uint32_t)(RPB * NLW * ldb_b) : (uint32_t)(NLW * RPI * ldb_b);
+        const uint8_t *pa[KC], *pb[KC];
+#pragma unroll
+        for (int h = 0; h < KC; ++h) {
+            const bool second = (P == 2 && p == 1) || h == 1;
+            pa[h] = (second ? g.a1 : g.a0) + m0 * lda_b;
+            pb[h] = (second ? g.b1 : g.b0) + (BNC ? n0 * 2 : n0 * ldb_b);
+        }
+        // panels end at the operand's last element; BNC columns past N in
+        // other rows read the next row's values, whose products only reach
+        // outputs that are not stored
+        const int64_t na = (min(g.M - m0, (int64_t)BM) - 1) * lda_b + g.K * 2;
+        const int64_t nb = BNC ? (g.K - 1) * ldb_b + (g.N - n0) * 2 : (min(g.N - n0, (int64_t)BN) - 1) * ldb_b + g.K * 2;
+        const uint32_t ring0 = lds_u32(&ring[0]);
+        auto load_stage = [&](int kt, uint32_t so) __attribute__((always_inline)) {
+            const int h = KC == 2 ? (kt & 1) : 0;
+            const int kb = KC == 2 ? kt >> 1 : kt;
+            const bool past = kt >= nk;   // refills past the end: empty descriptors, zeros
+            const int64_t ao = (int64_t)kb * BKB, bo = BNC ? (int64_t)kb * 64 * ldb_b : ao;
+            const v4i_rsrc rsA = buf_rsrc((h ? pa[KC - 1] : pa[0]) + (past ? 0 : ao), past ? 0 : (uint64_t)(na - ao));
+            const v4i_rsrc rsB = buf_rsrc((h ? pb[KC - 1] : pb[0]) + (past ? 0 : bo), past ? 0 : (uint64_t)(nb - bo));
+#pragma unroll
+            for (int i = 0; i < XA; ++i) dma_x4(offA0 + i * stepA, rsA, ring0 + so + (i * NLW + lw) * 1024);
+#pragma unroll
+            for (int i = 0; i < XB; ++i) dma_x4(offB0 + i * stepB, rsB, ring0 + so + OFF_B + (i * NLW + lw) * 1024);
+        };
+#pragma unroll
+        for (int q = 0; q < S; ++q) load_stage(q, q * SLOT);
+        wait_vm_barrier<(S - 1) * L>();
+        uint32_t so = 0;
+        for (int kt = 0; kt < nk; ++kt) {
+            wait_vm_barrier<(S - 2) * L>();
+            load_stage(kt + S, so);
+            so = so + SLOT == S * SLOT ? 0 : so + SLOT;
+        }
+        // no load may still be writing this workgroup's LDS when it exits
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        return;
+    }
+
+    // ---- MFMA waves
+    const int wm = wave >> 1, wn = wave & 1;
+    const int frow = lane & 31, half = lane >> 5;
+    const int bj = lane & 15, brs = bj >> 2;
+    const int bsw = BN == 64 ? brs >> 1 : brs;
+    uint32_t bjo[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+        bjo[j] = (uint32_t)(OFF_B + (half * 32 + brs) * ROWB + (((wn * TN + j) ^ bsw) << 6) +
+                            ((2 * ((lane >> 4) & 1) + ((bj & 3) >> 1)) << 4) + (bj & 1) * 8);
+    uint32_t ro[KS];   // 128-byte rows: chunk 4 half + st of row frow
+#pragma unroll
+    for (int st = 0; st < KS; ++st) ro[st] = (uint32_t)(frow * BKB + (((4 * half + st) ^ dr::swz(frow)) << 4));
+    v16f_d acc[TM][TN];
+    v4i_d fa[2][TM], fb[2][TN];
+    auto read_frag = [&](uint32_t so, int st, int q) __attribute__((always_inline)) {
+        if (BNC && q >= TM) {
+            const uint8_t *b = &ring[0] + so + bjo[q - TM] + st * 8 * ROWB;
+            const v2i_d lo = ds_read_tr16x4(b), hi = ds_read_tr16x4(b + 4 * ROWB);
+            fb[st & 1][q - TM] = v4i_d{lo.x, lo.y, hi.x, hi.y};
+            return;
+        }
+        const uint32_t base = q < TM ? (uint32_t)((wm * TM + q) * 32) * BKB
+                                     : (uint32_t)OFF_B + (uint32_t)((wn * TN + q - TM) * 32) * BKB;
+        const u32x4 v = *reinterpret_cast<const u32x4 *>(&ring[0] + so + base + ro[st]);
+        const v4i_d f = v4i_d{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
+        if (q < TM) fa[st & 1][q] = f;
+        else fb[st & 1][q - TM] = f;
+    };
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+    asm volatile("s_barrier" ::: "memory");
+#pragma unroll
+    for (int q = 0; q < NRD; ++q) read_frag(0, 0, q);
+    uint32_t so = 0;
+    for (int kt = 0; kt < nk; ++kt) {
+        const uint32_t sn = so + SLOT == S * SLOT ? 0 : so + SLOT;
+#pragma unroll
+        for (int st = 0; st < KS; ++st) {
+            if (st == KS - 1) {
+                // this wave's reads of the slot are complete; past the
+                // barrier it may be refilled and stage kt + 1 has landed
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int idx = 0; idx < NMF; ++idx) {
+                const int i = idx / TN, j = idx % TN;
+                acc[i][j] = mfma_dense16<DT>(fa[st & 1][i], fb[st & 1][j], acc[i][j]);
+#pragma unroll
+                for (int r = idx * NRD / NMF; r < (idx + 1) * NRD / NMF; ++r)
+                    read_frag(st < KS - 1 ? so : sn, (st + 1) % KS, r);
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        so = sn;
+    }
+
+    // ---- epilogue, as in gemm_dense_ring_kernel
+    const bool vec_c = ((reinterpret_cast<uintptr_t>(g.c0) & 15) == 0) &&
+                       (P == 1 || (reinterpret_cast<uintptr_t>(g.c1) & 15) == 0) && g.ldc % 4 == 0;
+    float *c = reinterpret_cast<float *>(P == 2 && p == 1 ? g.c1 : g.c0);
+    const int q = frow & 3;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int gq = 0; gq < 4; ++gq) {
+            const int64_t row = m0 + (wm * TM + i) * 32 + 8 * gq + 4 * half + q;
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                float x[4] = {acc[i][j][4 * gq], acc[i][j][4 * gq + 1], acc[i][j][4 * gq + 2], acc[i][j][4 * gq + 3]};
+                // all four lanes of a quad take part in the exchanges
+                quad_transpose(x, q);
+                const int64_t col = n0 + (wn * TN + j) * 32 + (frow & ~3);
+                if (row < g.M && col < g.N) {
+                    if (vec_c && col + 4 <= g.N) store_c4<LSMX_F32>(c, row * g.ldc + col, x[0], x[1], x[2], x[3]);
+                    else
+#pragma unroll
+                        for (int cc = 0; cc < 4; ++cc)
+                            if (col + cc < g.N) c[row * g.ldc + col + cc] = x[cc];
+                }
+            }
+        }
+}
+
 static int num_cus_dr() {
     static int cus = 0;
     if (cus == 0) {
@@ -407,7 +596,55 @@ bool dense_ring_ok(const DenseArgs &g, int dtype) {
            g.c_dtype == LSMX_F32;
 }
 
+// Output tile (pick_tile), stages of 64 elements.  The constants (us) are fits
+// of graph-replayed launches of every tile at 17 shapes, M and N 64 .. 4096,
+// K 1024 .. 8192, one and two problems:
+//   M x N x K (products)   256x256  256x128  192x128  128x128  64x128  64x64
+//   512x512x4096     (1)      68.9     38.8     33.0     26.7    21.5   18.0 us
+//   1024x1024x4096   (2)      70.1     42.2     36.1     29.1    25.7   34.4
+//   2048x2048x2048   (1)      43.7     28.9     27.5     24.1    30.9   36.2
+//   1500x2000x4096   (2)      81.9     60.3     56.5     69.7    79.7  101.2
+//   2048x2048x8192   (2)     185.3    127.4    160.6    163.8   216.2  264.1
+//   4096x4096x4096   (1)     116.8    124.9    140.8    163.1   183.2  226.8
+static const TileCost kTiles[] = {
+    {256, 256, 1, 8.5f, 0.95f, 1.68f}, {256, 128, 1, 5.5f, 0.55f, 0.93f}, {192, 128, 1, 4.2f, 0.46f, 0.80f},
+    {128, 128, 1, 3.5f, 0.33f, 0.61f}, {64, 128, 2, 3.0f, 0.32f, 0.74f},  {64, 64, 2, 2.5f, 0.26f, 0.48f},
+};
+
+template <int TM, int TN, int S>
+static hipError_t launch_dense_tile(const DenseArgs &g, int dtype, int mode, hipStream_t s) {
+    const int64_t grid = ((g.M + 64 * TM - 1) / (64 * TM)) * ((g.N + 64 * TN - 1) / (64 * TN)) * (mode == 2 ? 2 : 1);
+#define LSMX_DT(DT, MD)                                                                                              \
+    do {                                                                                                             \
+        if (g.b_nc) hipLaunchKernelGGL((gemm_dense_tile_kernel<DT, MD, true, TM, TN, S>), dim3((unsigned)grid), dim3(512), 0, s, g); \
+        else hipLaunchKernelGGL((gemm_dense_tile_kernel<DT, MD, false, TM, TN, S>), dim3((unsigned)grid), dim3(512), 0, s, g);      \
+    } while (0)
+    if (dtype == LSMX_BF16) {
+        if (mode == 0) LSMX_DT(LSMX_BF16, 0);
+        else if (mode == 1) LSMX_DT(LSMX_BF16, 1);
+        else LSMX_DT(LSMX_BF16, 2);
+    } else {
+        if (mode == 0) LSMX_DT(LSMX_F16, 0);
+        else if (mode == 1) LSMX_DT(LSMX_F16, 1);
+        else LSMX_DT(LSMX_F16, 2);
+    }
+#undef LSMX_DT
+    return hipGetLastError();
+}
+
 hipError_t launch_gemm_dense_ring(const DenseArgs &g, int dtype, int mode, hipStream_t s) {
+    int tile = pick_tile(kTiles, g.M, g.N, mode == 2 ? 2 : 1, (mode == 1 ? 2 : 1) * g.K / 64, num_cus_dr());
+#ifdef SWEEP
+    if (const char *e = getenv("LSMX_TILE")) tile = atoi(e);
+#endif
+    switch (tile) {
+    case 1: return launch_dense_tile<4, 2, 3>(g, dtype, mode, s);
+    case 2: return launch_dense_tile<3, 2, 4>(g, dtype, mode, s);
+    case 3: return launch_dense_tile<2, 2, 4>(g, dtype, mode, s);
+    case 4: return launch_dense_tile<1, 2, 3>(g, dtype, mode, s);
+    case 5: return launch_dense_tile<1, 1, 4>(g, dtype, mode, s);
+    default: break;
+    }
     const int tiles = (int)(((g.M + dr::BM - 1) / dr::BM) * ((g.N + dr::BN - 1) / dr::BN)) * (mode == 2 ? 2 : 1);
     const int grid = tiles < num_cus_dr() ? tiles : num_cus_dr();
 #define LSMX_DR(DT, MD)                                                                                  \

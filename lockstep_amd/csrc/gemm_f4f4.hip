@@ -1304,15 +1304,11 @@ static hipError_t launch_tile(const GemmArgs &g, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Tile of the K-major path.  A launch costs about
-//   2 us + rounds * fix + stages * (t of every full round + t of the last one)
-// with stages of 256 codes and rounds of (CUs * workgroups per CU) tiles; a
-// last round that leaves CUs idle runs its stages faster (lo) than a full one
-// (hi), since the loads share the L2s and the fabric.  The constants (us) are
-// fits of graph-replayed launches at 28 shapes, M and N 64 .. 8192, K 512 ..
-// 8192, every tile at every shape, and pick the fastest tile or one within
-// 6% of it there.  Largest tiles are the most economical with loads and win
-// once they fill the CUs; before that the smaller ones do:
+// Tile of the K-major path (pick_tile), stages of 256 codes.  The constants
+// (us) are fits of graph-replayed launches at 28 shapes, M and N 64 .. 8192, K
+// 512 .. 8192, every tile at every shape, and pick the fastest tile or one
+// within 6% of it there.  Large tiles load the fewest bytes and win once they
+// fill the CUs; before that the smaller ones do:
 //   M x N x K         256x256  256x128  192x128  128x128  64x128  64x64
 //   200x8192x2048        20.4     11.9     10.2      9.0     7.7    8.3 us
 //   256x2048x8192        40.5     26.4     21.7     18.3    15.0   11.7
@@ -1320,35 +1316,15 @@ static hipError_t launch_tile(const GemmArgs &g, hipStream_t s) {
 //   3000x2048x8192       47.9     30.2     30.1     43.8    40.2   50.2
 //   4096x2048x8192       43.2     35.4     46.0     42.7    50.6   67.3
 //   4096x4096x4096       37.4     44.1     49.0     52.5    60.0   75.6
-struct TileCost {
-    int bm, bn, per_cu;
-    float fix, lo, hi;
-};
 static const TileCost kTiles[] = {
     {256, 256, 1, 8.5f, 1.00f, 1.60f}, {256, 128, 1, 6.0f, 0.62f, 0.86f}, {192, 128, 1, 4.2f, 0.50f, 0.72f},
     {128, 128, 1, 3.5f, 0.43f, 0.58f}, {64, 128, 2, 2.6f, 0.36f, 0.665f}, {64, 64, 2, 2.0f, 0.27f, 0.45f},
 };
-static int pick_tile(int64_t M, int64_t N, int64_t K) {
-    const int cus = num_cus();
-    const float nk = (float)((K + 255) / 256);
-    int best = 0;
-    float tbest = 0.0f;
-    for (int i = 0; i < (int)(sizeof(kTiles) / sizeof(kTiles[0])); ++i) {
-        const TileCost &c = kTiles[i];
-        const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
-        const int64_t cap = (int64_t)cus * c.per_cu, full = (tiles - 1) / cap, last = tiles - full * cap;
-        const float tl = c.per_cu == 1 ? c.lo + (c.hi - c.lo) * (float)last / (float)cap : last <= cus ? c.lo : c.hi;
-        const float t = (float)(full + 1) * c.fix + nk * ((float)full * c.hi + tl);
-        if (i == 0 || t < tbest) best = i, tbest = t;
-    }
-    return best;
-}
-
 hipError_t launch_gemm_f4f4(const GemmArgs &g, hipStream_t s) {
     // the 16 x 16 x 128 kernels form 32 * ld * i in 24-bit multiplies
     const bool kmajor = g.scale_fmt == LSMX_SCALE_E8M0_KMAJOR && g.lda < (1 << 19) && g.ldb < (1 << 19);
     if (kmajor) {
-        int tile = pick_tile(g.M, g.N, g.K);
+        int tile = pick_tile(kTiles, g.M, g.N, 1, (g.K + 255) / 256, num_cus());
 #ifdef SWEEP
         if (const char *e = getenv("LSMX_TILE")) tile = atoi(e);
 #endif

@@ -84,4 +84,31 @@ LSMX_HD int tiles_of_workgroup(int tiles, int wg, int grid) { return (tiles - wg
 // clamping keeps their addresses inside the operands.
 LSMX_HD int stage_tile_iter(int u, int nk, int my_tiles) { return imin(u / nk, my_tiles - 1); }
 
+// Cost model for the output tile of a GEMM launch (host).  A launch of
+// `tiles` tiles on `cus` CUs with per_cu workgroups on each runs in rounds of
+// cap = cus * per_cu tiles and costs, in us,
+//   rounds * fix + stages * (hi per full round + the last round's time),
+// where the last round's stages take from lo (few tiles: the loads have the
+// L2s and the fabric to themselves) to hi (every CU loads): in proportion to
+// its tiles with one workgroup per CU; with two, lo until CUs get a second
+// one.  fix, lo and hi are measured per kernel and tile, see the tables.
+struct TileCost {
+    int bm, bn, per_cu;
+    float fix, lo, hi;
+};
+template <int NT>
+inline int pick_tile(const TileCost (&table)[NT], int64_t M, int64_t N, int64_t problems, int64_t stages, int cus) {
+    int best = 0;
+    float tbest = 0.0f;
+    for (int i = 0; i < NT; ++i) {
+        const TileCost &c = table[i];
+        const int64_t tiles = problems * ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+        const int64_t cap = (int64_t)cus * c.per_cu, full = (tiles - 1) / cap, last = tiles - full * cap;
+        const float tl = c.per_cu == 1 ? c.lo + (c.hi - c.lo) * (float)last / (float)cap : last <= cus ? c.lo : c.hi;
+        const float t = (float)(full + 1) * c.fix + (float)stages * ((float)full * c.hi + tl);
+        if (i == 0 || t < tbest) best = i, tbest = t;
+    }
+    return best;
+}
+
 }  // namespace lsmx
