@@ -20,7 +20,6 @@
 // buffer_load ... lds from waves 0-3 only, one barrier per stage, refill
 // panels set once per tile phase, stages in pairs with compile-time slots,
 // epilogue of 16-byte fp32 stores after an in-quad transpose.
-#include <stdlib.h>
 #include "lsmx_dma.h"
 #include "lsmx_internal.h"
 #include "lsmx_sched.h"
@@ -634,9 +633,6 @@ static hipError_t launch_dense_tile(const DenseArgs &g, int dtype, int mode, hip
 
 hipError_t launch_gemm_dense_ring(const DenseArgs &g, int dtype, int mode, hipStream_t s) {
     int tile = pick_tile(kTiles, g.M, g.N, mode == 2 ? 2 : 1, (mode == 1 ? 2 : 1) * g.K / 64, num_cus_dr());
-#ifdef SWEEP
-    if (const char *e = getenv("LSMX_TILE")) tile = atoi(e);
-#endif
     switch (tile) {
     case 1: return launch_dense_tile<4, 2, 3>(g, dtype, mode, s);
     case 2: return launch_dense_tile<3, 2, 4>(g, dtype, mode, s);

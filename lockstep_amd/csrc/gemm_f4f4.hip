@@ -1325,9 +1325,6 @@ hipError_t launch_gemm_f4f4(const GemmArgs &g, hipStream_t s) {
     const bool kmajor = g.scale_fmt == LSMX_SCALE_E8M0_KMAJOR && g.lda < (1 << 19) && g.ldb < (1 << 19);
     if (kmajor) {
         int tile = pick_tile(kTiles, g.M, g.N, 1, (g.K + 255) / 256, num_cus());
-#ifdef SWEEP
-        if (const char *e = getenv("LSMX_TILE")) tile = atoi(e);
-#endif
         switch (tile) {
         case 1: return launch_tile<8, 4, 3>(g, s);
         case 2: return launch_tile<6, 4, 3>(g, s);

@@ -347,6 +347,206 @@ __global__ __launch_bounds__(f8::NT, 1) void gemm_f8f8_kernel(DenseArgs g) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
+// ---------------------------------------------------------------------------
+// The same product on smaller tiles, for outputs whose 256 x 256 tiles leave
+// compute units idle: one tile of 64 TM x 64 TN per workgroup, 4 MFMA waves
+// (2 x 2, TM x TN tiles of 32 x 32 each) and 4 loader waves, same instruction
+// and order of summation as gemm_f8f8_kernel, so the same bits.  Bound by the
+// loads of a stage (32 KiB per 512 matrix-core cycles at 128 x 128), hence a
+// ring as deep as the LDS allows and loads issued by waves of their own (see
+// gemm_f4f4_tile_kernel, whose schedule this is).  1500 x 4096 x 4096: 61 ->
+// 29.9 us.
+constexpr int f8_tile_slot(int tm, int tn) { return (tm + tn) * 64 * (f8::BKB + 4); }
+template <int CT, bool BNC, int TM, int TN, int S>
+__global__ __launch_bounds__(512, 2) void gemm_f8f8_tile_kernel(DenseArgs g) {
+    constexpr int BM = 64 * TM, BN = 64 * TN, BKB = f8::BKB, CPR = f8::CPR, RPI = f8::RPI;
+    constexpr int NLW = 4;
+    constexpr int XA = BM / (NLW * RPI), XB = BN / (NLW * RPI);
+    // scales: 64 rows per 4-byte DMA, shared out over the loader waves (the
+    // last ones repeat a load when the count is not a multiple of 4)
+    constexpr int NSG = TM + TN, XS = (NSG + NLW - 1) / NLW, L = XA + XB + XS;
+    // N-contiguous B: stage rows of BN bytes, RPB rows per DMA instruction;
+    // LDS chunk c of row r holds source chunk c ^ 2 bswz(r), which spreads the
+    // 8 rows a half-wave reads at once over the 256-byte bank span
+    constexpr int CPB = BN / 16, RPB = 64 / CPB, BSH = BN == 256 ? 0 : BN == 128 ? 1 : 2, BMASK = BN / 32 - 1;
+    static_assert(!BNC || BN == 256 || BN == 128 || BN == 64, "power-of-two rows");
+    static_assert(!BNC || 128 / (RPB * NLW) == XB, "a stage of B is the same bytes in both layouts");
+    constexpr int OFF_B = BM * BKB, OFF_SA = OFF_B + BN * BKB, OFF_SB = OFF_SA + BM * 4, SLOT = OFF_SB + BN * 4;
+    static_assert(SLOT == f8_tile_slot(TM, TN) && S * SLOT <= 160 * 1024 && (S - 1) * L < 64, "LDS, vmcnt");
+    constexpr int NMF = TM * TN, NRD = TM + TN;
+    __shared__ __attribute__((aligned(16))) uint8_t ring[S * SLOT];
+
+    const int tiles_m = (int)((g.M + BM - 1) / BM), tiles_n = (int)((g.N + BN - 1) / BN);
+    const int nk = (int)(g.K / BKB);
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    int tm, tn;
+    tile_coords((int)blockIdx.x, make_tile_map(tiles_m, tiles_n, f8::GROUP_M), tm, tn);
+    const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
+
+    if (wave >= NLW) {
+        // ---- loader waves
+        __builtin_amdgcn_s_setprio(3);
+        const int lw = wave - NLW;
+        const int drow0 = lw * RPI + lane / CPR;
+        const uint32_t offA0 = (uint32_t)(drow0 * g.lda + (((lane % CPR) ^ f8::swz(drow0)) << 4));
+        const int brow0 = RPB * lw + lane / CPB;   // its low 3 bits do not depend on the load index
+        const uint32_t offB0 =
+            BNC ? (uint32_t)(brow0 * g.ldb + (((lane % CPB) ^ (2 * ((brow0 >> BSH) & BMASK))) << 4))
+                : (uint32_t)(drow0 * g.ldb + (((lane % CPR) ^ f8::swz(drow0)) << 4));
+        const uint32_t stepA = (uint32_t)(NLW * RPI * g.lda);
+        const uint32_t stepB = BNC ? (uint32_t)(RPB * NLW * g.ldb) : (uint32_t)(NLW * RPI * g.ldb);
+        const uint8_t *pa = g.a0 + m0 * g.lda, *pb = g.b0 + (BNC ? n0 : n0 * g.ldb);
+        const int64_t na = (min(g.M - m0, (int64_t)BM) - 1) * g.lda + g.K;
+        // BNC: columns past N in other rows read the next row's values, whose
+        // products reach no stored output
+        const int64_t nb = BNC ? (g.K - 1) * g.ldb + (g.N - n0) : (min(g.N - n0, (int64_t)BN) - 1) * g.ldb + g.K;
+        const int64_t sbytes_a = ((g.K / 128 - 1) * g.ld_sa + g.M) * 4, sbytes_b = ((g.K / 128 - 1) * g.ld_sb + g.N) * 4;
+        const uint32_t ring0 = lds_u32(&ring[0]);
+        auto load_stage = [&](int kt, uint32_t so) __attribute__((always_inline)) {
+            const bool past = kt >= nk;   // refills past the end: empty descriptors, zeros
+            const int64_t ao = (int64_t)kt * BKB, bo = BNC ? ao * g.ldb : ao;
+            const v4i_rsrc rsA = buf_rsrc(pa + (past ? 0 : ao), past ? 0 : (uint64_t)(na - ao));
+            const v4i_rsrc rsB = buf_rsrc(pb + (past ? 0 : bo), past ? 0 : (uint64_t)(nb - bo));
+#pragma unroll
+            for (int i = 0; i < XA; ++i) dma_x4(offA0 + i * stepA, rsA, ring0 + so + (i * NLW + lw) * 1024);
+#pragma unroll
+            for (int i = 0; i < XB; ++i) dma_x4(offB0 + i * stepB, rsB, ring0 + so + OFF_B + (i * NLW + lw) * 1024);
+#pragma unroll
+            for (int i = 0; i < XS; ++i) {
+                const int e = min(i * NLW + lw, NSG - 1);
+                const bool to_b = e >= TM;
+                const int gi = to_b ? e - TM : e;
+                const int64_t b0 = ((int64_t)kt * (to_b ? g.ld_sb : g.ld_sa) + (to_b ? n0 : m0) + gi * 64) * 4;
+                const int64_t left = (to_b ? sbytes_b : sbytes_a) - b0;
+                const bool none = past || left <= 0;
+                dma_x1((uint32_t)lane * 4, buf_rsrc((to_b ? g.sb : g.sa) + (none ? 0 : b0), none ? 0 : (uint64_t)left),
+                       ring0 + so + (to_b ? OFF_SB : OFF_SA) + gi * 256);
+            }
+        };
+#pragma unroll
+        for (int q = 0; q < S; ++q) load_stage(q, q * SLOT);
+        wait_vm_barrier<(S - 1) * L>();
+        uint32_t so = 0;
+        for (int kt = 0; kt < nk; ++kt) {
+            wait_vm_barrier<(S - 2) * L>();
+            load_stage(kt + S, so);
+            so = so + SLOT == S * SLOT ? 0 : so + SLOT;
+        }
+        // no load may still be writing this workgroup's LDS when it exits
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        return;
+    }
+
+    // ---- MFMA waves; fragment and scale layouts as in gemm_f8f8_kernel
+    const int wm = wave >> 1, wn = wave & 1;
+    const int frow = lane & 31, half = lane >> 5;
+    const int bj8 = lane & 15, brs8 = bj8 >> 1;
+    uint32_t bfo[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+        bfo[j] = (uint32_t)(OFF_B + (half * 16 + brs8) * BN +
+                            ((2 * ((wn * TN + j) ^ ((brs8 >> BSH) & BMASK)) + ((lane >> 4) & 1)) << 4) + 8 * (bj8 & 1));
+    uint32_t ro[4];   // chunks 4 st + half and 4 st + 2 + half of row frow
+#pragma unroll
+    for (int k = 0; k < 4; ++k) ro[k] = (uint32_t)(frow * BKB + (((2 * k + half) ^ f8::swz(frow)) << 4));
+    v16f8 acc[TM][TN];
+    uint32_t scA[TM], scB[TN], nxA[TM], nxB[TN];
+    v8i fa[2][TM], fb[2][TN];
+    auto read_frag = [&](uint32_t so, int st, int q) __attribute__((always_inline)) {
+        if (BNC && q >= TM) {
+            const uint8_t *p = &ring[0] + so + bfo[q - TM] + st * (64 * BN);
+            const v2i_f8 r0 = ds_read_tr8x8(p), r1 = ds_read_tr8x8(p + 8 * BN);
+            const v2i_f8 r2 = ds_read_tr8x8(p + 32 * BN), r3 = ds_read_tr8x8(p + 40 * BN);
+            fb[st][q - TM] = v8i{r0.x, r0.y, r1.x, r1.y, r2.x, r2.y, r3.x, r3.y};
+            return;
+        }
+        const uint8_t *base = &ring[0] + so + (q < TM ? (wm * TM + q) * 32 * BKB : OFF_B + (wn * TN + q - TM) * 32 * BKB);
+        const u32x4 lo = *reinterpret_cast<const u32x4 *>(base + ro[2 * st]);
+        const u32x4 hi = *reinterpret_cast<const u32x4 *>(base + ro[2 * st + 1]);
+        const v8i f = v8i{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+        if (q < TM) fa[st][q] = f;
+        else fb[st][q - TM] = f;
+    };
+    auto read_scale = [&](uint32_t so, int q) __attribute__((always_inline)) {
+        const int r = q < TM ? (wm * TM + q) * 32 + frow : (wn * TN + q - TM) * 32 + frow;
+        const uint32_t v = *reinterpret_cast<const uint32_t *>(&ring[0] + so + (q < TM ? OFF_SA : OFF_SB) + r * 4);
+        if (q < TM) nxA[q] = v;
+        else nxB[q - TM] = v;
+    };
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+    asm volatile("s_barrier" ::: "memory");
+#pragma unroll
+    for (int q = 0; q < NRD; ++q) read_scale(0, q);
+#pragma unroll
+    for (int q = 0; q < NRD; ++q) read_frag(0, 0, q);
+    uint32_t so = 0;
+    for (int kt = 0; kt < nk; ++kt) {
+        const uint32_t sn = so + SLOT == S * SLOT ? 0 : so + SLOT;
+        // op_sel = 2 st picks block 2 st + half of the stage's scale dword
+#pragma unroll
+        for (int i = 0; i < TM; ++i) scA[i] = nxA[i] >> (8 * half);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) scB[j] = nxB[j] >> (8 * half);
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+            if (st == 1) {
+                // this wave's reads of the slot are complete; past the
+                // barrier it may be refilled and stage kt + 1 has landed
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int idx = 0; idx < NMF; ++idx) {
+                const int i = idx / TN, j = idx % TN;
+                acc[i][j] = mfma_scale_f8(fa[st][i], fb[st][j], acc[i][j], 0, 0, 2 * st, (int)scA[i], 2 * st, (int)scB[j]);
+                if (st == 0) {
+#pragma unroll
+                    for (int r = idx * NRD / NMF; r < (idx + 1) * NRD / NMF; ++r) read_frag(so, 1, r);
+                } else {
+#pragma unroll
+                    for (int r = idx * 2 * NRD / NMF; r < (idx + 1) * 2 * NRD / NMF; ++r) {
+                        if (r < NRD) read_scale(sn, r);
+                        else read_frag(sn, 0, r - NRD);
+                    }
+                }
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        so = sn;
+    }
+
+    // ---- epilogue, as in gemm_f8f8_kernel
+    const bool vec_c = ((reinterpret_cast<uintptr_t>(g.c0) & 15) == 0) && (g.ldc % 4 == 0);
+    const int q = frow & 3;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int gq = 0; gq < 4; ++gq) {
+            const int64_t row = m0 + (wm * TM + i) * 32 + 8 * gq + 4 * half + q;
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                float x[4] = {acc[i][j][4 * gq], acc[i][j][4 * gq + 1], acc[i][j][4 * gq + 2], acc[i][j][4 * gq + 3]};
+                // all four lanes of a quad take part in the exchanges
+                quad_transpose(x, q);
+                const int64_t col = n0 + (wn * TN + j) * 32 + (frow & ~3);
+                if (row < g.M && col < g.N) {
+                    if (vec_c && col + 4 <= g.N) store_c4<CT>(g.c0, row * g.ldc + col, x[0], x[1], x[2], x[3]);
+                    else
+#pragma unroll
+                        for (int c = 0; c < 4; ++c)
+                            if (col + c < g.N) store_c<CT>(g.c0, row * g.ldc + col + c, x[c]);
+                }
+            }
+        }
+}
+
 static int num_cus_f8() {
     static int cus = 0;
     if (cus == 0) {
@@ -360,7 +560,46 @@ static int num_cus_f8() {
     return cus;
 }
 
+// Output tile (pick_tile), stages of 128 elements.  The constants (us) are fits
+// of graph-replayed launches of every tile at 18 shapes, M and N 64 .. 8192,
+// K 1024 .. 8192, B N-contiguous:
+//   M x N x K         256x256  256x128  192x128  128x128  64x128  64x64
+//   64x4096x2048         32.1     15.3     12.9     10.4     8.2    7.2 us
+//   1024x1024x4096       55.0     26.8     22.1     18.0    14.1   13.8
+//   2048x2048x2048       32.7     18.9     16.2     15.0    17.4   24.1
+//   1500x4096x4096       59.8     33.1     29.9     36.1    39.7   56.4
+//   4096x2048x4096       54.2     35.6     45.4     42.1    48.8   72.2
+//   4096x4096x4096       61.9     66.4     75.9     77.3    90.8  135.3
+static const TileCost kTiles[] = {
+    {256, 256, 1, 11.0f, 1.30f, 1.58f}, {256, 128, 1, 6.0f, 0.60f, 0.93f}, {192, 128, 1, 5.0f, 0.48f, 0.78f},
+    {128, 128, 1, 4.0f, 0.40f, 0.56f},  {64, 128, 2, 3.0f, 0.34f, 0.72f},  {64, 64, 2, 2.5f, 0.31f, 0.55f},
+};
+
+template <int TM, int TN, int S>
+static hipError_t launch_f8_tile(const DenseArgs &g, hipStream_t s) {
+    const int64_t grid = ((g.M + 64 * TM - 1) / (64 * TM)) * ((g.N + 64 * TN - 1) / (64 * TN));
+#define LSMX_F8T(CT)                                                                                                \
+    do {                                                                                                           \
+        if (g.b_nc) hipLaunchKernelGGL((gemm_f8f8_tile_kernel<CT, true, TM, TN, S>), dim3((unsigned)grid), dim3(512), 0, s, g); \
+        else hipLaunchKernelGGL((gemm_f8f8_tile_kernel<CT, false, TM, TN, S>), dim3((unsigned)grid), dim3(512), 0, s, g);      \
+    } while (0)
+    if (g.c_dtype == LSMX_F32) LSMX_F8T(LSMX_F32);
+    else if (g.c_dtype == LSMX_BF16) LSMX_F8T(LSMX_BF16);
+    else LSMX_F8T(LSMX_F16);
+#undef LSMX_F8T
+    return hipGetLastError();
+}
+
 hipError_t launch_gemm_f8f8_kmajor(const DenseArgs &g, hipStream_t s) {
+    int tile = pick_tile(kTiles, g.M, g.N, 1, g.K / f8::BKB, num_cus_f8());
+    switch (tile) {
+    case 1: return launch_f8_tile<4, 2, 3>(g, s);
+    case 2: return launch_f8_tile<3, 2, 3>(g, s);
+    case 3: return launch_f8_tile<2, 2, 4>(g, s);
+    case 4: return launch_f8_tile<1, 2, 3>(g, s);
+    case 5: return launch_f8_tile<1, 1, 4>(g, s);
+    default: break;
+    }
     const int tiles = (int)(((g.M + f8::BM - 1) / f8::BM) * ((g.N + f8::BN - 1) / f8::BN));
     const int grid = tiles < num_cus_f8() ? tiles : num_cus_f8();
     const dim3 blk(f8::NT);
