@@ -586,7 +586,8 @@ int lsmx_scale_to_e8m0_batch(const lsmx_e8m0_item *items, int n, uint64_t *flag,
         if (blocks % 4) return fail(LSMX_ERR_SHAPE, "%s: item %d: K-major output needs a multiple of 4 blocks", fn, k);
         if (!aligned(it.s, 4) || !aligned(it.out, 4)) return fail(LSMX_ERR_ALIGN, "%s: item %d misaligned", fn, k);
         if (it.rows > 0 && it.cols > ((int64_t)1 << 38) / it.rows) return fail(LSMX_ERR_SHAPE, "%s: item %d too large", fn, k);
-        const int64_t w = ((orows + 63) / 64) * ((blocks / 4 + 15) / 16);
+        const int64_t wr = tin ? lsmx::kE8TinRows : lsmx::kE8Rows, wg = tin ? lsmx::kE8TinGroups : lsmx::kE8Groups;
+        const int64_t w = ((orows + wr - 1) / wr) * ((blocks / 4 + wg - 1) / wg);
         if (w == 0) continue;  // empty tensors take no workgroup
         if (wgs + w > 0x7FFFFFFF) return fail(LSMX_ERR_SHAPE, "%s: too many workgroups", fn);
         const int vec4 = !tin && aligned(it.s, 16) && it.lds % 4 == 0;

@@ -399,75 +399,86 @@ __global__ __launch_bounds__(256) void scale_to_e8m0_km4_tiled_kernel(const floa
 }
 
 // Up to four fp32 scale tensors -> K-major E8M0 dwords in one launch (the A
-// and B scales of one GEMM call).  A workgroup converts 64 output rows x 16
-// four-block groups of one tensor through a dword tile in LDS (one padding
-// dword per group row): row-major input with 16-byte rows is read as in
-// scale_to_e8m0_km4_tiled_kernel (four blocks per float4, 256 contiguous
-// bytes per 16 threads); [blocks, rows] input (tin) one float per thread, 64
-// consecutive rows of a block per wave, each lane writing a byte of its own
-// dword.  The stores are 64 consecutive dwords of a group.  A scale with no
-// E8M0 form becomes 0xFF as above and, unless it is a NaN (which E8M0 has,
-// with the same effect on every output that uses it), makes the wave that
+// and B scales of one GEMM call).  Row-major input: a workgroup converts
+// kE8Rows output rows x kE8Groups four-block groups through a dword tile in
+// LDS (one padding dword per group row), four blocks per load (float4 where
+// the rows are 16-byte aligned, 256 contiguous bytes per 16 threads), the
+// stores kE8Rows consecutive dwords of a group.  [blocks, rows] input (tin):
+// kE8TinRows rows x kE8TinGroups groups, one dword per thread from four
+// loads that are contiguous across the wave, stored as they are.  A few MB of
+// scales in all, so it is bound by the latency of a workgroup's loads: many
+// small workgroups, every load of a thread issued before the first is used
+// (64 rows x 16 groups with 16 loads per thread in turns took 9.4 us for the
+// scales of 1500 x 4096 and 4096 x 4096 operands, this 4.5).  A scale
+// with no E8M0 form becomes 0xFF as above and, unless it is a NaN (which E8M0
+// has, with the same effect on every output that uses it), makes the wave that
 // met it write the caller's epoch to the flag (one store per wave), which
 // the promotion GEMM that follows checks.
 __global__ __launch_bounds__(256) void scale_to_e8m0_batch_kernel(E8m0Batch b) {
-    __shared__ uint32_t tile[16][65];
+    __shared__ uint32_t tile[kE8Groups][kE8Rows + 1];
     const int64_t blk = (int64_t)blockIdx.x;
     int k = 0;
     while (k + 1 < b.n && blk >= b.end[k]) ++k;
     const E8m0Item &it = b.it[k];
     const int64_t local = blk - (k ? b.end[k - 1] : 0);
-    const int64_t tiles_o = (it.orows + 63) / 64;
-    const int64_t o0 = (local % tiles_o) * 64, g0 = (local / tiles_o) * 16;
     const int t = threadIdx.x;
     bool bad = false;
+    auto convert = [&](const uint32_t (&x)[4]) {
+        uint32_t w = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t e = f32_scale_e8m0(x[j]);
+            bad |= e == 0xFFu && (x[j] & 0x7FFFFFFFu) <= 0x7F800000u;
+            w |= e << (8 * j);
+        }
+        return w;
+    };
     if (it.tin) {
-        uint8_t *tb = reinterpret_cast<uint8_t *>(tile);
-#pragma unroll 4
-        for (int i = 0; i < 16; ++i) {
-            const int q = i * 256 + t, r = q & 63, c = q >> 6;  // out row, block in tile
-            const int64_t o = o0 + r, bk = 4 * g0 + c;
-            if (o < it.orows && bk < 4 * it.groups) {
-                const uint32_t x = f2u(it.s[bk * it.lds + o]), e = f32_scale_e8m0(x);
-                bad |= e == 0xFFu && (x & 0x7FFFFFFFu) <= 0x7F800000u;
-                tb[((c >> 2) * 65 + r) * 4 + (c & 3)] = (uint8_t)e;
-            }
+        const int64_t tiles_o = (it.orows + kE8TinRows - 1) / kE8TinRows;
+        const int64_t o = (local % tiles_o) * kE8TinRows + t % kE8TinRows;
+        const int64_t gr = (local / tiles_o) * kE8TinGroups + t / kE8TinRows;
+        if (o < it.orows && gr < it.groups) {
+            uint32_t x[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) x[j] = f2u(it.s[(4 * gr + j) * it.lds + o]);
+            *reinterpret_cast<uint32_t *>(it.out + (gr * it.ldo + o) * 4) = convert(x);
         }
     } else {
+        const int64_t tiles_o = (it.orows + kE8Rows - 1) / kE8Rows;
+        const int64_t o0 = (local % tiles_o) * kE8Rows, g0 = (local / tiles_o) * kE8Groups;
+        constexpr int NI = kE8Rows * kE8Groups / 256;
+        uint32_t x[NI][4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int q = i * 256 + t, r = q >> 4, gi = q & 15;
+        for (int i = 0; i < NI; ++i) {
+            const int q = i * 256 + t, r = q / kE8Groups, gi = q % kE8Groups;
             const int64_t o = o0 + r, gr = g0 + gi;
+            x[i][0] = x[i][1] = x[i][2] = x[i][3] = 0x3F800000u;
             if (o < it.orows && gr < it.groups) {
-                uint32_t x[4];
                 if (it.vec4) {
                     const float4 v = *reinterpret_cast<const float4 *>(it.s + o * it.lds + 4 * gr);
-                    x[0] = f2u(v.x), x[1] = f2u(v.y), x[2] = f2u(v.z), x[3] = f2u(v.w);
+                    x[i][0] = f2u(v.x), x[i][1] = f2u(v.y), x[i][2] = f2u(v.z), x[i][3] = f2u(v.w);
                 } else {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) x[j] = f2u(it.s[o * it.lds + 4 * gr + j]);
+                    for (int j = 0; j < 4; ++j) x[i][j] = f2u(it.s[o * it.lds + 4 * gr + j]);
                 }
-                uint32_t w = 0;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t e = f32_scale_e8m0(x[j]);
-                    bad |= e == 0xFFu && (x[j] & 0x7FFFFFFFu) <= 0x7F800000u;
-                    w |= e << (8 * j);
-                }
-                tile[gi][r] = w;
             }
+        }
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int q = i * 256 + t;
+            tile[q % kE8Groups][q / kE8Groups] = convert(x[i]);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int q = i * 256 + t, gi = q / kE8Rows, r = q % kE8Rows;
+            const int64_t o = o0 + r, gr = g0 + gi;
+            if (o < it.orows && gr < it.groups) *reinterpret_cast<uint32_t *>(it.out + (gr * it.ldo + o) * 4) = tile[gi][r];
         }
     }
     if (b.flag) {
         const uint64_t m = __ballot(bad);
         if (m && (t & 63) == __builtin_ctzll(m)) *b.flag = b.epoch;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int q = i * 256 + t, gi = q >> 6, r = q & 63;
-        const int64_t o = o0 + r, gr = g0 + gi;
-        if (o < it.orows && gr < it.groups) *reinterpret_cast<uint32_t *>(it.out + (gr * it.ldo + o) * 4) = tile[gi][r];
     }
 }
 

@@ -161,6 +161,9 @@ struct PromoteArgs {
 // end[k] = workgroups of tensors 0 .. k.  When a scale has no E8M0 form the
 // launch writes epoch to *flag (if flag is not null).
 constexpr int kE8Batch = 4;
+// output rows x four-block groups of one workgroup (256 threads)
+constexpr int kE8Rows = 32, kE8Groups = 16;       // row-major input
+constexpr int kE8TinRows = 64, kE8TinGroups = 4;  // [blocks, rows] input
 struct E8m0Item {
     const float *s;
     int64_t orows, groups, lds;  // out rows, 4-block groups, stride of s
