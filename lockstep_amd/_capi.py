@@ -140,11 +140,15 @@ def last_error() -> str:
     return load().lsmx_last_error().decode()
 
 
-def call(name: str, *args) -> None:
-    """Call an entry point and raise LsmxError on a non-zero status."""
-    rc = getattr(load(), name)(*args)
+def check(rc: int) -> None:
+    """Raise LsmxError for a non-zero status of this thread's last call."""
     if rc != OK:
         raise LsmxError(rc, last_error())
+
+
+def call(name: str, *args) -> None:
+    """Call an entry point and raise LsmxError on a non-zero status."""
+    check(getattr(load(), name)(*args))
 
 
 def stream_of(t: torch.Tensor) -> int:
@@ -198,3 +202,23 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor:
         ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
         _workspaces[key] = ws
     return ws
+
+
+class _MissingFast:
+    """Stands in for the native call path when it has not been built."""
+
+    def __init__(self, why):
+        self._why = why
+
+    def __getattr__(self, name):
+        raise RuntimeError(f"lockstep_amd/_fast.so cannot be loaded ({self._why}): build it with "
+                           "`python -m lockstep_amd.build`")
+
+
+# The plain forms of the public calls in native code (csrc/fast.cpp): each
+# function returns None for any other form, which then takes the Python path.
+try:
+    from . import _fast as fast
+    fast.init(check, workspace, next_epoch)
+except ImportError as e:
+    fast = _MissingFast(e)

@@ -22,6 +22,7 @@ SOURCES = ["capi.hip", "quantize.hip", "gemm_f4f4.hip", "gemm_bf16f4.hip", "gemm
 ARCH = "gfx950"
 
 # -packed-fp32-ops: no v_pk_{add,mul,fma}_f32 anywhere in the device code.
+FAST_LIB = PKG / "_fast.so"
 FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-shared",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -42,6 +43,23 @@ def _run(cmd, verbose):
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"hipcc failed ({res.returncode}):\n{res.stdout}\n{res.stderr}")
+
+
+def build_fast(verbose: bool = False) -> Path:
+    """Compile _fast.so, the native call path (csrc/fast.cpp): host code
+    against torch's headers, linked to the liblsmx.so next to it."""
+    import sysconfig
+
+    from torch.utils import cpp_extension as ext
+
+    tmp = FAST_LIB.with_suffix(".so.tmp")
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+          *[f"-isystem{p}" for p in ext.include_paths("cuda")], f"-isystem{sysconfig.get_paths()['include']}",
+          str(CSRC / "fast.cpp"), "-o", str(tmp), f"-L{PKG}", "-l:liblsmx.so",
+          *[f"-L{p}" for p in ext.library_paths("cuda")], "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip",
+          "-ltorch", "-ltorch_python", "-Wl,-rpath,$ORIGIN"], verbose)
+    os.replace(tmp, FAST_LIB)
+    return FAST_LIB
 
 
 def build(verbose: bool = False, jobs: int | None = None) -> Path:
@@ -68,4 +86,5 @@ def build(verbose: bool = False, jobs: int | None = None) -> Path:
 
 if __name__ == "__main__":
     build(verbose=True)
-    print(f"built {LIB}", file=sys.stderr)
+    build_fast(verbose=True)
+    print(f"built {LIB} and {FAST_LIB}", file=sys.stderr)

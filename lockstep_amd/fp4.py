@@ -44,8 +44,8 @@ def _mark_e8m0_exact(s: torch.Tensor) -> torch.Tensor:
     # tensor that owns the storage: every view of it points to that one.
     b = s._base if s._base is not None else s
     key = id(b)
-    _E8M0_EXACT[key] = (b._version, b.data_ptr())
-    weakref.finalize(b, _E8M0_EXACT.pop, key, None)
+    # the weak reference drops the entry with the tensor
+    _E8M0_EXACT[key] = (b._version, b.data_ptr(), weakref.ref(b, lambda _, key=key: _E8M0_EXACT.pop(key, None)))
     return s
 
 
@@ -55,7 +55,8 @@ def e8m0_exact(*scales: torch.Tensor) -> bool:
     written since (views share the version counter of their base)."""
     def known(s):
         b = s._base if s._base is not None else s
-        return _E8M0_EXACT.get(id(b)) == (b._version, b.data_ptr())
+        e = _E8M0_EXACT.get(id(b))
+        return e is not None and e[0] == b._version and e[1] == b.data_ptr()
     return all(known(s) for s in scales)
 
 # ---------------------------------------------------------------- E2M1 tables
@@ -119,6 +120,8 @@ def quantize_mxfp4(x: torch.Tensor, block: int = 32):
     Returns (codes uint8 [..., K], scale fp32 [..., K//block]).
     Shared scale follows OCP MX: 2^(floor(log2(amax)) - emax_elem), emax_elem = 2,
     with log2 rounded to float32 as torch computes it."""
+    if block == 32 and (r := C.fast.quantize(x)) is not None:
+        return r[0], _mark_e8m0_exact(r[1])
     *lead, K = x.shape
     assert K % block == 0, f"K={K} must be a multiple of block={block}"
     C.require_device(x)
@@ -142,6 +145,9 @@ def quantize_pack_mxfp4(x: torch.Tensor, block: int = 32, scale_layout: str = "r
     scale_layout "rows": e8m0 is [..., K//block] (row-major, like fp4.py's
     scales).  "kmajor" (2-D x, block 32, K % 128 == 0): e8m0 is
     [K//128, rows, 4], the layout the f4 x f4 GEMM streams fastest."""
+    if block == 32 and scale_layout in ("rows", "kmajor") and \
+            (r := C.fast.quantize_pack(x, scale_layout == "kmajor")) is not None:
+        return r
     *lead, K = x.shape
     assert K % block == 0, f"K={K} must be a multiple of block={block}"
     C.require_device(x)
@@ -175,6 +181,8 @@ def quantize_pack_mxfp4_many(xs, scale_layout: str = "rows"):
     if scale_layout not in ("rows", "kmajor"):
         raise ValueError(f"scale_layout must be 'rows' or 'kmajor', got {scale_layout!r}")
     km = scale_layout == "kmajor"
+    if (r := C.fast.quantize_pack2(xs, km)) is not None:
+        return r
     out = [None] * len(xs)
     groups = {}
     for i, x in enumerate(xs):
@@ -258,6 +266,8 @@ def quantize_pack_mxfp4_2d(x: torch.Tensor, scale_layout: str = "kmajor"):
     columns (blocks of 32 rows, laid out for x^T), E8M0 scales.  bf16 / fp16
     x with R and C multiples of 128 run the fused one-pass kernel
     (lsmx_quantize_mxfp4_2d); other inputs run the two quantizers."""
+    if scale_layout == "kmajor" and (r := C.fast.quantize_2d(x)) is not None:
+        return r
     C.require_device(x)
     assert x.dim() == 2, "quantize_pack_mxfp4_2d takes a 2-D tensor"
     R, Cn = x.shape
@@ -424,6 +434,8 @@ def codes_to_q(codes: torch.Tensor) -> torch.Tensor:
 
 def pack_fp4(codes: torch.Tensor) -> torch.Tensor:
     """[..., K] uint8 codes -> [..., K//2] bytes; even index in the low nibble (fp4.py:91-94)."""
+    if (r := C.fast.pack(codes)) is not None:
+        return r
     assert codes.shape[-1] % 2 == 0
     C.require_device(codes)
     c = codes.contiguous()

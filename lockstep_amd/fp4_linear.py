@@ -60,6 +60,8 @@ def path():
 def _forward_hip(x2: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """The forward of fp4_linear.py:34-40 on the GPU: quantize X and W along K
     (fused quantize + pack kernels, E8M0 scales) and call kernel()."""
+    if (r := C.fast.linear(x2, w, x2.dtype)) is not None:
+        return r
     # K-major E8M0 scales: the layout the GEMM streams fastest (same bits out)
     lay = "kmajor" if x2.shape[-1] % 128 == 0 else "rows"
     xp, xs = fp4.quantize_pack_mxfp4(x2, scale_layout=lay)
@@ -160,7 +162,11 @@ class MXFP4Linear(nn.Linear):
         self.quantized_backward = quantized_backward
 
     def forward(self, x):
-        dt = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x.dtype
-        with torch.autocast("cuda", enabled=False):
-            y = mxfp4_matmul(x.reshape(-1, x.shape[-1]).to(dt), self.weight, self.quantized_backward)
+        x2 = x.reshape(-1, x.shape[-1])
+        if torch.is_autocast_enabled("cuda"):
+            x2 = x2.to(torch.get_autocast_dtype("cuda"))
+            with torch.autocast("cuda", enabled=False):
+                y = mxfp4_matmul(x2, self.weight, self.quantized_backward)
+        else:
+            y = mxfp4_matmul(x2, self.weight, self.quantized_backward)
         return y.view(*x.shape[:-1], -1)

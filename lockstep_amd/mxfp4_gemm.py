@@ -67,6 +67,9 @@ def mxfp4_gemm_packed(a_pk, bt_pk, a_scale, b_scale, out_dtype=torch.bfloat16):
     that launch exits at once, and for scales fp4.quantize_mxfp4 returned
     (and nobody wrote since) it is not made.  Returns C = A @ B_T.T [M, N]
     in out_dtype, fp32 accumulate."""
+    exact = a_scale.dtype == torch.float32 and _fp4.e8m0_exact(a_scale, b_scale)
+    if (r := C.fast.gemm_packed(a_pk, bt_pk, a_scale, b_scale, out_dtype, exact)) is not None:
+        return r
     M, Kh = a_pk.shape
     N, Kh2 = bt_pk.shape
     K = Kh * 2
@@ -100,7 +103,6 @@ def mxfp4_gemm_packed(a_pk, bt_pk, a_scale, b_scale, out_dtype=torch.bfloat16):
         promote = None
     else:
         # the reference's spelling (fp32 scales from quantize_mxfp4)
-        exact = _fp4.e8m0_exact(a_scale, b_scale)
         sa32, sb32 = _f32_rows(a_scale), _f32_rows(b_scale)
         (a_scale, b_scale), flag, epoch = _e8m0_kmajor_flagged([(sa32, M, False), (sb32, N, False)], K // 32,
                                                                flagged=not exact)
@@ -167,6 +169,8 @@ def mxfp4_gemm_bf16(a, w_pk, w_scale, out_dtype=torch.bfloat16):
     activations are not narrowed: each is split exactly into bf16 terms
     (lsmx_gemm_wonly_f4), so an fp32 X gives the arithmetic of an fp32
     matmul (the reference's fake-quant Y = X @ dequantize_mxfp4(W)^T)."""
+    if out_dtype is not None and (r := C.fast.weight(a, None, w_pk, w_scale, out_dtype)) is not None:
+        return r
     M, K = a.shape
     N, Kh = w_pk.shape
     assert K == 2 * Kh and K % 128 == 0, "K must be a multiple of 128 (max BLOCK_K)"
@@ -213,6 +217,8 @@ def mxfp4_linear_w(a, w_pk, w_scale, out_dtype=None):
     """Y = a @ deq(W)^T for an unquantized activation a [..., K] (any of
     bf16 / fp32 / fp16) and a packed MXFP4 weight: the weight-only linear
     forward, output in a's dtype unless out_dtype is given."""
+    if (r := C.fast.weight(a, None, w_pk, w_scale, out_dtype)) is not None:
+        return r
     K = a.shape[-1]
     y = mxfp4_gemm_bf16(a.reshape(-1, K), w_pk, w_scale, out_dtype=out_dtype or a.dtype)
     return y.reshape(*a.shape[:-1], w_pk.shape[0])
@@ -357,6 +363,9 @@ def mxfp4_gemm_fp8(a_fp8, b_fp8, a_scale, b_scale, out_dtype=torch.bfloat16):
     by both kernels (lsmx_gemm_f8f8_nb, LSMX_B_NCONTIG); otherwise B is
     transposed to K-contiguous rows on the device first unless b_fp8 is a
     transposed view of such rows."""
+    exact = a_scale.dtype == torch.float32 and b_scale.dtype == torch.float32 and _fp4.e8m0_exact(a_scale, b_scale)
+    if (r := C.fast.gemm_fp8(a_fp8, b_fp8, a_scale, b_scale, out_dtype, exact)) is not None:
+        return r
     M, K = a_fp8.shape
     K2, N = b_fp8.shape
     assert K == K2 and K % 128 == 0, "K must be a multiple of 128 (max BLOCK_K)"
@@ -379,7 +388,6 @@ def mxfp4_gemm_fp8(a_fp8, b_fp8, a_scale, b_scale, out_dtype=torch.bfloat16):
         sa = _e8m0_kmajor(a_scale, M, K // 32, transposed=False)
         sb = _e8m0_kmajor(b_scale, N, K // 32, transposed=True)
     else:
-        exact = _fp4.e8m0_exact(a_scale, b_scale)
         sa32, sb32 = _f32_rows(a_scale), _f32_rows(b_scale)
         (sa, sb), flag, epoch = _e8m0_kmajor_flagged([(sa32, M, False), (sb32, N, True)], K // 32,
                                                      flagged=not exact)

@@ -1,0 +1,137 @@
+"""The native call path (csrc/fast.cpp) against the Python one: forms it does
+not take give None (CPU), and those it takes give the general path's bits."""
+
+import pytest
+import torch
+
+
+@pytest.fixture
+def C():
+    from lockstep_amd import _capi
+    return _capi
+
+
+class Sub(torch.Tensor):
+    pass
+
+
+def test_other_forms_are_left_to_the_python_path(C):
+    """CPU tensors, tensor subclasses, non-tensors and wrong argument counts."""
+    x = torch.zeros(4, 128)
+    u = torch.zeros(4, 64, dtype=torch.uint8)
+    for bad in (x, x.as_subclass(Sub), None, 3, [1, 2]):
+        assert C.fast.quantize(bad) is None and C.fast.quantize_pack(bad, True) is None
+        assert C.fast.quantize_2d(bad) is None and C.fast.pack(bad) is None
+        assert C.fast.quantize_pack2(bad, False) is None and C.fast.quantize_pack2([bad, bad], True) is None
+        assert C.fast.linear(bad, bad, torch.float32) is None
+        assert C.fast.gemm_packed(bad, u, u, u, torch.float32, False) is None
+        assert C.fast.weight(bad, None, u, u, None) is None
+        assert C.fast.gemm_fp8(bad, u, x, x, torch.float32, False) is None
+    assert C.fast.quantize() is None and C.fast.weight(x) is None
+    with pytest.raises(RuntimeError, match="gfx950 GPU only"):
+        from lockstep_amd import fp4
+        fp4.quantize_pack_mxfp4(x)
+
+
+def _general(monkeypatch, C, f):
+    """f() with every native call declined."""
+    class Declines:
+        def __getattr__(self, name):
+            return lambda *a: None
+    with monkeypatch.context() as m:
+        m.setattr(C, "fast", Declines())
+        return _outcome(f)
+
+
+def _outcome(f):
+    """What f returns, or the error it raises."""
+    try:
+        return f()
+    except Exception as e:
+        return type(e), str(e)
+
+
+def _same(a, b):
+    if not isinstance(a, (tuple, list, torch.Tensor)):
+        return a == b
+    if isinstance(a, (tuple, list)):
+        return type(a) is type(b) and len(a) == len(b) and all(_same(x, y) for x, y in zip(a, b))
+    return a.dtype == b.dtype and a.shape == b.shape and a.device == b.device and torch.equal(
+        a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("R,K", [(1, 128), (3, 160), (128, 256), (257, 1152)])
+def test_quantizers_match_the_python_path(C, monkeypatch, R, K, dtype):
+    from lockstep_amd import fp4
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(R + K)
+    base = torch.randn((R, K + 16), device=dev, generator=g).to(dtype)
+    other = torch.randn((K, R + 3), device=dev, generator=g).to(dtype)
+    for x in (base[:, :K], base[:, :K].contiguous(), base[:, 1:K + 1], other.t()[:R], base[:0, :K]):
+        forms = [lambda: fp4.quantize_mxfp4(x), lambda: fp4.quantize_pack_mxfp4(x),
+                 lambda: fp4.quantize_pack_mxfp4_many([x, x]), lambda: fp4.pack_fp4(fp4.quantize_mxfp4(x)[0])]
+        if K % 128 == 0:
+            forms.append(lambda: fp4.quantize_pack_mxfp4(x, scale_layout="kmajor"))
+            forms.append(lambda: fp4.quantize_pack_mxfp4_many([x, x.contiguous()], scale_layout="kmajor"))
+        if K % 128 == 0 and R % 128 == 0 and x.numel():
+            forms.append(lambda: fp4.quantize_pack_mxfp4_2d(x))
+        for f in forms:
+            assert _same(_outcome(f), _general(monkeypatch, C, f))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 1, 128), (5, 70, 384), (40, 96, 512), (130, 256, 640), (300, 1040, 2048)])
+def test_products_match_the_python_path(C, monkeypatch, M, N, K):
+    from lockstep_amd import dual_gemm, fp4, mxfp4_gemm
+    from lockstep_amd.fp4_linear import MXFP4Linear
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    x, x1, w = (torch.randn(s, device=dev, generator=g) for s in ((M, K), (M, K), (N, K)))
+    (xp, xk), (wp, wk) = (fp4.quantize_pack_mxfp4(t, scale_layout="kmajor") for t in (x, w))
+    xr, wr = fp4.quantize_pack_mxfp4(x)[1], fp4.quantize_pack_mxfp4(w)[1]
+    (xc, xs), (wc, ws) = fp4.quantize_mxfp4(x), fp4.quantize_mxfp4(w)
+    odd = xs * 1.5   # scales that need the promotion
+    wide = torch.zeros((M, K // 2 + 32), dtype=torch.uint8, device=dev)
+    wide[:, :K // 2] = xp
+    forms = []
+    for dt in (torch.float32, torch.bfloat16, torch.float16):
+        for sa, sb in ((xk, wk), (xr, wr), (xs, ws), (xs.clone(), ws), (odd, ws), (xs.t().contiguous().t(), ws)):
+            forms.append(lambda sa=sa, sb=sb, dt=dt: mxfp4_gemm.mxfp4_gemm_packed(xp, wp, sa, sb, out_dtype=dt))
+        forms.append(lambda dt=dt: mxfp4_gemm.mxfp4_gemm_packed(wide[:, :K // 2], wp, xk, wk, out_dtype=dt))
+        a, a1 = x.to(dt), x1.to(dt)
+        pad = torch.zeros((M, K + 8), device=dev, dtype=dt)
+        pad[:, :K] = a
+        for act in (a, pad[:, :K], a.t().contiguous().t()):
+            for sw in (wr, ws):
+                forms.append(lambda act=act, sw=sw: mxfp4_gemm.mxfp4_gemm_bf16(act, wp, sw))
+                forms.append(lambda act=act, sw=sw: mxfp4_gemm.mxfp4_linear_w(act, wp, sw))
+                forms.append(lambda act=act, sw=sw, a1=a1: dual_gemm.dual_mxfp4(act, a1, wp, sw, out_dtype=torch.float32))
+        layer = MXFP4Linear(K, N).to(dev)
+        layer.weight = torch.nn.Parameter(w.to(dt) if dt != torch.float16 else w)
+        for t in (a, a.reshape(1, M, K)):
+            forms.append(lambda layer=layer, t=t: layer(t).detach())
+    if N % 16 == 0:
+        a8, b8 = fp4.codes_to_e4m3(xc), fp4.codes_to_e4m3(wc.t().contiguous())
+        wst = ws.t().contiguous()
+        for sa, sb in ((xs, wst), (odd, wst), (xr, wr.t().contiguous())):
+            forms.append(lambda sa=sa, sb=sb: mxfp4_gemm.mxfp4_gemm_fp8(a8, b8, sa, sb))
+    for f in forms:
+        assert _same(_outcome(f), _general(monkeypatch, C, f))
+
+
+@pytest.mark.gpu
+def test_errors_are_the_python_path_s(C):
+    from lockstep_amd import mxfp4_gemm
+    dev = torch.device("cuda", 0)
+    p = torch.zeros((4, 64), dtype=torch.uint8, device=dev)
+    s = torch.full((4, 4), 127, dtype=torch.uint8, device=dev)
+    with pytest.raises(AssertionError, match="multiple of 128"):
+        mxfp4_gemm.mxfp4_gemm_packed(p[:, :48], p[:, :48], s, s)
+    with pytest.raises(AssertionError, match="scale must be"):
+        mxfp4_gemm.mxfp4_gemm_bf16(torch.zeros((2, 128), device=dev, dtype=torch.bfloat16), p, s[:, :3])
+    with pytest.raises(TypeError):
+        mxfp4_gemm.mxfp4_gemm_packed(p, p, s, s, out_dtype=torch.float64)
+    with pytest.raises(C.LsmxError):
+        C.check(-2)
