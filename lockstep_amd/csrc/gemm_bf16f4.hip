@@ -82,8 +82,14 @@ LSMX_DEV uint32_t load_scale2(const void *s, int64_t off) {
     }
 }
 
+// E8M0 byte -> fp32 scale: 2^(e - 127), with byte 0 -> 2^-127 (0x00400000)
+// and byte 255 -> NaN (0x7FC00000), both of which are (e << 23) | 2^22.
+// Written without selects: the compiler turned a select per special byte into
+// branches on the exec mask in front of every conversion (against a 14336 x
+// 4096 weight M = 1: 7.9 us with them, 7.3 without; M = 4096: 412 and 377).
 LSMX_DEV float e8m0_scale_f32(uint32_t e) {
-    return e == 0u ? u2f(0x00400000u) : (e == 255u ? u2f(0x7FC00000u) : u2f(e << 23));
+    const uint32_t special = ((((e + 1u) & 0xFEu) - 1u) >> 9) & 0x00400000u;
+    return u2f((e << 23) | special);
 }
 
 // BR A rows (all batches) x BN weight columns per workgroup of 4 waves in a
@@ -1086,13 +1092,6 @@ LSMX_DEV u32x4 gload_x4(const void *p) {
     return v;
 }
 
-// E8M0 byte -> fp32 scale without branches: 2^(e - 127), with byte 0 ->
-// 2^-127 (0x00400000) and byte 255 -> NaN (0x7FC00000), both of which are
-// (e << 23) | 2^22.
-LSMX_DEV float e8m0_scale_nb(uint32_t e) {
-    const uint32_t special = ((((e + 1u) & 0xFEu) - 1u) >> 9) & 0x00400000u;
-    return u2f((e << 23) | special);
-}
 // fp32 scale -> itself when it has an E8M0 form (a power of two in
 // [2^-127, 2^127]), else NaN, without branches.
 LSMX_DEV float f32_scale_nb(uint32_t b) {
@@ -1219,7 +1218,7 @@ __global__ __launch_bounds__(dk::NT, 2) void gemm_bf16f4_decode_kernel(GemmArgs 
 #pragma unroll
                     for (int s = 0; s < 16; ++s)
                         sc[s] = SF32 ? f32_scale_nb(sv[t][s >> 2][s & 3])
-                                     : e8m0_scale_nb((sv[t][0][s >> 2] >> (8 * (s & 3))) & 0xFFu);
+                                     : e8m0_scale_f32((sv[t][0][s >> 2] >> (8 * (s & 3))) & 0xFFu);
                 } else {
 #pragma unroll
                     for (int s = 0; s < 16; ++s) sc[s] = u2f(((sv[t][0][s >> 2] >> (8 * (s & 3))) & 0xFFu) << 23);
@@ -1528,7 +1527,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_bf16f4_midm_kernel(GemmArgs g
 #pragma unroll
                 for (int t = 0; t < TN; ++t) {
                     const uint32_t pw = pc[st % 2][t];
-                    const float sc8 = e8m0_scale_nb((sv[t][st >> 4][(st >> 2) & 3] >> (8 * (st & 3))) & 0xFFu);
+                    const float sc8 = e8m0_scale_f32((sv[t][st >> 4][(st >> 2) & 3] >> (8 * (st & 3))) & 0xFFu);
                     const v2bf d0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(pw, sc8, 0);
                     const v2bf d1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(pw, sc8, 1);
                     const v2bf d2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(pw, sc8, 2);
