@@ -537,9 +537,6 @@ LSMX_DEV int swz(int row) { return (row >> 1) & 7; }
 // BR x BN tile (256 x 256 for large M; 128 x 64 and 128 x 128 for M of a few
 // hundred rows, where a 256-row tile would leave most CUs idle and every CU
 // streams all of A), S-slot ring.
-// SPLITK: the workgroup takes K slice blockIdx % splits of its tile (g.k_split
-// deep) and writes its fp32 partial tile to the workspace g.ws;
-// splitk_reduce_kernel then adds the slices in slice order and stores C.
 // WGM x (8 / WGM) waves: 4 x 2 (each wave a quarter of the rows and half of
 // the columns) or, for 128-row tiles, 1 x 8 (each wave all rows and a 32-
 // column strip, so every weight fragment is dequantized by one wave instead
@@ -554,7 +551,7 @@ template <bool V>
 struct LoaderC {
     static constexpr bool value = V;
 };
-template <int NB, int CT, int BR, int BN, int S, bool SPLITK = false, int WGM = 4, int NLW = wr::NW>
+template <int NB, int CT, int BR, int BN, int S, int WGM = 4, int NLW = wr::NW>
 __global__ __launch_bounds__(wr::NT, 1) void gemm_bf16f4_ring_kernel(GemmArgs g) {
     using namespace wr;
     constexpr int RPB = BR / NB;        // A rows per batch per workgroup
@@ -583,14 +580,11 @@ __global__ __launch_bounds__(wr::NT, 1) void gemm_bf16f4_ring_kernel(GemmArgs g)
     __shared__ __attribute__((aligned(16))) uint8_t sNull[XWL * NLW > WW ? 1024 : 16];
 
     const int tiles_m = (int)((g.M + RPB - 1) / RPB), tiles_n = (int)((g.N + BN - 1) / BN);
-    const int tile = SPLITK ? (int)blockIdx.x / g.splits : (int)blockIdx.x;
-    const int split = SPLITK ? (int)blockIdx.x - tile * g.splits : 0;
+    const int tile = (int)blockIdx.x;
     int tm, tn;
     tile_coords(tile, tiles_m, tiles_n, GROUP_M, tm, tn);
     const int64_t m0 = (int64_t)tm * RPB, n0 = (int64_t)tn * BN;
-    // this workgroup's K range: [kb0, kb0 + kdepth)
-    const int64_t kb0 = SPLITK ? (int64_t)split * g.k_split : 0, kdepth = SPLITK ? g.k_split : g.K;
-    const int nk = (int)(kdepth / BK);
+    const int nk = (int)(g.K / BK);
 
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -616,10 +610,10 @@ __global__ __launch_bounds__(wr::NT, 1) void gemm_bf16f4_ring_kernel(GemmArgs g)
         const int rb = r0 - b * RPB;                    // row inside the batch tile
         const int row = r0 + arow_l;
         a_off[i] = (uint32_t)(arow_l * lda_b + (((lane & 7) ^ swz(row)) << 4));
-        a_base[i] = (b ? g.a1 : g.a) + (m0 + rb) * lda_b + kb0 * 2;
+        a_base[i] = (b ? g.a1 : g.a) + (m0 + rb) * lda_b;
         // rows left in the operand from this instruction's first row, at most 8
         const int64_t left = g.M - (m0 + rb), rows = left < 8 ? (left > 0 ? left : 0) : 8;
-        a_bytes[i] = rows > 0 ? (uint64_t)((rows - 1) * lda_b + (g.K - kb0) * 2) : 0;
+        a_bytes[i] = rows > 0 ? (uint64_t)((rows - 1) * lda_b + g.K * 2) : 0;
     }
     // W: load j of loader w covers slot rows (j*NLW + w)*32 .. +31 (when that
     // is below BN), lane -> row lane%32, 16-byte half lane/32
@@ -631,9 +625,9 @@ __global__ __launch_bounds__(wr::NT, 1) void gemm_bf16f4_ring_kernel(GemmArgs g)
     for (int j = 0; j < XWL; ++j) {
         const int wi = j * NLW + wave;
         const bool real = wi < WW;
-        w_base[j] = g.b + (n0 + (real ? wi : 0) * 32) * g.ldb + kb0 / 2;
+        w_base[j] = g.b + (n0 + (real ? wi : 0) * 32) * g.ldb;
         const int64_t left = real ? g.N - (n0 + wi * 32) : 0, rows = left < 32 ? (left > 0 ? left : 0) : 32;
-        w_bytes[j] = rows > 0 ? (uint64_t)((rows - 1) * g.ldb + (g.K - kb0) / 2) : 0;
+        w_bytes[j] = rows > 0 ? (uint64_t)((rows - 1) * g.ldb + g.K / 2) : 0;
         w_lds[j] = real ? lds_u32(&sW[0][0]) + wi * 1024 : lds_u32(&sNull[0]);
         w_slot[j] = real ? W_SLOT : 0;
     }
@@ -642,12 +636,12 @@ __global__ __launch_bounds__(wr::NT, 1) void gemm_bf16f4_ring_kernel(GemmArgs g)
     // same loads)
     const int s_w = wave % SWV;
     const int64_t s_rows = g.N - n0;
-    const uint8_t *s_base = reinterpret_cast<const uint8_t *>(g.sb) + n0 * g.ld_sb + kb0 / 32;
+    const uint8_t *s_base = reinterpret_cast<const uint8_t *>(g.sb) + n0 * g.ld_sb;
     const uint32_t s_off = (uint32_t)(((s_w * 64) + lane) * g.ld_sb);
     auto issue_scales = [&](int grp) __attribute__((always_inline)) {
         const int64_t ks = (int64_t)grp * 16;
         const int64_t rows = s_rows < BN ? s_rows : BN;
-        const uint64_t bytes = (uint64_t)((rows - 1) * g.ld_sb + (g.K - kb0) / 32 - ks);
+        const uint64_t bytes = (uint64_t)((rows - 1) * g.ld_sb + g.K / 32 - ks);
         dma_x4(s_off, buf_rsrc(s_base + ks, bytes), lds_u32(&sS[grp & 1][0]) + s_w * 1024);
     };
 
@@ -790,37 +784,6 @@ __global__ __launch_bounds__(wr::NT, 1) void gemm_bf16f4_ring_kernel(GemmArgs g)
     // no load may still be writing this workgroup's LDS when it exits
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
-    if constexpr (SPLITK) {
-        // The K slice's partial tile goes to partial array `split` of the
-        // workspace, [splits][NB][Mp][Np] fp32 with Mp, Np the tile-padded
-        // sizes, so every store is in bounds; 16-byte stores of 4
-        // consecutive columns after the in-quad transpose.  The reduction
-        // kernel launched next on the stream adds the slices.
-        const int64_t Mp = (int64_t)tiles_m * RPB, Np = (int64_t)tiles_n * BN;
-        const int bq = NB == 2 ? (wm * TM * 32) / RPB : 0;
-        float *pbase = g.ws + ((int64_t)split * NB + bq) * Mp * Np;
-        const int64_t prow0 = m0 + wm * (TM * 32) - bq * RPB, pcol0 = n0 + wn * (TN * 32);
-        const int q = frow & 3;
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int gq = 0; gq < 4; ++gq)
-#pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    float x[4] = {acc[i][j][4 * gq], acc[i][j][4 * gq + 1], acc[i][j][4 * gq + 2],
-                                  acc[i][j][4 * gq + 3]};
-                    quad_transpose(x, q);
-                    const int64_t row = prow0 + i * 32 + 8 * gq + 4 * half + q;
-                    // rows past M are never read by the reduction; streaming
-                    // stores (the reduction kernel reads each value once)
-                    if (row < g.M)
-                        __builtin_nontemporal_store(u32x4{f2u(x[0]), f2u(x[1]), f2u(x[2]), f2u(x[3])},
-                                                    reinterpret_cast<u32x4 *>(pbase + row * Np + pcol0 + j * 32 +
-                                                                              (frow & ~3)));
-                }
-        return;
-    }
-
     // epilogue: acc element e of tile (i, j) is row i*32 + 8*(e/4) + 4*half + e%4, column j*32 + frow
     const int b = NB == 2 ? (wm * TM * 32) / RPB : 0;
     void *cb = b ? g.c1 : g.c;
@@ -890,7 +853,7 @@ static hipError_t launch_ring(const GemmArgs &g, hipStream_t s) {
     constexpr int RPB = BR / NB;
     const int tiles = (int)(((g.M + RPB - 1) / RPB) * ((g.N + BN - 1) / BN));
     const dim3 grid(tiles), blk(wr::NT);
-#define LSMX_R(CT) hipLaunchKernelGGL((gemm_bf16f4_ring_kernel<NB, CT, BR, BN, S, false, WGM, NLW>), grid, blk, 0, s, g)
+#define LSMX_R(CT) hipLaunchKernelGGL((gemm_bf16f4_ring_kernel<NB, CT, BR, BN, S, WGM, NLW>), grid, blk, 0, s, g)
     if (g.c_dtype == LSMX_F32) LSMX_R(LSMX_F32);
     else if (g.c_dtype == LSMX_BF16) LSMX_R(LSMX_BF16);
     else LSMX_R(LSMX_F16);
@@ -1328,284 +1291,6 @@ static bool decode_ok(const GemmArgs &g) {
     return g.K % dk::SLICE_K == 0 && (reinterpret_cast<uintptr_t>(g.sb) & 15) == 0 && g.ld_sb % 16 == 0;
 }
 
-// ------------------------------------------------------------------ mid M
-// 17 to 64 activation rows per batch: the decode kernel's weight layout, with
-// the activations streamed instead of held.
-//   - a workgroup owns the weight rows the decode kernel would give it (the
-//     weight spread evenly over the CUs, at most 64 rows, four 16-row MFMA
-//     tiles) and the whole K: its 8 waves split each 4096-deep pass into
-//     512-deep slices, each wave's slice of every row loaded once into LDS
-//     (the decode kernel's 4-row, 256-byte direct-to-LDS loads and chunk
-//     swizzle) together with its 16 E8M0 scale bytes per row;
-//   - the activation rows are processed in groups of 64 (4 MFMA tiles; the
-//     dual form's 2M virtual rows can make two): for each 32-deep K-step of
-//     its slice a wave loads the group's fragments row-contiguous (lane l:
-//     16-byte piece l%4 of row l/4, so a quarter-wave touches 4 rows, not
-//     16) in pairs of steps (both halves of each 128-byte line together), a
-//     pair or two ahead, moves them to the MFMA layout with ds_bpermute and
-//     reads the step's weight code words one step ahead of its 16
-//     independent v_mfma_f32_16x16x32_bf16, dequantizing them just before
-//     (v_cvt_scalef32_pk_bf16_fp4, exact); with one pass (K <= 4096) the
-//     weight slice stays in LDS for every group;
-//   - the 8 waves' partial sums of a group meet in a separate 32 KiB LDS
-//     buffer, one activation tile at a time, and are added in wave order.
-// No partial tiles go to memory and there is no second launch (the split-K
-// ring's cost at these shapes).  The summation order of an output element
-// depends on K only, so single and dual launches of the same M give
-// identical bits.
-namespace mk {
-constexpr int PASS_K = 4096;                     // K per pass (all waves' slices)
-constexpr int R = 64, TN = R / 16;               // weight rows (at most), 16-row MFMA tiles
-constexpr int MT = 4, GROUP = 16 * MT;           // activation tiles per group, rows per group
-}  // namespace mk
-
-template <int I, int N, typename F>
-LSMX_DEV void static_for(F &&f) {
-    if constexpr (I < N) {
-        f(SlotC<I>{});
-        static_for<I + 1, N>(f);
-    }
-}
-template <int N>
-LSMX_DEV void wait_vmcnt() {
-    static_assert(N >= 0 && N < 64, "vmcnt range");
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-// NW waves (each a PASS_K / NW deep slice of K), activation step pairs
-// loaded PD pairs ahead of the pair in use.
-template <int NW, int PD, int CT>
-__global__ __launch_bounds__(64 * NW, 1) void gemm_bf16f4_midm_kernel(GemmArgs g) {
-    using namespace mk;
-    constexpr int NT = 64 * NW, SLICE_K = PASS_K / NW, STEPS = SLICE_K / 32, NPAIR = STEPS / 2;
-    constexpr int H = SLICE_K / 512;                // 256-byte halves of a row's slice
-    constexpr int XW = (R / 4) * H;                 // weight loads per wave per pass (4 rows x 256 bytes)
-    constexpr int SV = SLICE_K / 512;               // 16-byte E8M0 vectors per row per slice
-    constexpr int NSLOT = 2 * (PD + 1);             // activation fragment slots (steps)
-    __shared__ __attribute__((aligned(16))) uint8_t sW[NW][H][R * 256];   // 128 KiB
-    __shared__ __attribute__((aligned(16))) float red[NW][TN * 256];
-
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int n16 = lane & 15, q = lane >> 4;
-    const bool dual = g.a1 != nullptr;
-    const int64_t VM = dual ? 2 * g.M : g.M;
-    const int64_t n0 = (int64_t)blockIdx.x * g.rows_wg;
-    const int64_t nend = min(n0 + g.rows_wg, g.N);   // rows past nend read zeros
-    const bool one_pass = g.K <= PASS_K;
-
-    // scale rows of this lane's weight rows (rows past nend repeat the last one)
-    const uint8_t *srow[TN];
-#pragma unroll
-    for (int t = 0; t < TN; ++t)
-        srow[t] = reinterpret_cast<const uint8_t *>(g.sb) + min(n0 + 16 * t + n16, nend - 1) * g.ld_sb;
-    // weight load (j, h) covers rows 4j .. 4j + 3, bytes 256h .. 256h + 255 of
-    // their slices: lane l -> row 4j + l/16, LDS chunk l%16 holding source
-    // chunk (l%16) ^ (row & 15)
-    uint32_t w_off[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int r = 4 * j + (lane >> 4);
-        w_off[j] = (uint32_t)((lane >> 4) * g.ldb + 16 * ((lane & 15) ^ (r & 15)));
-    }
-    u32x4 sv[TN][SV];
-    // byte address of the lane that loaded this lane's MFMA piece
-    const int src4 = 4 * (4 * n16 + q);
-
-#pragma nounroll
-    for (int64_t vg = 0; vg < VM; vg += GROUP) {
-        // Activation fragments are loaded row-contiguous -- lane l reads the
-        // 16-byte piece l%4 of row l/4 of the tile's 64-byte step segment, so
-        // a quarter-wave touches 4 rows instead of 16 -- and moved to the MFMA
-        // layout (lane (n16, q): row n16, piece q) with ds_bpermute.  Rows
-        // past VM repeat the last one; their outputs are not stored.
-        const uint8_t *arow[MT];
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            const int64_t v = min(vg + 16 * mt + (lane >> 2), VM - 1);
-            const bool second = dual && v >= g.M;
-            arow[mt] = (second ? g.a1 : g.a) + (second ? v - g.M : v) * g.lda * 2 + (lane & 3) * 16;
-        }
-        v4f acc[MT][TN];
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int t = 0; t < TN; ++t) acc[mt][t] = v4f{0.f, 0.f, 0.f, 0.f};
-
-#pragma nounroll
-        for (int64_t kp = 0; kp < g.K; kp += PASS_K) {
-            const int64_t k0 = kp + (int64_t)wave * SLICE_K;   // this wave's slice
-            const bool live = k0 < g.K;                         // K % SLICE_K == 0: whole slices
-            const bool load_w = vg == 0 || !one_pass;
-            // every wave is done with the LDS slice it is about to overwrite
-            if (load_w && kp > 0) __syncthreads();
-            if (!live) continue;
-            // The scales and the weight slice (when not already in LDS), then
-            // the first PD + 1 pairs of steps' activation fragments: asm
-            // loads, all counted by the explicit waits below, in issue order,
-            // so the wait for step 0's fragments also covers the weights.
-            if (load_w) {
-#pragma unroll
-                for (int t = 0; t < TN; ++t)
-#pragma unroll
-                    for (int v = 0; v < SV; ++v) sv[t][v] = gload_x4(srow[t] + k0 / 32 + 16 * v);
-#pragma unroll
-                for (int j = 0; j < R / 4; ++j) {
-                    const int64_t r0 = n0 + 4 * j, left = nend - r0;
-                    const uint64_t bytes = left > 0 ? (uint64_t)((left - 1) * g.ldb + (g.K - k0) / 2) : 0;
-#pragma unroll
-                    for (int h = 0; h < H; ++h)
-                        dma_x4(w_off[j & 3], buf_rsrc(g.b + r0 * g.ldb + k0 / 2 + 256 * h, bytes > 256u * h ? bytes - 256u * h : 0),
-                               lds_u32(&sW[wave][h][0]) + j * 1024);
-                }
-            }
-            // Steps s and s + 1 (s even) are loaded back to back per tile, so
-            // the two 64-byte halves of each 128-byte line are requested
-            // together (one line fill).
-            u32x4 af[NSLOT][MT];
-            auto fetch2 = [&](int s) __attribute__((always_inline)) {
-                const uint32_t off0 = (uint32_t)(k0 * 2) + 64u * (uint32_t)s;
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt) {
-                    af[s % NSLOT][mt] = gload_x4(arow[mt] + off0);
-                    af[(s + 1) % NSLOT][mt] = gload_x4(arow[mt] + off0 + 64);
-                }
-            };
-            // A step's operands (the permuted activation fragments ab and the
-            // weight code words pc) are prepared one step ahead, so their LDS
-            // latencies overlap the previous step's MFMAs.
-            auto prep = [&](int s, u32x4 (&ab)[MT], uint32_t (&pc)[TN]) __attribute__((always_inline)) {
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt) {
-                    asm volatile("" : "+v"(af[s % NSLOT][mt]));
-                    const u32x4 v = af[s % NSLOT][mt];
-                    ab[mt] = u32x4{(uint32_t)__builtin_amdgcn_ds_bpermute(src4, (int)v.x),
-                                   (uint32_t)__builtin_amdgcn_ds_bpermute(src4, (int)v.y),
-                                   (uint32_t)__builtin_amdgcn_ds_bpermute(src4, (int)v.z),
-                                   (uint32_t)__builtin_amdgcn_ds_bpermute(src4, (int)v.w)};
-                }
-                const int h = s >> 4, c = s & 15;
-#pragma unroll
-                for (int t = 0; t < TN; ++t)
-                    pc[t] = *reinterpret_cast<const uint32_t *>(&sW[wave][h][(16 * t + n16) * 256 + 16 * (c ^ n16) + 4 * q]);
-            };
-            // Pair p (steps 2p, 2p + 1) is issued in the prologue for p <= PD,
-            // else at the end of step 2(p - PD) - 1.  wait_for<s, cur>: step
-            // s's fragments have landed, given the pairs issued by step cur;
-            // what may stay in flight is what was issued after step s's last
-            // fragment (that of tile MT - 1).
-            auto wait_for = [&](auto sc, auto cc) __attribute__((always_inline)) {
-                constexpr int st = decltype(sc)::value, cur = decltype(cc)::value;
-                constexpr int newest = (PD + (cur + 1) / 2) < NPAIR - 1 ? PD + (cur + 1) / 2 : NPAIR - 1;
-                constexpr int ahead = st % 2 == 0 ? 1 + (newest - st / 2) * 2 * MT : (newest - (st - 1) / 2) * 2 * MT;
-                __builtin_amdgcn_sched_barrier(0);
-                wait_vmcnt<ahead>();
-                __builtin_amdgcn_sched_barrier(0);
-            };
-#pragma unroll
-            for (int p = 0; p <= PD; ++p) fetch2(2 * p);
-            wait_for(SlotC<0>{}, SlotC<-1>{});
-            if (load_w) {
-#pragma unroll
-                for (int t = 0; t < TN; ++t)
-#pragma unroll
-                    for (int v = 0; v < SV; ++v) asm volatile("" : "+v"(sv[t][v]));
-            }
-            u32x4 ab[2][MT];
-            uint32_t pc[2][TN];
-            prep(0, ab[0], pc[0]);
-            static_for<0, STEPS>([&](auto sc) __attribute__((always_inline)) {
-                constexpr int st = decltype(sc)::value;
-                // the pair PD + 1 ahead of the one ending here
-                if constexpr (st % 2 == 1 && (st + 1) / 2 + PD < NPAIR) fetch2(2 * ((st + 1) / 2 + PD));
-                if constexpr (st + 1 < STEPS) {
-                    wait_for(SlotC<st + 1>{}, SlotC<st>{});
-                    prep(st + 1, ab[(st + 1) % 2], pc[(st + 1) % 2]);
-                }
-                // dequantize the step's weight fragments (exact, block scale applied)
-                v8bf wf[TN];
-#pragma unroll
-                for (int t = 0; t < TN; ++t) {
-                    const uint32_t pw = pc[st % 2][t];
-                    const float sc8 = e8m0_scale_f32((sv[t][st >> 4][(st >> 2) & 3] >> (8 * (st & 3))) & 0xFFu);
-                    const v2bf d0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(pw, sc8, 0);
-                    const v2bf d1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(pw, sc8, 1);
-                    const v2bf d2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(pw, sc8, 2);
-                    const v2bf d3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(pw, sc8, 3);
-                    wf[t] = v8bf{d0[0], d0[1], d1[0], d1[1], d2[0], d2[1], d3[0], d3[1]};
-                }
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                    for (int t = 0; t < TN; ++t)
-                        acc[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                            __builtin_bit_cast(v8bf, ab[st % 2][mt]), wf[t], acc[mt][t], 0, 0, 0);
-            });
-        }
-
-        // acc[mt][t][r] = D[4q + r][n16] of the 16 x 16 tile (rows: activation
-        // rows vg + 16 mt .., columns: weight rows 16 t ..); one activation
-        // tile at a time, the waves' partial sums are added in wave order
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            __syncthreads();
-#pragma unroll
-            for (int t = 0; t < TN; ++t)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) red[wave][t * 256 + r * 64 + lane] = acc[mt][t][r];
-            __syncthreads();
-            for (int o = threadIdx.x; o < TN * 256; o += NT) {
-                float v = 0.f;
-#pragma unroll
-                for (int w = 0; w < NW; ++w) v += red[w][o];
-                const int t = o >> 8, e = o & 255, r = e >> 6, l = e & 63;
-                const int64_t vr = vg + 16 * mt + 4 * (l >> 4) + r, n = n0 + 16 * t + (l & 15);
-                if (vr < VM && n < nend) {
-                    const bool second = dual && vr >= g.M;
-                    store_cw<CT>(second ? g.c1 : g.c, (second ? vr - g.M : vr) * g.ldc + n, v);
-                }
-            }
-        }
-    }
-}
-
-// 8 waves with the next pair in flight: 4 waves (one per SIMD, 512
-// registers) with 2 or 3 pairs in flight measured 11-16% slower at M = 32,
-// 64 and 128 (cfg3's weight, one box)
-constexpr int kMidNW = 8, kMidPD = 1;
-template <int CT>
-static void launch_midm_ct(GemmArgs g, hipStream_t s) {
-    const int64_t cus = num_cus_w(), per = (g.N + cus - 1) / cus, rows = (per + 3) / 4 * 4;
-    g.rows_wg = (int)(rows > mk::R ? mk::R : rows < 16 ? 16 : rows);
-    const dim3 grid((unsigned)((g.N + g.rows_wg - 1) / g.rows_wg)), blk(64 * kMidNW);
-    hipLaunchKernelGGL((gemm_bf16f4_midm_kernel<kMidNW, kMidPD, CT>), grid, blk, 0, s, g);
-}
-
-static hipError_t launch_midm(const GemmArgs &g, hipStream_t s) {
-    if (g.c_dtype == LSMX_F32) launch_midm_ct<LSMX_F32>(g, s);
-    else if (g.c_dtype == LSMX_BF16) launch_midm_ct<LSMX_BF16>(g, s);
-    else launch_midm_ct<LSMX_F16>(g, s);
-    return hipGetLastError();
-}
-
-// Per-batch rows the mid-M kernel takes (above the decode kernel's).  Up to
-// 64 it beats the skinny and split-K kernels at cfg3's weight (M = 32: 20.3
-// against 26.3 us, M = 64: 21.0 against 27.1, the dual form of M = 64: 33.5
-// against 38.9); at M = 128 the activation stream through each CU's vector
-// memory path makes it slower than split-K (33.5 against 29.5).
-constexpr int64_t kMidMaxM = 64;
-// The shape test (M, N, K only, so that the split-K workspace query agrees):
-// whole 512-deep K slices, the weight spread as the decode kernel spreads it
-// (at most 64 rows per workgroup) over at least one workgroup per CU.
-static bool midm_shape(int64_t M, int64_t N, int64_t K) {
-    const int64_t cus = num_cus_w();
-    return M > kDecodeMaxM && M <= kMidMaxM && K % (mk::PASS_K / kMidNW) == 0 && N >= 16 * cus && (N + cus - 1) / cus <= mk::R;
-}
-// and E8M0 byte scales in 16-byte aligned rows (the decode kernel's scale loads)
-static bool midm_ok(const GemmArgs &g) {
-    return g.scale_fmt == LSMX_SCALE_E8M0 && decode_ok(g) && midm_shape(g.M, g.N, g.K);
-}
-
 // ------------------------------------------------------------------ GEMV
 // For one or two activation rows per batch (decode) the whole cost is reading
 // W once, and the matrix cores have almost nothing to do.  This kernel reads
@@ -1878,75 +1563,366 @@ static hipError_t launch_w4(const GemmArgs &g, hipStream_t s) {
     return hipGetLastError();
 }
 
-// the ring kernel (256 x 256 tiles) from half a wave of tiles on, else the
-// largest VGPR-staged tile that still gives every CU a workgroup: 256 x 256,
-// then 128 x 128, then 128 x 64 (mid M, e.g. 128 rows against 14336 columns)
+// What the tile kernel does not take (fp32 scales, rows that are not 4-byte
+// aligned): the largest VGPR-staged tile that still gives every CU a
+// workgroup: 256 x 256, then 128 x 128, then 128 x 64
 template <int NB>
 static hipError_t launch_w4_any(const GemmArgs &g, hipStream_t s) {
     auto tiles = [&](int br, int bn) { return ((g.M + br / NB - 1) / (br / NB)) * ((g.N + bn - 1) / bn); };
     const int64_t cus = num_cus_w();
-    // the ring kernel is worth it from half a wave of 256 x 256 tiles on (M = 1024, N = 14336: 224 tiles)
-    // single form whose 256 x 256 tiles leave CUs idle while 128 x 256 tiles
-    // still fit in one wave of workgroups: 128-row tiles, 1 x 8 waves (each
-    // all 128 rows and a 32-column strip), loads from waves 0-3.  cfg2's
-    // single batch (M = 2048 against a 4096 x 4096 weight, 128 -> 256
-    // workgroups) 97 -> 63 us; M = 1024 against 8192 x 4096 91 -> 62 us
-    if constexpr (NB == 1)
-        if (ring_ok(g) && tiles(256, 256) < cus && tiles(128, 256) <= cus &&
-            2 * tiles(128, 256) > cus)
-            return launch_ring<NB, 128, 256, 4, 1, 4>(g, s);
-    if (ring_ok(g) && 2 * tiles(256, 256) >= cus) return launch_ring<NB, 256, 256, 3, 2, 4>(g, s);
     if (tiles(256, 256) >= cus) return launch_w4<NB, 256, 256>(g, s);
     if (tiles(128, 128) >= cus) return launch_w4<NB, 128, 128>(g, s);
-    // a few hundred rows: 128 x 64 tiles through a 4-slot DMA ring (N =
-    // 14336, K = 4096, M = 128: 48 -> 38 us; M = 64: 44 -> 35 us against the skinny kernel)
-    if (ring_ok(g)) return launch_ring<NB, 128, 64, 4>(g, s);
     return launch_w4<NB, 128, 64>(g, s);
 }
 
-// ------------------------------------------------------------------ split-K
-// A few hundred activation rows against a wide weight (M = 128, N = 14336:
-// 56 output tiles of 128 x 256 for 256 CUs) leave most CUs idle with whole-K
-// tiles, and narrower tiles make every CU re-read the whole activation
-// panel.  Instead each output tile of 128 rows (per batch) by 256 or 128
-// weight columns is cut into 2 or 4 K slices (>= 512 deep, a whole group of
-// E8M0 scale loads), one workgroup each; the fp32 partial tiles meet in a
-// caller-provided workspace.  Of the plans that fit one wave of workgroups,
-// the one with the most workgroups wins, and among those the one with the
-// fewest partial bytes: M = 128 against N = 14336 runs 112 tiles of 128 x
-// 128 in 2 slices (224 workgroups, 14.7 MB of partials) rather than 56 tiles
-// of 128 x 256 in 4.  The plan depends on M, N and K only (128-row tiles per
-// batch in both forms), so the single and the dual launch of one M give
-// identical bits.
-struct SplitPlan {
-    int splits, bn;
+// ------------------------------------------------------------------ tiles
+// 17 activation rows up to where the 256 x 256 ring fills the CUs: one tile of
+// BM rows x BN weight columns of one batch per workgroup, WM x WN MFMA waves
+// of TM x TN 32 x 32 tiles each, and 4 loader waves.
+//
+// What bounds it: at few rows the stream of weights and, per weight column
+// tile, the re-reading of the activations from L2; at a few hundred rows the
+// matrix cores, and before that tiles that do not divide the CUs evenly.  So
+// the tile and the number of K slices are chosen by the shape (bf16f4_plan).
+// A stage is 128 K: 256 bytes of every A row, 64 bytes (4 MX blocks) of every
+// weight row.  The ring is as deep as the LDS allows and the loads come from
+// waves of their own, since an MFMA behind a load that waits for a place in
+// the memory pipeline would wait too.  E8M0 scales (row-major) come 16 bytes
+// per weight row, 4 stages, at a time.
+//
+// K order: sub-stage g (64 K), K-step st: lane half h supplies A[row][64 g +
+// 32 h + 8 st .. +8] and codes 8 st .. of W's block 2 g + h -- the ring
+// kernel's order, so a whole-K output has the ring kernel's bits whatever
+// the tile.  With g.splits > 1 workgroup (tile, slice) sums its run of
+// stages and writes an fp32 partial tile; splitk_reduce_kernel adds the
+// slices in slice order.
+namespace wt {
+constexpr int BK = 128, NLW = 4, GROUP_M = 4;
+constexpr int A_ROW_B = BK * 2, W_ROW_B = BK / 2;
+constexpr int lds(int bm, int bn, int s) { return s * (bm * A_ROW_B + bn * W_ROW_B) + ((s + 3) / 4 + 1) * bn * 16; }
+// two workgroups per CU where the LDS holds both rings
+constexpr int waves_per_simd(int bm, int bn, int s, int waves) { return waves / 4 * (2 * lds(bm, bn, s) <= 160 * 1024 ? 2 : 1); }
+}  // namespace wt
+template <int CT, bool SPLITK, int WM, int WN, int TM, int TN, int S, int LA>
+__global__ __launch_bounds__(64 * (WM * WN + wt::NLW), wt::waves_per_simd(32 * TM * WM, 32 * TN * WN, S, WM * WN + wt::NLW))
+void gemm_bf16f4_tile_kernel(GemmArgs g) {
+    using namespace wt;
+    constexpr int NMW = WM * WN;
+    constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN;
+    constexpr int A_SLOT = BM * A_ROW_B, SLOT = A_SLOT + BN * W_ROW_B;
+    constexpr int XA = BM / (4 * NLW), XW = BN / (16 * NLW), L = XA + XW;   // loads per loader lane per stage
+    constexpr int NSB = (S + 3) / 4 + 1;            // scale buffers: groups of 4 stages in use or in flight
+    constexpr int NSG = (BN + 63) / 64;             // 64-row scale loads per group
+    static_assert(XA * 4 * NLW == BM && XW * 16 * NLW == BN, "whole DMA instructions");
+    static_assert(lds(BM, BN, S) <= 160 * 1024 && (S - 1) * (L + 1) < 63, "LDS, vmcnt");
+    constexpr int OFF_S = S * SLOT;
+    __shared__ __attribute__((aligned(16))) uint8_t ring[lds(BM, BN, S)];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nb = g.a1 ? 2 : 1;
+    const int tiles_m = (int)((g.M + BM - 1) / BM), tiles_n = (int)((g.N + BN - 1) / BN);
+    // blockIdx -> (tile, batch, K slice): the batches of one (m, n) tile are
+    // neighbours, which share its weights in L2
+    int id = (int)blockIdx.x;
+    if ((gridDim.x & 7) == 0) id = (id & 7) * ((int)gridDim.x >> 3) + (id >> 3);
+    const int split = SPLITK ? id % g.splits : 0;
+    if (SPLITK) id /= g.splits;
+    const int batch = nb == 2 ? (id & 1) : 0;
+    int tm, tn;
+    group_coords(nb == 2 ? id >> 1 : id, make_tile_map(tiles_m, tiles_n, GROUP_M), tm, tn);
+    const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
+    // this slice's stages
+    const int nk_all = (int)(g.K / BK);
+    const int k0 = SPLITK ? (int)((int64_t)nk_all * split / g.splits) : 0;
+    const int nk = (SPLITK ? (int)((int64_t)nk_all * (split + 1) / g.splits) : nk_all) - k0;
+
+    if (wave >= NMW) {
+        // ---- loader waves
+        __builtin_amdgcn_s_setprio(3);
+        const int lw = wave - NMW;
+        // A load i: rows (i * 4 + lw) * 4 + lane / 16, LDS chunk lane % 16
+        // holding source chunk (lane % 16) ^ (row & 15)
+        const int ar = lw * 4 + (lane >> 4);
+        const uint32_t a_off = (uint32_t)(ar * g.lda * 2 + (((lane & 15) ^ (ar & 15)) << 4));
+        const uint32_t a_step = (uint32_t)(4 * NLW * g.lda * 2);
+        // W load i: rows (i * 4 + lw) * 16 + lane / 4, LDS chunk lane % 4
+        // holding source chunk (lane % 4) ^ ((row >> 2) & 3)
+        const int wrw = lw * 16 + (lane >> 2);
+        const uint32_t w_off = (uint32_t)(wrw * g.ldb + (((lane & 3) ^ ((wrw >> 2) & 3)) << 4));
+        const uint32_t w_step = (uint32_t)(16 * NLW * g.ldb);
+        const int sg = lw < NSG ? lw : NSG - 1;     // this wave's 64 rows of scales (the last ones repeat)
+        const uint32_t s_off = (uint32_t)((sg * 64 + lane) * g.ld_sb);
+        const int64_t nrow = min(g.N - n0, (int64_t)BN);
+        const uint8_t *pa = (batch ? g.a1 : g.a) + m0 * g.lda * 2 + (int64_t)k0 * A_ROW_B;
+        const uint8_t *pw = g.b + n0 * g.ldb + (int64_t)k0 * W_ROW_B;
+        const uint8_t *ps = reinterpret_cast<const uint8_t *>(g.sb) + n0 * g.ld_sb + (int64_t)k0 * (BK / 32);
+        const int64_t kl = g.K - (int64_t)k0 * BK;  // K left from this slice's start
+        const int64_t na = ((min(g.M - m0, (int64_t)BM) - 1) * g.lda + kl) * 2;
+        const int64_t nw = (nrow - 1) * g.ldb + kl / 2;
+        const int64_t ns = (nrow - 1) * g.ld_sb + kl / 32;
+        const uint32_t ring0 = lds_u32(&ring[0]);
+        auto load_stage = [&](int kt, uint32_t so) __attribute__((always_inline)) {
+            const bool past = kt >= nk;   // refills past the end: empty descriptors, zeros
+            // the scales of stages kt .. kt + 3, ahead of the first of them;
+            // bytes past a row's end are other scales or zeros, never used
+            if ((kt & 3) == 0) {
+                const int64_t o = (int64_t)kt * (BK / 32);
+                dma_x4(s_off, buf_rsrc(ps + (past ? 0 : o), past ? 0 : (uint64_t)(ns - o)),
+                       ring0 + OFF_S + ((kt >> 2) % NSB) * (BN * 16) + sg * 1024);
+            }
+            const int64_t ao = (int64_t)kt * A_ROW_B, wo = (int64_t)kt * W_ROW_B;
+            const v4i_rsrc ra = buf_rsrc(pa + (past ? 0 : ao), past ? 0 : (uint64_t)(na - ao));
+            const v4i_rsrc rw = buf_rsrc(pw + (past ? 0 : wo), past ? 0 : (uint64_t)(nw - wo));
+#pragma unroll
+            for (int i = 0; i < XW; ++i) dma_x4(w_off + i * w_step, rw, ring0 + so + A_SLOT + (i * NLW + lw) * 1024);
+#pragma unroll
+            for (int i = 0; i < XA; ++i) dma_x4(a_off + i * a_step, ra, ring0 + so + (i * NLW + lw) * 1024);
+        };
+#pragma unroll
+        for (int q = 0; q < S; ++q) load_stage(q, q * SLOT);
+        // (the scale loads among the newest only make these waits stricter)
+        wait_vm_barrier<(S - 1) * L>();
+        uint32_t so = 0;
+        for (int kt = 0; kt < nk; ++kt) {
+            wait_vm_barrier<(S - 2) * L>();
+            load_stage(kt + S, so);
+            so = so + SLOT == S * SLOT ? 0 : so + SLOT;
+        }
+        // no load may still be writing this workgroup's LDS when it exits
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        return;
+    }
+
+    // ---- MFMA waves
+    const int wm = wave / WN, wn = wave % WN;
+    const int frow = lane & 31, half = lane >> 5;
+    uint32_t aoff[4];   // A chunk 4 half + st of row frow; sub-stage g flips bit 3 of the chunk
+#pragma unroll
+    for (int st = 0; st < 4; ++st)
+        aoff[st] = (uint32_t)((wm * TM * 32 + frow) * A_ROW_B + (((4 * half + st) ^ (frow & 15)) << 4));
+    uint32_t woff[2];   // W chunk 2 g + half of row frow
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+        woff[q] = (uint32_t)(A_SLOT + (wn * TN * 32 + frow) * W_ROW_B + (((2 * q + half) ^ ((frow >> 2) & 3)) << 4));
+    const uint32_t soff = (uint32_t)(OFF_S + (wn * TN * 32 + frow) * 16);
+    v16f acc[TM][TN];
+    v8bf fa[2][LA][TM];     // A fragments of LA K-steps, and of the next LA
+    u32x4 wb[2][TN];        // weight blocks of the sub-stage in use and of the next one
+    uint32_t sraw[TN], snext[TN];
+    float sc[TN];
+    auto read_a = [&](uint32_t so, int k, int i) __attribute__((always_inline)) {   // K-step k = 4 g + st
+        fa[(k / LA) & 1][k % LA][i] = *reinterpret_cast<const v8bf *>(&ring[0] + so + i * 32 * A_ROW_B + (aoff[k & 3] ^ ((k >> 2) << 7)));
+    };
+    auto read_w = [&](uint32_t so, int gq, int j) __attribute__((always_inline)) {
+        wb[gq][j] = *reinterpret_cast<const u32x4 *>(&ring[0] + so + j * 32 * W_ROW_B + woff[gq]);
+    };
+    auto read_s = [&](int kt, int j) __attribute__((always_inline)) {
+        snext[j] = *reinterpret_cast<const uint32_t *>(&ring[0] + soff + ((kt >> 2) % NSB) * (BN * 16) + (kt & 3) * 4 +
+                                                       j * 32 * 16);
+    };
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+    asm volatile("s_barrier" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < TN; ++j) read_s(0, j);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) read_w(0, 0, j);
+#pragma unroll
+    for (int k = 0; k < LA; ++k)
+#pragma unroll
+        for (int i = 0; i < TM; ++i) read_a(0, k, i);
+    uint32_t so = 0;
+    for (int kt = 0; kt < nk; ++kt) {
+        const uint32_t sn = so + SLOT == S * SLOT ? 0 : so + SLOT;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) sraw[j] = snext[j];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int gq = k >> 2, st = k & 3;
+            if (k == 8 - LA) {
+                // this wave's reads of the slot are complete; past the
+                // barrier it may be refilled and stage kt + 1 has landed
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            v8bf fw[TN];
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                if (st == 0) sc[j] = e8m0_scale_f32((sraw[j] >> (8 * (2 * gq + half))) & 0xFFu);
+                const uint32_t p = wb[gq][j][st];
+                const v2bf d0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(p, sc[j], 0);
+                const v2bf d1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(p, sc[j], 1);
+                const v2bf d2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(p, sc[j], 2);
+                const v2bf d3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(p, sc[j], 3);
+                fw[j] = v8bf{d0[0], d0[1], d1[0], d1[1], d2[0], d2[1], d3[0], d3[1]};
+            }
+            // every LA K-steps the A fragments of the next LA; the weight
+            // blocks a sub-stage ahead; the next stage's scales with its first
+            // fragments
+            if (k % LA == 0) {
+                if (k == 0)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) read_w(so, 1, j);
+                if (k == 8 - LA)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) {
+                        read_s(kt + 1, j);
+                        read_w(sn, 0, j);
+                    }
+#pragma unroll
+                for (int x = 0; x < LA; ++x)
+#pragma unroll
+                    for (int i = 0; i < TM; ++i) read_a(k < 8 - LA ? so : sn, (k + LA + x) & 7, i);
+            }
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[(k / LA) & 1][k % LA][i], fw[j], acc[i][j], 0, 0, 0);
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        so = sn;
+    }
+
+    // ---- epilogue: acc element e of tile (i, j) sits at row i*32 + 8*(e/4) +
+    //      4*half + e%4, column j*32 + frow; a 4x4 transpose inside each quad
+    //      of lanes gives every lane 4 consecutive columns of one row
+    const int q = frow & 3;
+    if constexpr (SPLITK) {
+        // partial tile of this slice: [splits][nb][Mp][Np], Mp and Np padded
+        // to whole tiles, so every store is in bounds
+        const int64_t Mp = (int64_t)tiles_m * BM, Np = (int64_t)tiles_n * BN;
+        float *pt = g.ws + ((int64_t)split * nb + batch) * Mp * Np;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int gr = 0; gr < 4; ++gr) {
+                const int64_t row = m0 + (wm * TM + i) * 32 + 8 * gr + 4 * half + q;
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    float x[4] = {acc[i][j][4 * gr], acc[i][j][4 * gr + 1], acc[i][j][4 * gr + 2], acc[i][j][4 * gr + 3]};
+                    quad_transpose(x, q);
+                    const int64_t col = n0 + (wn * TN + j) * 32 + (frow & ~3);
+                    // rows past M are never read by the reduction, which reads
+                    // each other value once
+                    if (row < g.M)
+                        __builtin_nontemporal_store(u32x4{f2u(x[0]), f2u(x[1]), f2u(x[2]), f2u(x[3])},
+                                                    reinterpret_cast<u32x4 *>(pt + row * Np + col));
+                }
+            }
+    } else {
+        void *c = batch ? g.c1 : g.c;
+        const bool vec_c = (reinterpret_cast<uintptr_t>(c) & 15) == 0 && g.ldc % 8 == 0;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int gr = 0; gr < 4; ++gr) {
+                const int64_t row = m0 + (wm * TM + i) * 32 + 8 * gr + 4 * half + q;
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    float x[4] = {acc[i][j][4 * gr], acc[i][j][4 * gr + 1], acc[i][j][4 * gr + 2], acc[i][j][4 * gr + 3]};
+                    // all four lanes of a quad take part in the exchanges
+                    quad_transpose(x, q);
+                    const int64_t col = n0 + (wn * TN + j) * 32 + (frow & ~3);
+                    if (row < g.M && col < g.N) {
+                        if (vec_c && col + 4 <= g.N) store_c4<CT>(c, row * g.ldc + col, x[0], x[1], x[2], x[3]);
+                        else
+#pragma unroll
+                            for (int k = 0; k < 4; ++k)
+                                if (col + k < g.N) store_c<CT>(c, row * g.ldc + col + k, x[k]);
+                    }
+                }
+            }
+    }
+}
+
+// ------------------------------------------------------------------ plan
+// Tile and K slices of a shape.  Output tiles (tile_time; us, stages of 128
+// K): graph-replayed launches of every tile at 30 shapes, M 4 .. 4096, N 1000
+// .. 16384, K 1024 .. 14336; kRingTile is the 256 x 256 ring.
+//   M x N x K        32x128  64x128 128x128 128x256 192x256  ring (256 x 256)
+//   20x4096x4096       13.2    16.4                                     us
+//   128x14336x4096             19.9    26.5
+//   200x14336x4096             34.5    28.5    44.1
+//   600x4096x4096              33.1    25.7
+//   300x14336x4096             50.1    50.6    44.4    60.5
+//   600x14336x4096             85.5    83.3            68.7    85.0
+//   1000x14336x4096                   113.3   103.4           104.1
+//   4096x4096x4096                    121.3   111.9           107.4
+// K slices: partials and their reduction add ~1.2 us and, per slice, 0.45 us +
+// 0.6 us per MB, which pays where few tiles face a long K: 20x4096x14336 whole
+// K 38 us, 7 slices 13.6; 64x4096x14336 45 and 17; 200x1024x4096 16 and 12.3.
+static const TileCost kTiles[] = {
+    {32, 128, 2, 3.5f, 0.33f, 0.55f},  {64, 128, 2, 4.0f, 0.42f, 0.95f},  {128, 128, 1, 4.5f, 0.64f, 0.86f},
+    {128, 256, 1, 4.5f, 1.20f, 1.66f}, {192, 256, 1, 5.5f, 1.80f, 2.05f}, {256, 256, 1, 8.0f, 2.20f, 3.05f},
 };
-static SplitPlan splitk_plan(int64_t M, int64_t N, int64_t K) {
-    SplitPlan best{1, 256};
-    if (M <= kSkinnyMaxM || midm_shape(M, N, K)) return best;  // the GEMV, decode, mid-M and skinny kernels own these
+constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]), kRingTile = kNumTiles - 1;
+
+// Bytes of fp32 partials a shape may use (one batch): what fills the CUs once
+// with 128-row tiles of 256 or 128 columns in 2 or 4 slices.  0 where whole-K
+// tiles do as well: half of the CUs filled already, one pass of the decode
+// kernel (M <= 16, K <= 4096), or up to 64 rows against more than 16 weight
+// rows per CU unless K is the long side.
+static int64_t split_budget(int64_t M, int64_t N, int64_t K) {
     const int64_t mt = (M + 127) / 128, cus = num_cus_w();
-    if (2 * mt * ((N + 255) / 256) > cus) return best;  // whole-K tiles fill half of the CUs
+    if (M <= 1 || (M <= kDecodeMaxM && K <= dk::PASS_K)) return 0;
+    if (M <= 64 && N > 16 * cus && K <= 2 * N) return 0;
+    if (2 * mt * ((N + 255) / 256) > cus) return 0;
     int64_t best_wg = 0, best_bytes = 0;
     for (int bn = 256; bn >= 128; bn /= 2)
         for (int sp = 2; sp <= 4; sp *= 2) {
             const int64_t nt = (N + bn - 1) / bn, wg = mt * nt * sp, bytes = sp * nt * bn;
-            if (wg > cus || K % (512 * sp) != 0) continue;
-            if (wg > best_wg || (wg == best_wg && bytes < best_bytes)) {
-                best = SplitPlan{sp, bn};
-                best_wg = wg;
-                best_bytes = bytes;
-            }
+            if (wg > cus || K < 512 * sp) continue;
+            if (wg > best_wg || (wg == best_wg && bytes < best_bytes)) best_wg = wg, best_bytes = bytes;
         }
+    return best_bytes * mt * 128 * 4;
+}
+
+struct Plan {
+    int tile, splits;
+    float us;
+};
+static int64_t partial_bytes(const TileCost &c, int64_t M, int64_t N, int splits) {
+    return splits < 2 ? 0 : splits * ((M + c.bm - 1) / c.bm * c.bm) * ((N + c.bn - 1) / c.bn * c.bn) * 4;
+}
+// The fastest tile for `splits` slices (0: any number of slices) of nb batches
+// within `budget` bytes of partials per batch.  The ring kernel counts its 256
+// rows over both batches.
+static Plan best_plan(int64_t M, int64_t N, int64_t K, int nb, int splits, int64_t budget, bool ring) {
+    const int cus = num_cus_w();
+    const int64_t nk = K / wt::BK;
+    Plan best{0, 1, 1e30f};
+    for (int i = 0; i < kNumTiles; ++i) {
+        const TileCost &c = kTiles[i];
+        const int64_t bm = i == kRingTile ? c.bm / nb : c.bm;
+        const int64_t tiles = ((M + bm - 1) / bm) * ((N + c.bn - 1) / c.bn) * (i == kRingTile ? 1 : nb);
+        for (int sp = 1; sp <= 16 && 2 * sp <= imax(2, (int)imin((int)nk, 1 << 20)); ++sp) {
+            if ((splits && sp != splits) || (i == kRingTile && (sp > 1 || !ring))) continue;
+            if (sp > 1 && partial_bytes(c, M, N, sp) > budget) continue;
+            float t = tile_time(c, tiles * sp, (nk + sp - 1) / sp, cus);
+            if (sp > 1) t += 1.2f + (float)sp * (0.45f + 0.6e-6f * (float)(nb * M * N * 4));
+            if (t < best.us) best = Plan{i, sp, t};
+        }
+    }
     return best;
 }
-int gemm_bf16f4_splits(int64_t M, int64_t N, int64_t K, bool /*dual*/) { return splitk_plan(M, N, K).splits; }
+// The slices depend on M, N and K only, so the single and the dual launch of
+// one M add the same partial sums and give identical bits; the tile of the
+// dual form is chosen for its own number of tiles.
+static Plan bf16f4_plan(int64_t M, int64_t N, int64_t K, bool dual, bool ws, bool ring) {
+    const Plan one = best_plan(M, N, K, 1, ws ? 0 : 1, ws ? split_budget(M, N, K) : 0, ring);
+    return dual ? best_plan(M, N, K, 2, one.splits, split_budget(M, N, K), ring) : one;
+}
 
-// Workspace: the fp32 partial tiles [splits][NB][Mp][Np] (Mp = M rounded up
-// to 128 rows, Np = N rounded up to the plan's tile width).
+// Workspace bytes to give: the budget, for each batch.
 int64_t gemm_bf16f4_workspace(int64_t M, int64_t N, int64_t K, bool dual) {
-    const SplitPlan p = splitk_plan(M, N, K);
-    if (p.splits < 2) return 0;
-    return (int64_t)p.splits * (dual ? 2 : 1) * ((M + 127) / 128 * 128) * ((N + p.bn - 1) / p.bn * p.bn) * 4;
+    return split_budget(M, N, K) * (dual ? 2 : 1);
 }
 
 // C[b][m][n] = sum over slices s = 0, 1, ... of partial[s][b][m][n], in that
@@ -1984,41 +1960,37 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
     }
 }
 
-// Ring depth of the single form's split-K kernel (24 KiB per slot): 3 and 4
-// slots time within 3% of each other for M = 64 .. 256 against a 14336 x
-// 4096 weight, 4 the faster, so the loads in flight do not set its pace
-// (deeper rings would need the scale loads issued earlier).  The dual form's
-// 40 KiB slots fit 3.
-// Wave layouts of the split-K tiles: 128 x 256 single, 1 x 8 waves (each all
-// 128 rows and a 32-column strip, so each weight fragment is dequantized
-// once); 128 x 128 single, 2 x 4 (64 x 32 per wave); dual (256 A rows), 4 x 2
-// waves for both widths.
-template <int NB, int BN>
-static hipError_t launch_ring_splitk(GemmArgs g, int splits, hipStream_t s) {
-    constexpr int BR = 128 * NB;
-    constexpr int WGM = NB == 2 ? 4 : (BN == 256 ? 1 : 2);
-    constexpr int SL = NB == 1 ? 4 : 3;
-    const int64_t tiles = ((g.M + 127) / 128) * ((g.N + BN - 1) / BN);
+template <int WM, int WN, int TM, int TN, int S, int LA>
+static hipError_t launch_tile(GemmArgs g, int splits, hipStream_t s) {
+    constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
+    const int64_t tm = (g.M + BM - 1) / BM, tn = (g.N + BN - 1) / BN;
+    const int nb = g.a1 ? 2 : 1;
+    const dim3 grid((unsigned)(tm * tn * nb * splits)), blk(64 * (WM * WN + wt::NLW));
     g.splits = splits;
-    g.k_split = g.K / splits;
-    const dim3 grid((unsigned)(tiles * splits)), blk(wr::NT);
-    const int64_t Mp = (g.M + 127) / 128 * 128, Np = (g.N + BN - 1) / BN * BN;
-    const dim3 rgrid((unsigned)(NB * g.M * ((Np / 4 + 255) / 256))), rblk(256);
-#define LSMX_RS(CT)                                                                                              \
-    do {                                                                                                         \
-        hipLaunchKernelGGL((gemm_bf16f4_ring_kernel<NB, CT, BR, BN, SL, true, WGM>), grid, blk, 0, s, g);        \
-        hipLaunchKernelGGL((splitk_reduce_kernel<CT>), rgrid, rblk, 0, s, g.ws, splits, NB, Mp, Np, g.c, g.c1, \
-                           g.ldc, g.M, g.N);                                                                     \
+    const int64_t Mp = tm * BM, Np = tn * BN;
+    const dim3 rgrid((unsigned)(nb * g.M * ((Np / 4 + 255) / 256))), rblk(256);
+#define LSMX_T(CT)                                                                                                 \
+    do {                                                                                                           \
+        if (splits == 1) {                                                                                         \
+            hipLaunchKernelGGL((gemm_bf16f4_tile_kernel<CT, false, WM, WN, TM, TN, S, LA>), grid, blk, 0, s, g);        \
+        } else {                                                                                                   \
+            hipLaunchKernelGGL((gemm_bf16f4_tile_kernel<LSMX_F32, true, WM, WN, TM, TN, S, LA>), grid, blk, 0, s, g);   \
+            hipLaunchKernelGGL((splitk_reduce_kernel<CT>), rgrid, rblk, 0, s, g.ws, splits, nb, Mp, Np, g.c, g.c1, \
+                               g.ldc, g.M, g.N);                                                                   \
+        }                                                                                                          \
     } while (0)
-    if (g.c_dtype == LSMX_F32) LSMX_RS(LSMX_F32);
-    else if (g.c_dtype == LSMX_BF16) LSMX_RS(LSMX_BF16);
-    else LSMX_RS(LSMX_F16);
-#undef LSMX_RS
+    if (g.c_dtype == LSMX_F32) LSMX_T(LSMX_F32);
+    else if (g.c_dtype == LSMX_BF16) LSMX_T(LSMX_BF16);
+    else LSMX_T(LSMX_F16);
+#undef LSMX_T
     return hipGetLastError();
 }
-template <int NB>
-static hipError_t launch_ring_splitk(GemmArgs g, SplitPlan p, hipStream_t s) {
-    return p.bn == 256 ? launch_ring_splitk<NB, 256>(g, p.splits, s) : launch_ring_splitk<NB, 128>(g, p.splits, s);
+
+// E8M0 scale rows that start at multiples of 4 bytes (the kernel loads 16
+// bytes of a row at a time), and operand panels within 32-bit load offsets
+static bool tile_ok(const GemmArgs &g) {
+    return g.scale_fmt == LSMX_SCALE_E8M0 && g.ld_sb % 4 == 0 && (reinterpret_cast<uintptr_t>(g.sb) & 3) == 0 &&
+           g.lda < ((int64_t)1 << 22) && g.ldb < ((int64_t)1 << 22);
 }
 
 hipError_t launch_gemm_bf16f4(const GemmArgs &g, hipStream_t s) {
@@ -2026,14 +1998,26 @@ hipError_t launch_gemm_bf16f4(const GemmArgs &g, hipStream_t s) {
     // GEMV when the dual form's 2M activation rows of K bf16 fit in LDS (the
     // test depends on M and K only, so single and dual launches agree)
     if (g.M <= kGemvMaxM && 2 * g.M * g.K * 2 <= kGemvMaxLds) return launch_gemv(g, s);
-    if (g.M <= kDecodeMaxM && decode_ok(g)) return launch_decode(g, s);
-    if (midm_ok(g)) return launch_midm(g, s);
-    if (g.M <= kSkinnyMaxM && (g.a1 ? 2 * g.M : g.M) <= 128) return launch_skinny(g, s);
-    if (g.ws && ring_ok(g)) {
-        const SplitPlan p = splitk_plan(g.M, g.N, g.K);
-        if (p.splits > 1) return g.a1 ? launch_ring_splitk<2>(g, p, s) : launch_ring_splitk<1>(g, p, s);
+    const bool tiles = tile_ok(g);
+    // 2 .. 16 rows: the decode kernel while one pass covers K (M = 16, 4096 x
+    // 4096: 9.9 us against 9.1 - 9.7 in slices; M = 16, 14336 x 4096: 11.8
+    // against 12.4), past that K slices (M = 4, 4096 x 14336: 23.1 against 12.7)
+    const bool slices = tiles && g.ws && split_budget(g.M, g.N, g.K) > 0;
+    if (g.M <= kDecodeMaxM && decode_ok(g) && (g.K <= dk::PASS_K || !slices)) return launch_decode(g, s);
+    // few rows against a small weight: the skinny kernel's 16-row tiles spread
+    // it over more CUs (M = 32, 2048 x 2048: 7.3 us against 7.9)
+    const bool small = g.N <= 16 * (int64_t)num_cus_w() && g.K <= 2048;
+    if (g.M <= kSkinnyMaxM && (g.a1 ? 2 * g.M : g.M) <= 128 && (small || !tiles)) return launch_skinny(g, s);
+    if (!tiles) return g.a1 ? launch_w4_any<2>(g, s) : launch_w4_any<1>(g, s);
+    const Plan p = bf16f4_plan(g.M, g.N, g.K, g.a1 != nullptr, g.ws != nullptr, ring_ok(g));
+    switch (p.tile) {
+    case 0: return launch_tile<1, 4, 1, 1, 4, 4>(g, p.splits, s);
+    case 1: return launch_tile<1, 4, 2, 1, 3, 4>(g, p.splits, s);
+    case 2: return launch_tile<1, 4, 4, 1, 3, 2>(g, p.splits, s);
+    case 3: return launch_tile<2, 4, 2, 2, 3, 2>(g, p.splits, s);
+    case 4: return launch_tile<2, 4, 3, 2, 2, 1>(g, p.splits, s);
+    default: return g.a1 ? launch_ring<2, 256, 256, 3, 2, 4>(g, s) : launch_ring<1, 256, 256, 3, 2, 4>(g, s);
     }
-    return g.a1 ? launch_w4_any<2>(g, s) : launch_w4_any<1>(g, s);
 }
 
 }  // namespace lsmx

@@ -96,6 +96,11 @@ struct TileCost {
     int bm, bn, per_cu;
     float fix, lo, hi;
 };
+inline float tile_time(const TileCost &c, int64_t tiles, int64_t stages, int cus) {
+    const int64_t cap = (int64_t)cus * c.per_cu, full = (tiles - 1) / cap, last = tiles - full * cap;
+    const float tl = c.per_cu == 1 ? c.lo + (c.hi - c.lo) * (float)last / (float)cap : last <= cus ? c.lo : c.hi;
+    return (float)(full + 1) * c.fix + (float)stages * ((float)full * c.hi + tl);
+}
 template <int NT>
 inline int pick_tile(const TileCost (&table)[NT], int64_t M, int64_t N, int64_t problems, int64_t stages, int cus) {
     int best = 0;
@@ -103,9 +108,7 @@ inline int pick_tile(const TileCost (&table)[NT], int64_t M, int64_t N, int64_t 
     for (int i = 0; i < NT; ++i) {
         const TileCost &c = table[i];
         const int64_t tiles = problems * ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
-        const int64_t cap = (int64_t)cus * c.per_cu, full = (tiles - 1) / cap, last = tiles - full * cap;
-        const float tl = c.per_cu == 1 ? c.lo + (c.hi - c.lo) * (float)last / (float)cap : last <= cus ? c.lo : c.hi;
-        const float t = (float)(full + 1) * c.fix + (float)stages * ((float)full * c.hi + tl);
+        const float t = tile_time(c, tiles, stages, cus);
         if (i == 0 || t < tbest) best = i, tbest = t;
     }
     return best;
