@@ -185,17 +185,14 @@ int lsmx_quantize_mxfp4_batch(const lsmx_q_item *items, int n, int x_dtype, int 
     if (scale_fmt != LSMX_SCALE_E8M0 && scale_fmt != LSMX_SCALE_E8M0_KMAJOR)
         return fail(LSMX_ERR_DTYPE, "%s: scale_fmt must be E8M0 or K-major E8M0", fn);
     lsmx::QuantBatch b{};
-    int64_t rows = 0;
     for (int k = 0; k < n; ++k) {
         const lsmx_q_item &it = items[k];
         if (int r = check_quant(fn, it.x, x_dtype, it.rows, it.K, it.ldx, 32, it.codes, LSMX_CODES_PACKED,
                                 it.ld_codes, it.scale, scale_fmt, it.ld_scale, false))
             return r;
-        if (it.rows == 0 || it.K == 0) continue;   // empty tensors take no row of the grid
-        b.a[b.n] = lsmx::QuantArgs{it.x, x_dtype, it.rows, it.K, it.ldx, 32, it.codes, LSMX_CODES_PACKED,
-                                   it.ld_codes, it.scale, scale_fmt, it.ld_scale};
-        rows += it.rows;
-        b.end[b.n++] = rows;
+        if (it.rows == 0 || it.K == 0) continue;   // empty tensors take no workgroup
+        b.a[b.n++] = lsmx::QuantArgs{it.x, x_dtype, it.rows, it.K, it.ldx, 32, it.codes, LSMX_CODES_PACKED,
+                                     it.ld_codes, it.scale, scale_fmt, it.ld_scale};
     }
     if (int r = device_guard()) return r;
     if (b.n == 0) return LSMX_OK;

@@ -51,12 +51,13 @@ struct Quant2dArgs {
 };
 
 // Up to kQBatch tensors of one dtype and scale format quantized along their
-// rows by one launch (packed codes, 32-blocks, E8M0 scales); end[k] = rows of
-// tensors 0 .. k.
+// rows by one launch (packed codes, 32-blocks, E8M0 scales); the launcher fills
+// the vectors per row of each (and their udiv multiplier) and wend[k] =
+// workgroups of tensors 0 .. k.
 constexpr int kQBatch = 8;
 struct QuantBatch {
     QuantArgs a[kQBatch];
-    int64_t end[kQBatch];
+    uint32_t vpr[kQBatch], vdiv[kQBatch], wend[kQBatch];
     int n;
 };
 

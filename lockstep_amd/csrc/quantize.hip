@@ -12,6 +12,7 @@
 // the scale decision is all-integer (lsmx::block_e8m0).
 #include "lsmx_internal.h"
 #include "lsmx_q16.h"
+#include "lsmx_sched.h"
 
 namespace lsmx {
 
@@ -138,26 +139,6 @@ LSMX_DEV uint32_t e2m1_pack_hw(const uint32_t (&b)[E], uint32_t e8) {
     return w - dec;  // a tie's code magnitude is 2, 4 or 6: no borrow into the next nibble
 }
 
-// The same codes for elements that come from 16-bit inputs (bf16 / fp16,
-// widened to fp32 bits).  Ties toward the smaller magnitude without any
-// comparison: the hardware rounds |x| - 1 ulp (of fp32) to nearest-even
-// instead of |x|.  A 16-bit value has at most 11 significant bits, so no
-// input lies within 1 fp32 ulp above an E2M1 midpoint (midpoint / 2^e has at
-// most 3): every midpoint rounds down, as fp4.py:50-53 does, and every other
-// value lands on the same code as before.  Zeros (either sign) and infinities
-// are left alone, and the scale is still decided from the unmodified amax.
-LSMX_DEV uint32_t below_ulp(uint32_t b) {
-    const uint32_t ax = b & 0x7FFFFFFFu;
-    return (ax - 1u) < 0x7F7FFFFFu ? b - 1u : b;  // 0 < |x| < inf: one ulp toward zero
-}
-template <int E>
-LSMX_DEV uint32_t e2m1_pack_hw16(const uint32_t (&b)[E], uint32_t e8) {
-    uint32_t bd[E];
-#pragma unroll
-    for (int i = 0; i < E; ++i) bd[i] = below_ulp(b[i]);
-    return cvt_fp4_pairs<0, E>(0u, bd, u2f(e8 << 23));
-}
-
 // The same codes from the element-by-element rule (lsmx::e2m1_code), which
 // also covers a NaN block (e8 == 255).
 template <int E>
@@ -169,8 +150,13 @@ LSMX_DEV uint32_t e2m1_pack_exact(const uint32_t (&b)[E], uint32_t e8) {
 }
 
 // ------------------------------------------------------- row-mode quantize
-// Grid: (x = chunks of kThreads*kUnroll vectors along a row, y = rows, grid-
-// strided).  One vector = 16 input bytes.
+// One vector = 16 input bytes.  The vectors of all rows are numbered through
+// and every workgroup takes kQThreads * kQUnroll consecutive ones, whatever
+// the row length: with workgroups that stay inside a row, half the threads of
+// a 2048-wide bf16 row (256 vectors) had nothing to do and a workgroup moved
+// 4 KiB ([8192, 2048] bf16: 13.7 us, 10.8 so; [5000, 640] fp32 6.9 and 4.9).  Whole blocks, and
+// with K-major scales whole groups of four, lie in one row, so a lane's
+// neighbours in a block are its row's.
 constexpr int kQThreads = 256;
 constexpr int kQUnroll = 2;  // measured: 2 vectors per thread beat 1, 4 and 8 (more, shorter workgroups)
 
@@ -185,22 +171,34 @@ LSMX_DEV void store_scale(void *scale, int64_t r, int64_t kb, int64_t ld_scale, 
         reinterpret_cast<uint8_t *>(scale)[((kb >> 2) * ld_scale + r) * 4 + (kb & 3)] = (uint8_t)e8;
 }
 
-// Row r of x (xr: its first element), the kQUnroll vectors of this thread
-// from vector v0 on.  Every lane of the workgroup calls it for the same row
-// (the block maxima and K-major scale gathers are cross-lane).
-template <typename T, int BLOCK, bool PACKED, int SFMT>
-LSMX_DEV void quantize_row(const T *__restrict__ xr, int64_t K, uint8_t *__restrict__ codes, int64_t ld_codes,
-                           void *__restrict__ scale, int64_t ld_scale, int64_t r, int64_t v0) {
+// The rows of one tensor, or a run of them: x, codes and scale at the first
+// row, total = rows * vpr vectors (below 2^32), r_base its row number.
+struct RowSpan {
+    DivU32 vpr;       // vectors per row
+    uint32_t total;
+    int64_t r_base;
+};
+
+// The kQUnroll vectors n0, n0 + kQThreads, ... of the span.  Every lane of the
+// workgroup calls it (the block maxima and K-major scale gathers are
+// cross-lane).
+// WHOLE: a workgroup's vectors lie in one row (the row and its address are
+// then scalar: 3000 x 8192 fp32 23.1 us against 24.2).
+template <typename T, int BLOCK, bool PACKED, int SFMT, bool WHOLE>
+LSMX_DEV void quantize_vectors_of(const T *__restrict__ x, int64_t ldx, const RowSpan sp, uint8_t *__restrict__ codes,
+                               int64_t ld_codes, void *__restrict__ scale, int64_t ld_scale, uint32_t n0) {
     constexpr int E = Elem<T>::kPerVec;
     constexpr int G = BLOCK / E;  // lanes per block
-    const int64_t vpr = K / E;    // vectors per row
     uint4 buf[kQUnroll];
+    uint32_t row[kQUnroll], vec[kQUnroll];
 #pragma unroll
     for (int u = 0; u < kQUnroll; ++u) {
-        const int64_t v = v0 + u * kQThreads;
-        if (v < vpr) {
+        const uint32_t n = n0 + u * kQThreads;
+        row[u] = WHOLE ? (uint32_t)__builtin_amdgcn_readfirstlane(udiv(n0 - threadIdx.x, sp.vpr)) : udiv(n, sp.vpr);
+        vec[u] = n - row[u] * sp.vpr.d;
+        if (n < sp.total) {
             // streaming read: each input byte is used exactly once
-            const u32x4 w = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(xr) + v);
+            const u32x4 w = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(x + row[u] * ldx) + vec[u]);
             buf[u] = make_uint4(w[0], w[1], w[2], w[3]);
         } else {
             buf[u] = make_uint4(0, 0, 0, 0);
@@ -208,14 +206,15 @@ LSMX_DEV void quantize_row(const T *__restrict__ xr, int64_t K, uint8_t *__restr
     }
 #pragma unroll
     for (int u = 0; u < kQUnroll; ++u) {
-        const int64_t v = v0 + u * kQThreads;
         uint32_t b[E];
         Elem<T>::bits(buf[u], b);
         uint32_t am = 0;
 #pragma unroll
         for (int i = 0; i < E; ++i) am = max(am, b[i] & 0x7FFFFFFFu);
         am = group_max<G>(am);  // every lane of the block participates
-        const uint32_t e8 = block_e8m0(am);
+        uint32_t e8;
+        if constexpr (sizeof(T) == 2) e8 = block_e8m0_16x(am);
+        else e8 = block_e8m0(am);
         // K-major scales: the lane holding block kb (kb % 4 == 0) gathers
         // the bytes of kb..kb+3 -- the same row's dword -- for one store.
         // Every lane takes part in the cross-lane reads.
@@ -226,14 +225,21 @@ LSMX_DEV void quantize_row(const T *__restrict__ xr, int64_t K, uint8_t *__restr
                  ((uint32_t)__builtin_amdgcn_ds_bpermute(((l + 2 * G) & 63) << 2, (int)e8) << 16) |
                  ((uint32_t)__builtin_amdgcn_ds_bpermute(((l + 3 * G) & 63) << 2, (int)e8) << 24);
         }
-        if (v >= vpr) continue;  // whole blocks are in or out of range
+        if (n0 + u * kQThreads >= sp.total) continue;  // whole blocks are in or out of range
         // NaN blocks are rare: any lane with one takes the whole wave
         // through the exact per-element rule
         uint32_t w;
-        if (__any(e8 == 255u)) w = e2m1_pack_exact<E>(b, e8);
-        else if constexpr (sizeof(T) == 2) w = e2m1_pack_hw16<E>(b, e8);
-        else w = e2m1_pack_hw<E>(b, e8);
-        const int64_t col = v * E;
+        if (__any(e8 == 255u)) {
+            w = e2m1_pack_exact<E>(b, e8);
+        } else if constexpr (sizeof(T) == 2) {
+            float f[E];
+#pragma unroll
+            for (int i = 0; i < E; ++i) f[i] = tie_down16(b[i]);
+            w = cvt_fp4_x8(f, u2f(e8 << 23));
+        } else {
+            w = e2m1_pack_hw<E>(b, e8);
+        }
+        const int64_t r = row[u], col = (int64_t)vec[u] * E;
         if constexpr (PACKED) {
             if constexpr (E == 4) *reinterpret_cast<uint16_t *>(codes + r * ld_codes + col / 2) = (uint16_t)w;
             else *reinterpret_cast<uint32_t *>(codes + r * ld_codes + col / 2) = w;
@@ -247,39 +253,47 @@ LSMX_DEV void quantize_row(const T *__restrict__ xr, int64_t K, uint8_t *__restr
             const int64_t kb = col / BLOCK;
             // vectors of a wave start on a 4-block boundary (64 lanes x E elements)
             if ((threadIdx.x % (4 * G)) == 0)
-                reinterpret_cast<uint32_t *>(scale)[(kb >> 2) * ld_scale + r] = e4;
+                reinterpret_cast<uint32_t *>(scale)[(kb >> 2) * ld_scale + sp.r_base + r] = e4;
         } else {
-            if ((threadIdx.x % G) == 0) store_scale<SFMT>(scale, r, col / BLOCK, ld_scale, e8);
+            if ((threadIdx.x % G) == 0) store_scale<SFMT>(scale, sp.r_base + r, col / BLOCK, ld_scale, e8);
         }
     }
 }
 
 template <typename T, int BLOCK, bool PACKED, int SFMT>
-__global__ __launch_bounds__(kQThreads) void quantize_rows_kernel(
-    const T *__restrict__ x, int64_t rows, int64_t K, int64_t ldx, uint8_t *__restrict__ codes,
-    int64_t ld_codes, void *__restrict__ scale, int64_t ld_scale) {
-    const int64_t v0 = (int64_t)blockIdx.x * (kQThreads * kQUnroll) + threadIdx.x;
-    for (int64_t r = blockIdx.y; r < rows; r += gridDim.y)
-        quantize_row<T, BLOCK, PACKED, SFMT>(x + r * ldx, K, codes, ld_codes, scale, ld_scale, r, v0);
+LSMX_DEV void quantize_vectors(const T *__restrict__ x, int64_t ldx, const RowSpan sp, uint8_t *__restrict__ codes,
+                               int64_t ld_codes, void *__restrict__ scale, int64_t ld_scale, uint32_t n0) {
+    if (sp.vpr.d % (kQThreads * kQUnroll) == 0)
+        quantize_vectors_of<T, BLOCK, PACKED, SFMT, true>(x, ldx, sp, codes, ld_codes, scale, ld_scale, n0);
+    else
+        quantize_vectors_of<T, BLOCK, PACKED, SFMT, false>(x, ldx, sp, codes, ld_codes, scale, ld_scale, n0);
 }
 
-// Several tensors of one dtype and format in one launch: the rows of tensor
-// k are global rows end[k - 1] .. end[k] - 1, walked grid-strided along y;
-// the grid's x extent covers the longest row (workgroups past a shorter
-// row's end store nothing for it).
+// blockIdx.y: a run of seg rows (all rows unless they hold 2^31 vectors)
+template <typename T, int BLOCK, bool PACKED, int SFMT>
+__global__ __launch_bounds__(kQThreads) void quantize_rows_kernel(
+    const T *__restrict__ x, int64_t rows, int64_t seg, DivU32 vpr, int64_t ldx, uint8_t *__restrict__ codes,
+    int64_t ld_codes, void *__restrict__ scale, int64_t ld_scale) {
+    const int64_t r0 = blockIdx.y * seg;
+    const uint32_t n = (uint32_t)min(rows - r0, seg);
+    quantize_vectors<T, BLOCK, PACKED, SFMT>(x + r0 * ldx, ldx, RowSpan{vpr, n * vpr.d, r0}, codes + r0 * ld_codes,
+                                             ld_codes, scale, ld_scale,
+                                             blockIdx.x * (kQThreads * kQUnroll) + threadIdx.x);
+}
+
+// Several tensors of one dtype and format in one launch: workgroup b works on
+// the first tensor k with b < wend[k].
 template <typename T, int SFMT>
 __global__ __launch_bounds__(kQThreads) void quantize_rows_batch_kernel(QuantBatch b) {
-    const int64_t v0 = (int64_t)blockIdx.x * (kQThreads * kQUnroll) + threadIdx.x;
-    const int64_t total = b.end[b.n - 1];
+    const uint32_t blk = blockIdx.x;
     int k = 0;
-    for (int64_t gr = blockIdx.y; gr < total; gr += gridDim.y) {
-        while (gr >= b.end[k]) ++k;   // gr < total = end[n - 1]: k stays below n
-        const QuantArgs &a = b.a[k];
-        const int64_t r = gr - (k ? b.end[k - 1] : 0);
-        quantize_row<T, 32, true, SFMT>(reinterpret_cast<const T *>(a.x) + r * a.ldx, a.K,
-                                        reinterpret_cast<uint8_t *>(a.codes), a.ld_codes, a.scale, a.ld_scale, r,
-                                        v0);
-    }
+    while (k + 1 < b.n && blk >= b.wend[k]) ++k;
+    const QuantArgs &a = b.a[k];
+    const uint32_t local = blk - (k ? b.wend[k - 1] : 0u);
+    quantize_vectors<T, 32, true, SFMT>(reinterpret_cast<const T *>(a.x), a.ldx,
+                                        RowSpan{DivU32{b.vpr[k], b.vdiv[k]}, (uint32_t)a.rows * b.vpr[k], 0},
+                                        reinterpret_cast<uint8_t *>(a.codes), a.ld_codes, a.scale, a.ld_scale,
+                                        local * (kQThreads * kQUnroll) + threadIdx.x);
 }
 
 // ------------------------------------------ both axes in one pass
@@ -809,29 +823,56 @@ __global__ void dequant_kernel(const uint8_t *__restrict__ codes, int64_t ld_cod
 template <typename T, int BLOCK, bool PACKED, int SF32>
 static hipError_t launch_rows(const QuantArgs &a, hipStream_t s) {
     constexpr int E = Elem<T>::kPerVec;
-    const int64_t vpr = a.K / E;
-    const int64_t gx = (vpr + kQThreads * kQUnroll - 1) / (kQThreads * kQUnroll);
-    const int64_t gy = a.rows < 65535 ? a.rows : 65535;
-    hipLaunchKernelGGL((quantize_rows_kernel<T, BLOCK, PACKED, SF32>), dim3((unsigned)gx, (unsigned)gy),
-                       dim3(kQThreads), 0, s, reinterpret_cast<const T *>(a.x), a.rows, a.K, a.ldx,
+    constexpr int64_t per = kQThreads * kQUnroll;
+    constexpr int64_t kWide = (int64_t)1 << 30;   // elements: longer rows go in pieces of whole 128-element groups
+    if (a.K > kWide) {
+        for (int64_t k0 = 0; k0 < a.K; k0 += kWide) {
+            QuantArgs p = a;
+            p.K = a.K - k0 < kWide ? a.K - k0 : kWide;
+            p.x = reinterpret_cast<const T *>(a.x) + k0;
+            p.codes = reinterpret_cast<uint8_t *>(a.codes) + (PACKED ? k0 / 2 : k0);
+            const int64_t nb = k0 / BLOCK;
+            p.scale = reinterpret_cast<uint8_t *>(a.scale) +
+                      (SF32 == LSMX_SCALE_F32 ? nb * 4 : SF32 == LSMX_SCALE_E8M0 ? nb : nb * a.ld_scale);
+            const hipError_t e = launch_rows<T, BLOCK, PACKED, SF32>(p, s);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
+    const int64_t vpr = a.K / E, most = ((int64_t)1 << 31) / vpr;   // rows of one run
+    const int64_t seg = a.rows < most ? a.rows : most;
+    const dim3 grid((unsigned)((seg * vpr + per - 1) / per), (unsigned)((a.rows + seg - 1) / seg));
+    hipLaunchKernelGGL((quantize_rows_kernel<T, BLOCK, PACKED, SF32>), grid, dim3(kQThreads), 0, s,
+                       reinterpret_cast<const T *>(a.x), a.rows, seg, make_div((uint32_t)vpr), a.ldx,
                        reinterpret_cast<uint8_t *>(a.codes), a.ld_codes, a.scale, a.ld_scale);
     return hipGetLastError();
 }
 
 template <typename T>
-static hipError_t launch_rows_batch(const QuantBatch &b, hipStream_t s) {
+static hipError_t launch_rows_batch(QuantBatch b, hipStream_t s) {
     constexpr int E = Elem<T>::kPerVec;
-    int64_t kmax = 0;
-    for (int k = 0; k < b.n; ++k) kmax = b.a[k].K > kmax ? b.a[k].K : kmax;
-    const int64_t gx = (kmax / E + kQThreads * kQUnroll - 1) / (kQThreads * kQUnroll);
-    const int64_t total = b.end[b.n - 1];
-    const int64_t gy = total < 65535 ? total : 65535;
-    if (b.a[0].scale_fmt == LSMX_SCALE_E8M0_KMAJOR)
-        hipLaunchKernelGGL((quantize_rows_batch_kernel<T, LSMX_SCALE_E8M0_KMAJOR>), dim3((unsigned)gx, (unsigned)gy),
-                           dim3(kQThreads), 0, s, b);
-    else
-        hipLaunchKernelGGL((quantize_rows_batch_kernel<T, LSMX_SCALE_E8M0>), dim3((unsigned)gx, (unsigned)gy),
-                           dim3(kQThreads), 0, s, b);
+    constexpr int64_t per = kQThreads * kQUnroll;
+    int64_t wgs = 0;
+    bool big = false;
+    for (int k = 0; k < b.n; ++k) {
+        const int64_t vpr = b.a[k].K / E, total = b.a[k].rows * vpr;
+        big |= total > (int64_t)1 << 31 || b.a[k].K > (int64_t)1 << 30;
+        wgs += (total + per - 1) / per;
+        b.vpr[k] = (uint32_t)vpr;
+        b.vdiv[k] = make_div((uint32_t)vpr).m;
+        b.wend[k] = (uint32_t)wgs;
+    }
+    const bool km = b.a[0].scale_fmt == LSMX_SCALE_E8M0_KMAJOR;
+    if (big || wgs > 0x7FFFFFFF) {   // 2^31 vectors and more: one launch per tensor, in runs of rows
+        for (int k = 0; k < b.n; ++k) {
+            const hipError_t e = km ? launch_rows<T, 32, true, LSMX_SCALE_E8M0_KMAJOR>(b.a[k], s)
+                                    : launch_rows<T, 32, true, LSMX_SCALE_E8M0>(b.a[k], s);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
+    if (km) hipLaunchKernelGGL((quantize_rows_batch_kernel<T, LSMX_SCALE_E8M0_KMAJOR>), dim3((unsigned)wgs), dim3(kQThreads), 0, s, b);
+    else hipLaunchKernelGGL((quantize_rows_batch_kernel<T, LSMX_SCALE_E8M0>), dim3((unsigned)wgs), dim3(kQThreads), 0, s, b);
     return hipGetLastError();
 }
 
