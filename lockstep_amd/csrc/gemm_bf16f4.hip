@@ -1960,7 +1960,9 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
     }
 }
 
-template <int WM, int WN, int TM, int TN, int S, int LA>
+// LAS: LA of the K-slice form, whose epilogue holds two registers more: 64 x 128
+// tiles have 128 per lane (two workgroups per CU), and with LA = 4 spilled two
+template <int WM, int WN, int TM, int TN, int S, int LA, int LAS = LA>
 static hipError_t launch_tile(GemmArgs g, int splits, hipStream_t s) {
     constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
     const int64_t tm = (g.M + BM - 1) / BM, tn = (g.N + BN - 1) / BN;
@@ -1974,7 +1976,7 @@ static hipError_t launch_tile(GemmArgs g, int splits, hipStream_t s) {
         if (splits == 1) {                                                                                         \
             hipLaunchKernelGGL((gemm_bf16f4_tile_kernel<CT, false, WM, WN, TM, TN, S, LA>), grid, blk, 0, s, g);        \
         } else {                                                                                                   \
-            hipLaunchKernelGGL((gemm_bf16f4_tile_kernel<LSMX_F32, true, WM, WN, TM, TN, S, LA>), grid, blk, 0, s, g);   \
+            hipLaunchKernelGGL((gemm_bf16f4_tile_kernel<LSMX_F32, true, WM, WN, TM, TN, S, LAS>), grid, blk, 0, s, g);  \
             hipLaunchKernelGGL((splitk_reduce_kernel<CT>), rgrid, rblk, 0, s, g.ws, splits, nb, Mp, Np, g.c, g.c1, \
                                g.ldc, g.M, g.N);                                                                   \
         }                                                                                                          \
@@ -2012,7 +2014,7 @@ hipError_t launch_gemm_bf16f4(const GemmArgs &g, hipStream_t s) {
     const Plan p = bf16f4_plan(g.M, g.N, g.K, g.a1 != nullptr, g.ws != nullptr, ring_ok(g));
     switch (p.tile) {
     case 0: return launch_tile<1, 4, 1, 1, 4, 4>(g, p.splits, s);
-    case 1: return launch_tile<1, 4, 2, 1, 3, 4>(g, p.splits, s);
+    case 1: return launch_tile<1, 4, 2, 1, 3, 4, 2>(g, p.splits, s);
     case 2: return launch_tile<1, 4, 4, 1, 3, 2>(g, p.splits, s);
     case 3: return launch_tile<2, 4, 2, 2, 3, 2>(g, p.splits, s);
     case 4: return launch_tile<2, 4, 3, 2, 2, 1>(g, p.splits, s);
