@@ -445,13 +445,11 @@ __global__ __launch_bounds__(512, 2) void gemm_dense_tile_kernel(DenseArgs g) {
                                    : (uint32_t)(drow0 * ldb_b + ((lane % CPR) ^ dr::swz(drow0)) * 16);
         const uint32_t stepA = (uint32_t)(NLW * RPI * lda_b);
         const uint32_t stepB = BNC ? (uint32_t)(RPB * NLW * ldb_b) : (uint32_t)(NLW * RPI * ldb_b);
-        const uint8_t *pa[KC], *pb[KC];
-#pragma unroll
-        for (int h = 0; h < KC; ++h) {
-            const bool second = (P == 2 && p == 1) || h == 1;
-            pa[h] = (second ? g.a1 : g.a0) + m0 * lda_b;
-            pb[h] = (second ? g.b1 : g.b0) + (BNC ? n0 * 2 : n0 * ldb_b);
-        }
+        // scalars, not arrays of KC: the compiler kept those in scratch (one
+        // accumulator over both products, 700 x 2000 x 2048: 47.0 -> 23.3 us)
+        const int64_t ma = m0 * lda_b, mb = BNC ? n0 * 2 : n0 * ldb_b;
+        const uint8_t *pa0 = (p ? g.a1 : g.a0) + ma, *pb0 = (p ? g.b1 : g.b0) + mb;
+        const uint8_t *pa1 = KC == 2 ? g.a1 + ma : pa0, *pb1 = KC == 2 ? g.b1 + mb : pb0;
         // panels end at the operand's last element; BNC columns past N in
         // other rows read the next row's values, whose products only reach
         // outputs that are not stored
@@ -463,8 +461,8 @@ __global__ __launch_bounds__(512, 2) void gemm_dense_tile_kernel(DenseArgs g) {
             const int kb = KC == 2 ? kt >> 1 : kt;
             const bool past = kt >= nk;   // refills past the end: empty descriptors, zeros
             const int64_t ao = (int64_t)kb * BKB, bo = BNC ? (int64_t)kb * 64 * ldb_b : ao;
-            const v4i_rsrc rsA = buf_rsrc((h ? pa[KC - 1] : pa[0]) + (past ? 0 : ao), past ? 0 : (uint64_t)(na - ao));
-            const v4i_rsrc rsB = buf_rsrc((h ? pb[KC - 1] : pb[0]) + (past ? 0 : bo), past ? 0 : (uint64_t)(nb - bo));
+            const v4i_rsrc rsA = buf_rsrc((h ? pa1 : pa0) + (past ? 0 : ao), past ? 0 : (uint64_t)(na - ao));
+            const v4i_rsrc rsB = buf_rsrc((h ? pb1 : pb0) + (past ? 0 : bo), past ? 0 : (uint64_t)(nb - bo));
 #pragma unroll
             for (int i = 0; i < XA; ++i) dma_x4(offA0 + i * stepA, rsA, ring0 + so + (i * NLW + lw) * 1024);
 #pragma unroll
