@@ -255,7 +255,9 @@ int64_t lsmx_gemm_bf16f4_workspace(int64_t M, int64_t N, int64_t K, int dual);
  * bits).  The same sums as the reference's split-K GEMM (dual_gemm.py:
  * 117-179) without its atomics.  Workspace: 16-byte aligned, at least the
  * bytes lsmx_gemm_bf16f4_workspace returns, no initial contents required;
- * calls that share a workspace must be stream-ordered.  A NULL workspace,
+ * calls that share a workspace must be stream-ordered (calls of several host
+ * threads on one stream are: the library enqueues the launches of one call
+ * together).  A NULL workspace,
  * or a shape the library does not split, runs the whole-K kernels. */
 int lsmx_gemm_bf16f4_ws(const void *a0, const void *a1, int64_t lda, const uint8_t *w_pk, int64_t ldw,
                         const void *w_scale, int64_t ld_sw, int scale_fmt, void *c0, void *c1, int c_dtype, int64_t ldc,
@@ -270,8 +272,8 @@ int lsmx_gemm_bf16f4_ws(const void *a0, const void *a1, int64_t lda, const uint8
  * ends; its device address is looked up once per GPU on that first call).
  * A shape whose split-K partials need more is rejected with LSMX_ERR_SHAPE
  * (on a 256-CU gfx950 none does).  The call allocates nothing.  Every call
- * on one GPU shares the array: calls that overlap on one GPU (different
- * streams, or host threads without stream ordering) race. */
+ * on one GPU shares the array: calls that overlap on one GPU (on different
+ * streams without ordering between them) race. */
 int lsmx_gemm_bf16f4_noalloc(const void *a0, const void *a1, int64_t lda, const uint8_t *w_pk, int64_t ldw,
                              const void *w_scale, int64_t ld_sw, int scale_fmt, void *c0, void *c1, int c_dtype,
                              int64_t ldc, int64_t M, int64_t N, int64_t K, void *stream);

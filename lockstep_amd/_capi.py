@@ -183,7 +183,9 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     """A device workspace of at least nbytes for the split-K GEMMs.
 
     Eager calls share one per (device, stream): calls on one stream are
-    ordered, so they may share it.  It is kept for later calls and grown by
+    ordered, those of several host threads included (the library enqueues the
+    two launches of a sliced call with no other call's between them), so they
+    may share it.  It is kept for later calls and grown by
     replacing it with a larger one (the old one returns to torch's caching
     allocator, stream-ordered).
 

@@ -23,6 +23,8 @@
 // 128 x 128 per wave (4 x 4 MFMA tiles).  In dual mode the 256 A rows are
 // 128 rows of A0 followed by the same 128 rows of A1: one weight tile in LDS
 // feeds both batches and is read from memory once per stage.
+#include <mutex>
+
 #include "lsmx_dma.h"
 #include "lsmx_store.h"
 #include "lsmx_internal.h"
@@ -1960,6 +1962,11 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
     }
 }
 
+// The two launches of a sliced call, and no other thread's between them: all
+// host threads on a stream share its workspace, and a call's partials must
+// still be there when its reduction runs.
+static std::mutex g_slices_mu;
+
 // LAS: LA of the K-slice form, whose epilogue holds two registers more: 64 x 128
 // tiles have 128 per lane (two workgroups per CU), and with LA = 4 spilled two
 template <int WM, int WN, int TM, int TN, int S, int LA, int LAS = LA>
@@ -1976,6 +1983,7 @@ static hipError_t launch_tile(GemmArgs g, int splits, hipStream_t s) {
         if (splits == 1) {                                                                                         \
             hipLaunchKernelGGL((gemm_bf16f4_tile_kernel<CT, false, WM, WN, TM, TN, S, LA>), grid, blk, 0, s, g);        \
         } else {                                                                                                   \
+            std::lock_guard<std::mutex> lk(g_slices_mu);                                                           \
             hipLaunchKernelGGL((gemm_bf16f4_tile_kernel<LSMX_F32, true, WM, WN, TM, TN, S, LAS>), grid, blk, 0, s, g);  \
             hipLaunchKernelGGL((splitk_reduce_kernel<CT>), rgrid, rblk, 0, s, g.ws, splits, nb, Mp, Np, g.c, g.c1, \
                                g.ldc, g.M, g.N);                                                                   \

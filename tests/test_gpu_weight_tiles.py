@@ -59,3 +59,29 @@ def test_special_scale_bytes(M, N, K):
     keep = torch.ones(N, dtype=torch.bool, device=dev)
     keep[7] = keep[9] = False
     assert torch.equal(d[:, keep], c[:, keep])
+
+
+def test_sliced_calls_of_two_threads_on_one_stream():
+    """Both threads use the default stream and so one workspace; each gets its own result."""
+    import threading
+
+    from lockstep_amd import fp4, mxfp4_gemm
+    dev = torch.device("cuda", 0)
+    g = torch.Generator(device=dev).manual_seed(3)
+    pk, sc = fp4.quantize_pack_mxfp4(torch.randn((4096, 14336), device=dev, generator=g) * 0.02)
+    acts = [torch.randn((m, 14336), device=dev, generator=g).to(torch.bfloat16) for m in (20, 4)]
+    want = [mxfp4_gemm.mxfp4_gemm_bf16(a, pk, sc) for a in acts]
+    got = [[], []]
+
+    def work(i):
+        for _ in range(50):
+            got[i].append(mxfp4_gemm.mxfp4_gemm_bf16(acts[i], pk, sc))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for g_, w_ in zip(got, want):
+        assert len(g_) == 50 and all(torch.equal(c, w_) for c in g_)
