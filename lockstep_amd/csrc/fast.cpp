@@ -54,9 +54,9 @@ int dtype_of(at::ScalarType s) {
     return s == at::kFloat ? LSMX_F32 : s == at::kBFloat16 ? LSMX_BF16 : s == at::kHalf ? LSMX_F16 : -1;
 }
 
-// scalar type of a torch.dtype argument (None: `dflt`), or Undefined
-at::ScalarType out_type(PyObject *o, at::ScalarType dflt) {
-    if (o == Py_None) return dflt;
+// scalar type of a torch.dtype argument, or Undefined (None included: only
+// weight()'s callers give it a meaning)
+at::ScalarType out_type(PyObject *o) {
     if (!THPDtype_Check(o)) return at::ScalarType::Undefined;
     const at::ScalarType s = reinterpret_cast<THPDtype *>(o)->scalar_type;
     return dtype_of(s) >= 0 ? s : at::ScalarType::Undefined;
@@ -271,7 +271,7 @@ PyObject *gemm_packed(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     NONE_IF(n != 6);
     const Tensor *ap = plain(a[0]), *bp = plain(a[1]), *as = plain(a[2]), *bs = plain(a[3]);
-    const at::ScalarType ot = out_type(a[4], at::kBFloat16);
+    const at::ScalarType ot = out_type(a[4]);
     NONE_IF(!ap || !bp || !as || !bs || ot == at::ScalarType::Undefined || ap->scalar_type() != at::kByte ||
             bp->scalar_type() != at::kByte || !rows16(*ap) || !rows16(*bp) || ap->size(1) != bp->size(1));
     const int64_t M = ap->size(0), N = bp->size(0), K = 2 * ap->size(1);
@@ -316,7 +316,7 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     NONE_IF(n != 3);
     const Tensor *x = plain(a[0]), *w = plain(a[1]);
-    const at::ScalarType ot = out_type(a[2], at::kBFloat16);
+    const at::ScalarType ot = out_type(a[2]);
     NONE_IF(ot == at::ScalarType::Undefined || !quant_rows(x, 128) || !quant_rows(w, 128) || x->size(1) != w->size(1) ||
             x->device() != w->device());
     const int64_t K = x->size(1);
@@ -343,7 +343,7 @@ PyObject *weight(PyObject *, PyObject *const *a, Py_ssize_t n) {
     const Tensor *a1 = dual ? plain(a[1]) : nullptr;
     NONE_IF(!a0 || !w || !ws || (dual && !a1) || !rows16(*a0) || !rows16(*w) || dtype_of(a0->scalar_type()) < 0 ||
             w->scalar_type() != at::kByte || ws->scalar_type() != at::kByte);
-    const at::ScalarType at_ = a0->scalar_type(), ot = out_type(a[4], at_);
+    const at::ScalarType at_ = a0->scalar_type(), ot = a[4] == Py_None ? at_ : out_type(a[4]);
     const int64_t M = a0->size(0), K = a0->size(1), N = w->size(0);
     NONE_IF(ot == at::ScalarType::Undefined || M == 0 || N == 0 || K == 0 || K % 128 || 2 * w->size(1) != K ||
             w->device() != a0->device() || ws->device() != a0->device());
@@ -391,7 +391,7 @@ PyObject *gemm_fp8(PyObject *, PyObject *const *a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     NONE_IF(n != 6);
     const Tensor *x = plain(a[0]), *b = plain(a[1]), *as = plain(a[2]), *bs = plain(a[3]);
-    const at::ScalarType ot = out_type(a[4], at::kBFloat16);
+    const at::ScalarType ot = out_type(a[4]);
     auto bytes = [](const Tensor &t) { return t.scalar_type() == at::kFloat8_e4m3fn || t.scalar_type() == at::kByte; };
     NONE_IF(!x || !b || !as || !bs || ot == at::ScalarType::Undefined || !bytes(*x) || !bytes(*b) || !rows16(*x) ||
             !rows16(*b) || x->size(1) != b->size(0));

@@ -133,5 +133,12 @@ def test_errors_are_the_python_path_s(C):
         mxfp4_gemm.mxfp4_gemm_bf16(torch.zeros((2, 128), device=dev, dtype=torch.bfloat16), p, s[:, :3])
     with pytest.raises(TypeError):
         mxfp4_gemm.mxfp4_gemm_packed(p, p, s, s, out_dtype=torch.float64)
+    one = torch.ones((4, 4), device=dev)
+    f8 = torch.zeros((128, 128), dtype=torch.uint8, device=dev)
+    for scale in (torch.full((1, 4, 4), 127, dtype=torch.uint8, device=dev), one):
+        with pytest.raises(TypeError, match="unsupported dtype None"):
+            mxfp4_gemm.mxfp4_gemm_packed(p, p, scale, scale, out_dtype=None)
+    with pytest.raises(TypeError, match="unsupported dtype None"):
+        mxfp4_gemm.mxfp4_gemm_fp8(f8[:4], f8, one, torch.ones((4, 128), device=dev), out_dtype=None)
     with pytest.raises(C.LsmxError):
         C.check(-2)
