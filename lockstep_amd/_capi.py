@@ -11,6 +11,7 @@ import ctypes
 import itertools
 import os
 import threading
+import warnings
 from pathlib import Path
 
 import torch
@@ -206,15 +207,12 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     return ws
 
 
-class _MissingFast:
-    """Stands in for the native call path when it has not been built."""
-
-    def __init__(self, why):
-        self._why = why
+class _NoFast:
+    """Stands in for a native call path that cannot be loaded: takes no call,
+    so every one runs the Python path, on the same kernels."""
 
     def __getattr__(self, name):
-        raise RuntimeError(f"lockstep_amd/_fast.so cannot be loaded ({self._why}): build it with "
-                           "`python -m lockstep_amd.build`")
+        return lambda *args: None
 
 
 # The plain forms of the public calls in native code (csrc/fast.cpp): each
@@ -223,4 +221,7 @@ try:
     from . import _fast as fast
     fast.init(check, workspace, next_epoch)
 except ImportError as e:
-    fast = _MissingFast(e)
+    fast = _NoFast()
+    if LIB_PATH.exists():   # without it every call raises at load()
+        warnings.warn(f"lockstep_amd/_fast.so cannot be loaded ({e}): calls take the slower Python path; rebuild with "
+                      "`python -m lockstep_amd.build`", RuntimeWarning)

@@ -1,8 +1,14 @@
 """The native call path (csrc/fast.cpp) against the Python one: forms it does
 not take give None (CPU), and those it takes give the general path's bits."""
 
+import subprocess
+import sys
+from pathlib import Path
+
 import pytest
 import torch
+
+ROOT = Path(__file__).resolve().parents[1]
 
 
 @pytest.fixture
@@ -31,6 +37,29 @@ def test_other_forms_are_left_to_the_python_path(C):
     with pytest.raises(RuntimeError, match="gfx950 GPU only"):
         from lockstep_amd import fp4
         fp4.quantize_pack_mxfp4(x)
+
+
+def test_calls_do_without_the_native_path():
+    """A _fast.so that cannot be loaded (another torch, a partial build) is
+    reported, and the calls run or raise as the Python path does."""
+    code = """
+import sys, warnings
+sys.modules["lockstep_amd._fast"] = None   # import raises ImportError
+with warnings.catch_warnings(record=True) as w:
+    warnings.simplefilter("always")
+    from lockstep_amd import fp4
+assert any("_fast.so cannot be loaded" in str(x.message) for x in w)
+import torch
+for K, text in ((48, "multiple of block=32"), (64, "gfx950 GPU only")):
+    try:
+        fp4.quantize_mxfp4(torch.zeros(4, K))
+    except (AssertionError, RuntimeError) as e:
+        assert text in str(e), e
+    else:
+        raise SystemExit("no error")
+"""
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr
 
 
 def _general(monkeypatch, C, f):
