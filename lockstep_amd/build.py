@@ -1,4 +1,5 @@
-"""Build liblsmx.so (the gfx950 HIP kernels + C ABI) in-tree with hipcc.
+"""Build liblsmx.so (the gfx950 HIP kernels + C ABI) in-tree with hipcc, and
+_fast.so (the native call path of the Python functions) with the host compiler.
 
     python -m lockstep_amd.build          # or lockstep_amd.build.build()
 
@@ -18,11 +19,11 @@ from pathlib import Path
 PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 LIB = PKG / "liblsmx.so"
+FAST_LIB = PKG / "_fast.so"
 SOURCES = ["capi.hip", "quantize.hip", "gemm_f4f4.hip", "gemm_bf16f4.hip", "gemm_dense.hip", "gemm_dense_ring.hip", "gemm_f8f8.hip", "gemm_promote.hip"]
 ARCH = "gfx950"
 
 # -packed-fp32-ops: no v_pk_{add,mul,fma}_f32 anywhere in the device code.
-FAST_LIB = PKG / "_fast.so"
 FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-shared",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -65,7 +66,7 @@ def build_fast(verbose: bool = False) -> Path:
 def build(verbose: bool = False, jobs: int | None = None) -> Path:
     """Compile every source to an object in parallel (each kernel is launched
     from its own translation unit, so no relocatable device code is needed),
-    then link liblsmx.so."""
+    then link liblsmx.so and build _fast.so against it."""
     from concurrent.futures import ThreadPoolExecutor
 
     objdir = PKG / "_build"
@@ -81,10 +82,10 @@ def build(verbose: bool = False, jobs: int | None = None) -> Path:
     tmp = LIB.with_suffix(".so.tmp")
     _run([cc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)], verbose)
     os.replace(tmp, LIB)
+    build_fast(verbose)
     return LIB
 
 
 if __name__ == "__main__":
     build(verbose=True)
-    build_fast(verbose=True)
     print(f"built {LIB} and {FAST_LIB}", file=sys.stderr)

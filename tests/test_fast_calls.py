@@ -62,6 +62,17 @@ for K, text in ((48, "multiple of block=32"), (64, "gfx950 GPU only")):
     assert r.returncode == 0, r.stderr
 
 
+def test_build_makes_both_libraries(monkeypatch, tmp_path):
+    """lockstep_amd.build.build() alone (the compilers replaced by a touch)."""
+    from lockstep_amd import build as B
+    monkeypatch.setattr(B, "PKG", tmp_path)
+    monkeypatch.setattr(B, "LIB", tmp_path / "liblsmx.so")
+    monkeypatch.setattr(B, "FAST_LIB", tmp_path / "_fast.so")
+    monkeypatch.setattr(B, "_run", lambda cmd, verbose: Path(cmd[cmd.index("-o") + 1]).touch())
+    B.build()
+    assert B.LIB.exists() and B.FAST_LIB.exists()
+
+
 def _general(monkeypatch, C, f):
     """f() with every native call declined."""
     class Declines:
