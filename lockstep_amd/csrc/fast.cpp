@@ -8,14 +8,17 @@
 // takes the arguments of its Python caller and handles the form that programs
 // pass in a loop -- exact torch tensors on one GPU, the layouts the kernels
 // read in place -- and returns None for anything else (other strides,
-// alignments, types, empty shapes, wrong arguments, tensor subclasses and
-// functorch wrappers): the caller then runs its general path, which converts,
+// alignments, types, empty shapes, wrong arguments, tensor subclasses,
+// functorch wrappers, calls under a dispatch mode or a functorch transform):
+// the caller then runs its general path, which converts,
 // or raises as it always has.  The launches go through the same C ABI
 // (include/lsmx.h), on torch's current stream, with the GIL released.
 #include <Python.h>
 
 #include <ATen/ATen.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -30,10 +33,17 @@ PyObject *g_error = nullptr;      // _capi.check(rc): raises LsmxError
 PyObject *g_workspace = nullptr;  // _capi.workspace(device, nbytes)
 PyObject *g_epoch = nullptr;      // _capi.next_epoch()
 
+// A dispatch mode or a functorch transform around the call: at::empty gives
+// that mode's tensors, which may have no data pointer.
+bool transformed() {
+    return c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+           c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+}
+
 // A plain GPU tensor: exactly torch.Tensor (or Parameter), with storage, and no
 // dispatch key that changes what its data means.
 const Tensor *plain(PyObject *o) {
-    if (!THPVariable_CheckExact(o)) return nullptr;
+    if (!THPVariable_CheckExact(o) || transformed()) return nullptr;
     const Tensor &t = THPVariable_Unpack(o);
     if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || !t.has_storage()) return nullptr;
     constexpr c10::DispatchKeySet odd{c10::DispatchKey::Python, c10::DispatchKey::Conjugate, c10::DispatchKey::Negative,
@@ -69,14 +79,22 @@ void *stream_of(const Tensor &t) {
     return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream();
 }
 
+// Holds the GIL released; takes it back when a C++ exception leaves the scope
+// too, so that HANDLE_TH_ERRORS sets the Python error with it held.
+struct NoGil {
+    PyThreadState *s = PyEval_SaveThread();
+    ~NoGil() { PyEval_RestoreThread(s); }
+};
+
 // Runs launches with the GIL released; returns false with a Python error set
 // (LsmxError through _capi.check) if one fails.
 template <typename F>
 bool launch(F &&f) {
     int rc;
-    Py_BEGIN_ALLOW_THREADS;
-    rc = f();
-    Py_END_ALLOW_THREADS;
+    {
+        NoGil released;
+        rc = f();
+    }
     if (rc == LSMX_OK) return true;
     PyObject *r = PyObject_CallFunction(g_error, "i", rc);
     Py_XDECREF(r);

@@ -182,3 +182,32 @@ def test_errors_are_the_python_path_s(C):
         mxfp4_gemm.mxfp4_gemm_fp8(f8[:4], f8, one, torch.ones((4, 128), device=dev), out_dtype=None)
     with pytest.raises(C.LsmxError):
         C.check(-2)
+
+
+@pytest.mark.gpu
+def test_calls_under_modes_and_transforms_take_the_python_path(C, monkeypatch):
+    """A dispatch mode or functorch transform hands out tensors without data."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from lockstep_amd import fp4, mxfp4_gemm
+    dev = torch.device("cuda", 0)
+    x = torch.randn((4, 128), device=dev).to(torch.bfloat16)
+    pk, sc = fp4.quantize_pack_mxfp4(torch.randn((16, 128), device=dev))
+    native = []
+
+    def call():
+        native.append(C.fast.quantize(x))
+        native.append(C.fast.weight(x, None, pk, sc, None))
+        return fp4.quantize_pack_mxfp4(x), mxfp4_gemm.mxfp4_linear_w(x, pk, sc)
+
+    def fake():
+        with FakeTensorMode(allow_non_fake_inputs=True):
+            return call()
+
+    def grad():
+        return torch.func.grad(lambda s: (call()[1].float() * s).sum())(torch.ones((), device=dev))
+
+    for f in (fake, grad):
+        assert _same(_outcome(f), _general(monkeypatch, C, f))
+    assert native and all(r is None for r in native)
+    assert C.fast.quantize(x) is not None
