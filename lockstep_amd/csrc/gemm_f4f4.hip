@@ -675,7 +675,9 @@ LSMX_DEV void qepi_store(const uint32_t (&cb)[4][8][2], const uint32_t (&cam)[2]
     }
 }
 
-template <int JB, int CT, bool EPI = false>
+// LONG: rows of kShortRow bytes and more, whose loads have a descriptor each
+// instead of a multiple of 32 rows in their offsets.
+template <int JB, int CT, bool EPI = false, bool LONG = false>
 __global__ __launch_bounds__(512, 1) void gemm_f4f4_mx16_kernel(GemmArgs g) {
     using namespace f4;
     constexpr int S = 2;                             // ring slots
@@ -737,6 +739,7 @@ __global__ __launch_bounds__(512, 1) void gemm_f4f4_mx16_kernel(GemmArgs g) {
         int64_t n;
     };
     Panel pA, pB, pS;
+    Panel cA, cB;                                    // LONG: the stage's first rows
     const int64_t sstep = NSL * s_ld * 4;            // scale bytes one stage advances
     auto set_refill_origin = [&](int64_t m0, int64_t n0) {
         pA = Panel{g.a + m0 * g.lda, (min(g.M - m0, (int64_t)BM) - 1) * g.lda + g.K / 2};
@@ -754,11 +757,13 @@ __global__ __launch_bounds__(512, 1) void gemm_f4f4_mx16_kernel(GemmArgs g) {
     v4i_rsrc rsA, rsB, rsS;
     auto make_desc_a = [&](int kt) {
         const int64_t ko = (int64_t)kt * BKB;
-        rsA = buf_rsrc(pA.p + ko, (uint64_t)(pA.n - ko));
+        if constexpr (LONG) cA = Panel{pA.p + ko, pA.n - ko};
+        else rsA = buf_rsrc(pA.p + ko, (uint64_t)(pA.n - ko));
     };
     auto make_desc_b = [&](int kt) {
         const int64_t ko = (int64_t)kt * BKB;
-        rsB = buf_rsrc(pB.p + ko, (uint64_t)(pB.n - ko));
+        if constexpr (LONG) cB = Panel{pB.p + ko, pB.n - ko};
+        else rsB = buf_rsrc(pB.p + ko, (uint64_t)(pB.n - ko));
     };
     auto make_desc_s = [&](int kt) {
         const int64_t so = (int64_t)kt * sstep;
@@ -768,7 +773,11 @@ __global__ __launch_bounds__(512, 1) void gemm_f4f4_mx16_kernel(GemmArgs g) {
         if (q < 2 * XA) {
             const int i = q >> 1;
             const uint32_t m0 = lds_u32((q & 1) ? &sB[0][0] : &sA[0][0]) + s * TILE_B + (i * NLW + wave) * 1024;
-            if ((q & 1) == 0) dma_x4_at(offA0, i, stepA, rsA, m0);
+            if constexpr (LONG) {
+                const Panel &c = (q & 1) ? cB : cA;
+                const int64_t d = (int64_t)i * (NLW * RPI) * ((q & 1) ? g.ldb : g.lda);
+                dma_x4((q & 1) ? offB0 : offA0, buf_rsrc(c.p + d, (uint64_t)max(c.n - d, (int64_t)0)), m0);
+            } else if ((q & 1) == 0) dma_x4_at(offA0, i, stepA, rsA, m0);
             else dma_x4_at(offB0, i, stepB, rsB, m0);
             return;
         }
@@ -1320,9 +1329,10 @@ static const TileCost kTiles[] = {
     {256, 256, 1, 8.5f, 1.00f, 1.60f}, {256, 128, 1, 6.0f, 0.62f, 0.86f}, {192, 128, 1, 4.2f, 0.50f, 0.72f},
     {128, 128, 1, 3.5f, 0.43f, 0.58f}, {64, 128, 2, 2.6f, 0.36f, 0.665f}, {64, 64, 2, 2.0f, 0.27f, 0.45f},
 };
+// dma_x4_at forms i * (32 * ld) in a 24-bit multiply
+constexpr int64_t kShortRow = (int64_t)1 << 19;
 hipError_t launch_gemm_f4f4(const GemmArgs &g, hipStream_t s) {
-    // the 16 x 16 x 128 kernels form 32 * ld * i in 24-bit multiplies
-    const bool kmajor = g.scale_fmt == LSMX_SCALE_E8M0_KMAJOR && g.lda < (1 << 19) && g.ldb < (1 << 19);
+    const bool kmajor = g.scale_fmt == LSMX_SCALE_E8M0_KMAJOR && g.lda < kShortRow && g.ldb < kShortRow;
     if (kmajor) {
         int tile = pick_tile(kTiles, g.M, g.N, 1, (g.K + 255) / 256, num_cus());
         switch (tile) {
@@ -1359,7 +1369,8 @@ hipError_t launch_gemm_f4f4(const GemmArgs &g, hipStream_t s) {
 hipError_t launch_gemm_f4f4_quant(const GemmArgs &g, hipStream_t s) {
     const int tiles = (int)((g.M / f4::BM) * (g.N / f4::BN));
     const int grid = tiles < num_cus() ? tiles : num_cus();
-    hipLaunchKernelGGL((gemm_f4f4_mx16_kernel<4, LSMX_BF16, true>), grid, 512, 0, s, g);
+    if (g.lda < kShortRow && g.ldb < kShortRow) hipLaunchKernelGGL((gemm_f4f4_mx16_kernel<4, LSMX_BF16, true>), grid, 512, 0, s, g);
+    else hipLaunchKernelGGL((gemm_f4f4_mx16_kernel<4, LSMX_BF16, true, true>), grid, 512, 0, s, g);
     return hipGetLastError();
 }
 

@@ -87,3 +87,22 @@ def test_quant_epilogue_other_shapes_fall_back(dev, mods):
     GEMM and then the quantizer, with the same results."""
     fp4, mg = mods
     _check(fp4, mg, *_operands(fp4, dev, 384, 256, 512, seed=8), keep=True)
+
+
+@pytest.mark.parametrize("lda,ldb", [(1 << 19, 0), (0, 1 << 19), ((1 << 19) + 16, (1 << 19) + 4096)])
+def test_quant_epilogue_long_rows(dev, mods, lda, ldb):
+    """Rows of 2^19 bytes and more, where 32 rows pass 2^24 bytes: the bits of dense rows."""
+    fp4, mg = mods
+    M, N, K = 512, 256, 768
+    apk, ak, bpk, bk = _operands(fp4, dev, M, N, K, seed=19)
+    want = mg.mxfp4_gemm_packed_q2d(apk, bpk, ak, bk, keep_output=True)
+
+    def spread(t, ld):
+        if not ld:
+            return t
+        wide = torch.zeros((t.shape[0], ld), dtype=torch.uint8, device=dev)
+        wide[:, :t.shape[1]] = t
+        return wide[:, :t.shape[1]]
+    got = mg.mxfp4_gemm_packed_q2d(spread(apk, lda), spread(bpk, ldb), ak, bk, keep_output=True)
+    for x, y in zip(got, want):
+        assert torch.equal(x.view(torch.uint8), y.view(torch.uint8))

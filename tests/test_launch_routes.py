@@ -37,3 +37,11 @@ def test_calls_of_several_threads_on_one_stream_keep_their_launches_together(tra
     r, = trace(["threads 20 4096 14336 3 20"])
     assert r["rc"] == 0 and r["launches"] == 2 * r["calls"], "this shape must be sliced"
     assert r["split"] == 0
+
+
+@pytest.mark.parametrize("lda,ldb", [(1 << 19, 0), (0, 1 << 19), ((1 << 24) - 16, (1 << 24) - 16)])
+def test_quantizing_gemm_takes_long_rows_on_its_long_row_form(trace, lda, ldb):
+    """32 rows of 2^19 bytes do not fit the plain form's 24-bit load offsets."""
+    short, long_ = trace(["f4q 512 512 512 524272 524272", f"f4q 512 512 512 {lda} {ldb}"])
+    assert [x[0] for x in short["launches"]] == ["gemm_f4f4_mx16_kernel<4, 1, true, false>"]
+    assert [x[0] for x in long_["launches"]] == ["gemm_f4f4_mx16_kernel<4, 1, true, true>"]
