@@ -232,33 +232,39 @@ int lsmx_gemm_bf16f4(const void *a, int64_t lda, const uint8_t *w_pk, int64_t ld
                      const void *w_scale, int64_t ld_sw, int scale_fmt, void *c, int c_dtype,
                      int64_t ldc, int64_t M, int64_t N, int64_t K, void *stream);
 
-/* Workspace bytes the split-K form of the bf16 x MXFP4 GEMM below needs at
- * this shape (single form: dual = 0, dual-batch form: dual = 1), or 0 when
- * the library does not split this shape.  It splits K in 2 or 4 slices when
- * the whole-K 128 x 256 output tiles would fill less than half of the CUs
- * (a few hundred activation rows against a wide weight, e.g. M = 128
- * against N = 14336: 128 x 128 tiles in 2 slices).  The answer depends on
- * M, N and K only, but the split itself runs only for E8M0 scales whose rows
- * are 16-byte aligned with a stride that is a multiple of 16 bytes; other
- * scales (fp32, or E8M0 rows of another alignment) run the whole-K kernels
- * and leave a given workspace unused, with other bits than the split form
- * (same tolerance).  The Python layer converts fp32 weight scales to E8M0
- * bytes first, so both forms of a weight take the same kernels there. */
+/* K slices that the bf16 x MXFP4 GEMM below runs at this shape when it has a
+ * workspace: 1 (whole K, the workspace stays unused) or 2 .. 16, where the
+ * output tiles of a few hundred rows or less would leave most CUs idle and a
+ * cost model of the tiles says that the slices and their sum are faster (e.g.
+ * M = 20 against N = 4096, K = 14336: 8 slices).  The answer depends on M, N
+ * and K only, but the slices run only for E8M0 scales whose rows are 4-byte
+ * aligned with a stride that is a multiple of 4 bytes, and lda, ldw < 2^22;
+ * other calls (fp32 scales, other alignments) run the whole-K kernels, with
+ * other bits than the sliced form (same tolerance).  The Python layer converts
+ * fp32 weight scales to E8M0 bytes first, so both forms of a weight take the
+ * same kernels there. */
+int lsmx_gemm_bf16f4_slices(int64_t M, int64_t N, int64_t K);
+
+/* Workspace bytes to give the GEMM below at this shape (single form: dual = 0,
+ * dual-batch form: dual = 1): a bound on the partial tiles of its slices, or 0
+ * where it never slices K.  Where the bound is not 0 the GEMM may still run
+ * whole K and use none of it: lsmx_gemm_bf16f4_slices tells, and a call may
+ * then pass a NULL workspace with the same result. */
 int64_t lsmx_gemm_bf16f4_workspace(int64_t M, int64_t N, int64_t K, int dual);
 
 /* lsmx_gemm_bf16f4 (a1 = c1 = NULL) or lsmx_gemm_dual_bf16f4 (both set)
- * with a caller-provided device workspace, which lets the library split K
- * (lsmx_gemm_bf16f4_workspace): each K slice of a 128-row output tile is
- * one workgroup that writes an fp32 partial tile to the workspace, and a
- * second kernel on the same stream adds the slices in slice order (a fixed
- * order: repeated calls, and the single and dual forms, give identical
+ * with a caller-provided device workspace, which lets the library slice K
+ * (lsmx_gemm_bf16f4_slices): each K slice of an output tile (32 to 192
+ * rows) is one workgroup that writes an fp32 partial tile to the workspace,
+ * and a second kernel on the same stream adds the slices in slice order (a
+ * fixed order: repeated calls, and the single and dual forms, give identical
  * bits).  The same sums as the reference's split-K GEMM (dual_gemm.py:
  * 117-179) without its atomics.  Workspace: 16-byte aligned, at least the
  * bytes lsmx_gemm_bf16f4_workspace returns, no initial contents required;
  * calls that share a workspace must be stream-ordered (calls of several host
  * threads on one stream are: the library enqueues the launches of one call
  * together).  A NULL workspace,
- * or a shape the library does not split, runs the whole-K kernels. */
+ * or a shape the library does not slice, runs the whole-K kernels. */
 int lsmx_gemm_bf16f4_ws(const void *a0, const void *a1, int64_t lda, const uint8_t *w_pk, int64_t ldw,
                         const void *w_scale, int64_t ld_sw, int scale_fmt, void *c0, void *c1, int c_dtype, int64_t ldc,
                         int64_t M, int64_t N, int64_t K, void *workspace, int64_t workspace_bytes, void *stream);

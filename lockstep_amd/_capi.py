@@ -50,6 +50,7 @@ SIGNATURES = {
     "lsmx_gemm_f4f4_quant": [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64,
                              _vp, _i64, _i64, _i64, _i64, _vp],
     "lsmx_gemm_bf16f4": [_vp, _i64, _vp, _i64, _vp, _i64, _int, _vp, _int, _i64, _i64, _i64, _i64, _vp],
+    "lsmx_gemm_bf16f4_slices": [_i64, _i64, _i64],
     "lsmx_gemm_bf16f4_workspace": [_i64, _i64, _i64, _int],
     "lsmx_gemm_bf16f4_ws": [_vp, _vp, _i64, _vp, _i64, _vp, _i64, _int, _vp, _vp, _int, _i64, _i64, _i64, _i64, _vp,
                             _i64, _vp],
@@ -174,6 +175,12 @@ def require_device(*tensors: torch.Tensor) -> None:
             raise RuntimeError(
                 "lockstep_amd runs its MXFP4 ops on a gfx950 GPU only; got a tensor on "
                 f"{t.device} (there is no CPU fallback)")
+
+
+def slice_bytes(M: int, N: int, K: int, dual: bool) -> int:
+    """Workspace bytes of the weight-only GEMM: 0 where it runs whole K."""
+    L = load()
+    return L.lsmx_gemm_bf16f4_workspace(M, N, K, int(dual)) if L.lsmx_gemm_bf16f4_slices(M, N, K) > 1 else 0
 
 
 _workspaces: dict = {}

@@ -54,10 +54,10 @@ bool aligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) %
 
 int elem_size(int dt) { return dt == LSMX_F32 ? 4 : 2; }
 
-// Split-K scratch of lsmx_gemm_bf16f4_noalloc: the largest partial-tile
-// workspace the library asks for on a 256-CU gfx950 (4 K slices x 2 batches
-// x 256 tiles' worth of 128 x 256 fp32 partials = 64 MiB; the single form
-// needs at most half).
+// Scratch of lsmx_gemm_bf16f4_noalloc for the partial tiles of sliced calls:
+// the largest workspace the library asks for on a 256-CU gfx950.  The slices
+// of one batch stay within 256 workgroups of 128 x 256 fp32 partials, 32 MiB;
+// two batches 64.
 constexpr int64_t kScratchBytes = (int64_t)64 << 20;
 
 }  // namespace
@@ -679,6 +679,7 @@ static int w4_common(const char *fn, const void *a0, const void *a1, int a_dtype
     lsmx::GemmArgs g{reinterpret_cast<const uint8_t *>(a0), reinterpret_cast<const uint8_t *>(a1), lda, nullptr, 0,
                      w_pk, ldw, w_scale, ld_sw, scale_fmt, c0, c1, c_dtype, ldc, M, N, K};
     g.ws = reinterpret_cast<float *>(ws);
+    g.splits = ws ? lsmx::gemm_bf16f4_slices(M, N, K) : 1;
     if (a_dtype != LSMX_BF16) return launched(lsmx::launch_gemm_xf4(g, a_dtype, (hipStream_t)stream), fn);
     return launched(lsmx::launch_gemm_bf16f4(g, (hipStream_t)stream), fn);
 }
@@ -700,6 +701,11 @@ int lsmx_gemm_dual_bf16f4(const void *a0, const void *a1, int64_t lda, const uin
 int64_t lsmx_gemm_bf16f4_workspace(int64_t M, int64_t N, int64_t K, int dual) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 128) return 0;
     return lsmx::gemm_bf16f4_workspace(M, N, K, dual != 0);
+}
+
+int lsmx_gemm_bf16f4_slices(int64_t M, int64_t N, int64_t K) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % 128) return 1;
+    return lsmx::gemm_bf16f4_slices(M, N, K);
 }
 
 int lsmx_gemm_bf16f4_ws(const void *a0, const void *a1, int64_t lda, const uint8_t *w_pk, int64_t ldw,

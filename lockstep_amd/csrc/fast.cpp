@@ -373,7 +373,7 @@ PyObject *weight(PyObject *, PyObject *const *a, Py_ssize_t n) {
     const Tensor c0 = make({M, N}, ot, *a0), c1 = dual ? make({M, N}, ot, *a0) : Tensor();
     void *s = stream_of(c0);
     if (at_ == at::kBFloat16) {
-        const int64_t nws = lsmx_gemm_bf16f4_workspace(M, N, K, dual);
+        const int64_t nws = lsmx_gemm_bf16f4_slices(M, N, K) > 1 ? lsmx_gemm_bf16f4_workspace(M, N, K, dual) : 0;
         void *wsp = nullptr;
         PyObject *keep = nullptr;
         if (nws > 0) {   // the split-K workspace of this device and stream

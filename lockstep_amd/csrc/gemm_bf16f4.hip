@@ -1899,14 +1899,16 @@ static int64_t partial_bytes(const TileCost &c, int64_t M, int64_t N, int splits
 static Plan best_plan(int64_t M, int64_t N, int64_t K, int nb, int splits, int64_t budget, bool ring) {
     const int cus = num_cus_w();
     const int64_t nk = K / wt::BK;
+    const int most = splits ? splits : imax(1, imin(16, (int)imin((int)nk, 1 << 20) / 2));
     Plan best{0, 1, 1e30f};
     for (int i = 0; i < kNumTiles; ++i) {
+        if (i == kRingTile && (splits > 1 || !ring)) continue;
         const TileCost &c = kTiles[i];
         const int64_t bm = i == kRingTile ? c.bm / nb : c.bm;
         const int64_t tiles = ((M + bm - 1) / bm) * ((N + c.bn - 1) / c.bn) * (i == kRingTile ? 1 : nb);
-        for (int sp = 1; sp <= 16 && 2 * sp <= imax(2, (int)imin((int)nk, 1 << 20)); ++sp) {
-            if ((splits && sp != splits) || (i == kRingTile && (sp > 1 || !ring))) continue;
-            if (sp > 1 && partial_bytes(c, M, N, sp) > budget) continue;
+        const int64_t slice = partial_bytes(c, M, N, 2) / 2;
+        for (int sp = splits ? splits : 1; sp <= (i == kRingTile ? 1 : most); ++sp) {
+            if (sp > 1 && sp * slice > budget) break;
             float t = tile_time(c, tiles * sp, (nk + sp - 1) / sp, cus);
             if (sp > 1) t += 1.2f + (float)sp * (0.45f + 0.6e-6f * (float)(nb * M * N * 4));
             if (t < best.us) best = Plan{i, sp, t};
@@ -1914,12 +1916,25 @@ static Plan best_plan(int64_t M, int64_t N, int64_t K, int nb, int splits, int64
     }
     return best;
 }
+
+// up to 32 rows against a small weight: the skinny kernel (launch_gemm_bf16f4)
+static bool small_weight(int64_t N, int64_t K) { return N <= 16 * (int64_t)num_cus_w() && K <= 2048; }
+
 // The slices depend on M, N and K only, so the single and the dual launch of
 // one M add the same partial sums and give identical bits; the tile of the
 // dual form is chosen for its own number of tiles.
-static Plan bf16f4_plan(int64_t M, int64_t N, int64_t K, bool dual, bool ws, bool ring) {
-    const Plan one = best_plan(M, N, K, 1, ws ? 0 : 1, ws ? split_budget(M, N, K) : 0, ring);
-    return dual ? best_plan(M, N, K, 2, one.splits, split_budget(M, N, K), ring) : one;
+int gemm_bf16f4_slices(int64_t M, int64_t N, int64_t K) {
+    const int64_t budget = split_budget(M, N, K);
+    if (budget == 0 || (M <= kSkinnyMaxM && small_weight(N, K))) return 1;
+    // a call asks twice, before it allocates a workspace and at its launch: the
+    // search (0.4 us) runs once
+    static thread_local int64_t last[3] = {0, 0, 0};
+    static thread_local int slices = 1;
+    if (M != last[0] || N != last[1] || K != last[2]) {
+        slices = best_plan(M, N, K, 1, 0, budget, K % 512 == 0).splits;
+        last[0] = M, last[1] = N, last[2] = K;
+    }
+    return slices;
 }
 
 // Workspace bytes to give: the budget, for each batch.
@@ -2012,14 +2027,13 @@ hipError_t launch_gemm_bf16f4(const GemmArgs &g, hipStream_t s) {
     // 2 .. 16 rows: the decode kernel while one pass covers K (M = 16, 4096 x
     // 4096: 9.9 us against 9.1 - 9.7 in slices; M = 16, 14336 x 4096: 11.8
     // against 12.4), past that K slices (M = 4, 4096 x 14336: 23.1 against 12.7)
-    const bool slices = tiles && g.ws && split_budget(g.M, g.N, g.K) > 0;
-    if (g.M <= kDecodeMaxM && decode_ok(g) && (g.K <= dk::PASS_K || !slices)) return launch_decode(g, s);
+    const int splits = tiles && g.ws ? g.splits : 1;
+    if (g.M <= kDecodeMaxM && decode_ok(g) && (g.K <= dk::PASS_K || splits == 1)) return launch_decode(g, s);
     // few rows against a small weight: the skinny kernel's 16-row tiles spread
     // it over more CUs (M = 32, 2048 x 2048: 7.3 us against 7.9)
-    const bool small = g.N <= 16 * (int64_t)num_cus_w() && g.K <= 2048;
-    if (g.M <= kSkinnyMaxM && (g.a1 ? 2 * g.M : g.M) <= 128 && (small || !tiles)) return launch_skinny(g, s);
+    if (g.M <= kSkinnyMaxM && (small_weight(g.N, g.K) || !tiles)) return launch_skinny(g, s);
     if (!tiles) return g.a1 ? launch_w4_any<2>(g, s) : launch_w4_any<1>(g, s);
-    const Plan p = bf16f4_plan(g.M, g.N, g.K, g.a1 != nullptr, g.ws != nullptr, ring_ok(g));
+    const Plan p = best_plan(g.M, g.N, g.K, g.a1 ? 2 : 1, splits, splits > 1 ? split_budget(g.M, g.N, g.K) : 0, ring_ok(g));
     switch (p.tile) {
     case 0: return launch_tile<1, 4, 1, 1, 4, 4>(g, p.splits, s);
     case 1: return launch_tile<1, 4, 2, 1, 3, 4, 2>(g, p.splits, s);

@@ -193,8 +193,10 @@ hipError_t launch_gemm_f4f4(const GemmArgs &g, hipStream_t s);
 hipError_t launch_gemm_f4f4_quant(const GemmArgs &g, hipStream_t s);
 hipError_t launch_gemm_bf16f4(const GemmArgs &g, hipStream_t s);
 hipError_t launch_gemm_xf4(const GemmArgs &g, int a_dtype, hipStream_t s);
-// workspace bytes within which the weight-only GEMM may split K at this shape
-// (0: it does not)
+// K slices of the weight-only GEMM at this shape, given a workspace (1: whole
+// K), and the workspace bytes within which its partial tiles stay (0: it never
+// slices there)
+int gemm_bf16f4_slices(int64_t M, int64_t N, int64_t K);
 int64_t gemm_bf16f4_workspace(int64_t M, int64_t N, int64_t K, bool dual);
 hipError_t launch_gemm_dense(const DenseArgs &g, int dtype, int mode, hipStream_t s);
 bool dense_ring_ok(const DenseArgs &g, int dtype);

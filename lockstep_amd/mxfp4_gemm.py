@@ -186,8 +186,8 @@ def mxfp4_gemm_bf16(a, w_pk, w_scale, out_dtype=torch.bfloat16):
     w_scale = _wscales(w_scale, N, K // 32)
     c = torch.empty((M, N), device=a.device, dtype=out_dtype)
     if a.dtype == torch.bfloat16:
-        # with a workspace the library may split K (mid-size M against a wide W)
-        nws = C.load().lsmx_gemm_bf16f4_workspace(M, N, K, 0)
+        # with a workspace the library may slice K (few tiles facing a long K)
+        nws = C.slice_bytes(M, N, K, dual=False)
         ws = C.workspace(a.device, nws) if nws > 0 else None
         C.call("lsmx_gemm_bf16f4_ws", a.data_ptr(), None, a.stride(0) if M > 1 else K, w_pk.data_ptr(),
                w_pk.stride(0) if N > 1 else Kh, w_scale.data_ptr(), w_scale.stride(0) if N > 1 else K // 32,

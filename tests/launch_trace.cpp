@@ -104,9 +104,9 @@ T *P() {
     return reinterpret_cast<T *>(0x100000);
 }
 
-std::string answer(int rc, int64_t need) {
+std::string answer(int rc, int64_t need = 0, int slices = 1) {
     std::ostringstream o;
-    o << "{\"rc\": " << rc << ", \"workspace\": " << need << ", \"launches\": [";
+    o << "{\"rc\": " << rc << ", \"workspace\": " << need << ", \"slices\": " << slices << ", \"launches\": [";
     for (size_t i = 0; i < g_launches.size(); ++i)
         o << (i ? ", " : "") << "[\"" << g_launches[i].name << "\", " << g_launches[i].grid << "]";
     o << "]}";
@@ -137,33 +137,33 @@ int main(int argc, char **argv) {
             const int64_t lda = arg(K), ldw = arg(K / 2), lds = arg(K / 32);
             const int64_t need = L(lsmx_gemm_bf16f4_workspace)(M, N, K, dual);
             const int rc = w4(M, N, K, dual, ws ? need : 0, fmt, lda, ldw, lds);
-            std::cout << answer(rc, need) << std::endl;
+            std::cout << answer(rc, need, L(lsmx_gemm_bf16f4_slices)(M, N, K)) << std::endl;
         } else if (op == "f4") {
             const int fmt = (int)arg();
             const int64_t lda = arg(K / 2), ldb = arg(K / 2);
             const bool km = fmt == LSMX_SCALE_E8M0_KMAJOR;
             const int rc = L(lsmx_gemm_f4f4)(P<uint8_t>(), lda, P(), km ? M : K / 32, P<uint8_t>(), ldb, P(),
                                              km ? N : K / 32, fmt, P(), LSMX_F32, N, M, N, K, nullptr);
-            std::cout << answer(rc, 0) << std::endl;
+            std::cout << answer(rc) << std::endl;
         } else if (op == "f4q") {
             const int64_t lda = arg(K / 2), ldb = arg(K / 2);
             const int rc = L(lsmx_gemm_f4f4_quant)(P<uint8_t>(), lda, P(), M, P<uint8_t>(), ldb, P(), N, P(), N,
                                                    P<uint8_t>(), N / 2, P<uint8_t>(), M, P<uint8_t>(), M / 2,
                                                    P<uint8_t>(), N, M, N, K, nullptr);
-            std::cout << answer(rc, 0) << std::endl;
+            std::cout << answer(rc) << std::endl;
         } else if (op == "f8") {
             const int rc = arg() ? L(lsmx_gemm_f8f8_nb)(P<uint8_t>(), K, P<uint8_t>(), M, P<uint8_t>(), N, P<uint8_t>(), N,
                                                         P(), LSMX_F32, N, M, N, K, nullptr)
                                  : L(lsmx_gemm_f8f8)(P<uint8_t>(), K, P<uint8_t>(), M, P<uint8_t>(), K, P<uint8_t>(), N,
                                                      LSMX_SCALE_E8M0_KMAJOR, P(), LSMX_F32, N, M, N, K, nullptr);
-            std::cout << answer(rc, 0) << std::endl;
+            std::cout << answer(rc) << std::endl;
         } else if (op == "dense") {
             const int dt = (int)arg(), mode = (int)arg();
             const int rc = arg() ? L(lsmx_gemm_dense_nb)(P(), P(), K, P(), P(), N, dt, mode, P<float>(), P<float>(), N, M, N,
                                                          K, nullptr)
                                  : L(lsmx_gemm_dense)(P(), P(), K, P(), P(), K, dt, mode, P<float>(), P<float>(), N, M, N,
                                                       K, 1, nullptr);
-            std::cout << answer(rc, 0) << std::endl;
+            std::cout << answer(rc) << std::endl;
         } else if (op == "threads") {
             const int n = (int)arg(), calls = (int)arg();
             const int64_t need = L(lsmx_gemm_bf16f4_workspace)(M, N, K, 0);
