@@ -189,10 +189,11 @@ int lsmx_fp4_to_e4m3(const uint32_t *in, uint32_t *out, int64_t n_words, void *s
  * scales run the fastest kernels (16 x 16 x 128 scaled MFMA on 256-code
  * stages, with the output tile chosen by the shape); the other formats, and
  * K-major scales with lda or ldb >= 2^19, run a 32 x 32 x 64 kernel on
- * 128-code stages.  With K % 256 == 0 every format of the same scales sums
- * the blocks in the same groups; with K % 256 == 128 the two kernels group
- * them differently, so an fp32 sum that is not exact may differ in its last
- * bit between K-major and the other formats. */
+ * 128-code stages.  The two add the blocks of an output in different groups:
+ * where every partial sum is exact in fp32 all formats of the same scales give
+ * the same bits, other sums may differ in their rounding between K-major and
+ * the other formats (a quarter of the fp32 outputs at K = 2048 with block
+ * magnitudes over 24 binades). */
 int lsmx_gemm_f4f4(const uint8_t *a_pk, int64_t lda, const void *a_scale, int64_t ld_sa,
                    const uint8_t *bt_pk, int64_t ldb, const void *b_scale, int64_t ld_sb,
                    int scale_fmt, void *c, int c_dtype, int64_t ldc, int64_t M, int64_t N,
