@@ -11,6 +11,7 @@
 //   dense M N K dtype mode nc            lsmx_gemm_dense_nb or lsmx_gemm_dense
 //   threads M N K n calls                n threads x calls of lsmx_gemm_bf16f4_ws on one stream;
 //                                        "split": launches of a call that another thread's interrupted
+//   kernels                              the names of all kernels in the library
 // A leading dimension of 0 stands for the dense one.
 #include <cxxabi.h>
 #include <dlfcn.h>
@@ -184,6 +185,11 @@ int main(int argc, char **argv) {
             std::cout << "{\"rc\": " << rc << ", \"launches\": " << g_launches.size() << ", \"calls\": " << n * calls
                       << ", \"split\": " << runs - n * calls << "}" << std::endl;
             g_launches.clear();
+        } else if (op == "kernels") {
+            std::cout << "[";
+            const char *sep = "";
+            for (auto &k : g_names) std::cout << sep << "\"" << k.second << "\"", sep = ", ";
+            std::cout << "]" << std::endl;
         } else {
             return fprintf(stderr, "unknown command %s\n", op.c_str()), 2;
         }

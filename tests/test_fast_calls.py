@@ -73,27 +73,47 @@ def test_build_makes_both_libraries(monkeypatch, tmp_path):
     assert B.LIB.exists() and B.FAST_LIB.exists()
 
 
-def _general(monkeypatch, C, f):
-    """f() with every native call declined."""
-    class Declines:
-        def __getattr__(self, name):
-            return lambda *a: None
+class Recorder:
+    """Passes calls to the native path and notes which of them it took."""
+
+    def __init__(self, fast):
+        self._fast, self.took = fast, []
+
+    def __getattr__(self, name):
+        def call(*a):
+            r = getattr(self._fast, name)(*a)
+            self.took.append((name, r is not None))
+            return r
+        return call
+
+
+class Declines:
+    def __getattr__(self, name):
+        return lambda *a: None
+
+
+def _run_with(monkeypatch, C, fast, f):
     with monkeypatch.context() as m:
-        m.setattr(C, "fast", Declines())
-        return _outcome(f)
-
-
-def _outcome(f):
-    """What f returns, or the error it raises."""
-    try:
+        m.setattr(C, "fast", fast)
         return f()
-    except Exception as e:
-        return type(e), str(e)
+
+
+def _check(monkeypatch, C, f, native, error=None):
+    """f() gives the general path's result, and its first native call takes the
+    form (native), leaves it, or either (None); error: the type both raise
+    instead."""
+    rec = Recorder(C.fast)
+    if error:
+        assert not native
+        for fast in (rec, Declines()):
+            with pytest.raises(error):
+                _run_with(monkeypatch, C, fast, f)
+    else:
+        assert _same(_run_with(monkeypatch, C, rec, f), _run_with(monkeypatch, C, Declines(), f))
+    assert rec.took and native in (None, rec.took[0][1]), rec.took
 
 
 def _same(a, b):
-    if not isinstance(a, (tuple, list, torch.Tensor)):
-        return a == b
     if isinstance(a, (tuple, list)):
         return type(a) is type(b) and len(a) == len(b) and all(_same(x, y) for x, y in zip(a, b))
     return a.dtype == b.dtype and a.shape == b.shape and a.device == b.device and torch.equal(
@@ -109,16 +129,26 @@ def test_quantizers_match_the_python_path(C, monkeypatch, R, K, dtype):
     g = torch.Generator(device=dev).manual_seed(R + K)
     base = torch.randn((R, K + 16), device=dev, generator=g).to(dtype)
     other = torch.randn((K, R + 3), device=dev, generator=g).to(dtype)
-    for x in (base[:, :K], base[:, :K].contiguous(), base[:, 1:K + 1], other.t()[:R], base[:0, :K]):
-        forms = [lambda: fp4.quantize_mxfp4(x), lambda: fp4.quantize_pack_mxfp4(x),
-                 lambda: fp4.quantize_pack_mxfp4_many([x, x]), lambda: fp4.pack_fp4(fp4.quantize_mxfp4(x)[0])]
+    # (rows, taken): in place with 16-byte aligned starts; other alignments,
+    # other strides and empty tensors are the general path's
+    for x, ok in ((base[:, :K], True), (base[:, :K].contiguous(), True), (base[:, 1:K + 1], False),
+                  (other.t()[:R], False), (base[:0, :K], False)):
+        # one row is contiguous wherever it starts, so no copy aligns it
+        error = C.LsmxError if R == 1 and x.data_ptr() % 16 else None
+        forms = [(lambda: fp4.quantize_mxfp4(x), ok), (lambda: fp4.quantize_pack_mxfp4(x), ok),
+                 (lambda: fp4.quantize_pack_mxfp4_many([x, x]), ok)]
         if K % 128 == 0:
-            forms.append(lambda: fp4.quantize_pack_mxfp4(x, scale_layout="kmajor"))
-            forms.append(lambda: fp4.quantize_pack_mxfp4_many([x, x.contiguous()], scale_layout="kmajor"))
+            forms.append((lambda: fp4.quantize_pack_mxfp4(x, scale_layout="kmajor"), ok))
+            forms.append((lambda: fp4.quantize_pack_mxfp4_many([x, x.contiguous()], scale_layout="kmajor"), ok))
         if K % 128 == 0 and R % 128 == 0 and x.numel():
-            forms.append(lambda: fp4.quantize_pack_mxfp4_2d(x))
-        for f in forms:
-            assert _same(_outcome(f), _general(monkeypatch, C, f))
+            forms.append((lambda: fp4.quantize_pack_mxfp4_2d(x), ok and dtype != torch.float32))
+        for f, native in forms:
+            _check(monkeypatch, C, f, native, error)
+    codes = fp4.quantize_mxfp4(base[:, :K])[0]
+    # an empty tensor has no storage to pass: refused
+    for c, native, error in ((codes, True, None), (codes[:, :K - 32], R == 1, None), (codes[:0], False, C.LsmxError),
+                             (codes.reshape(-1), False, None)):
+        _check(monkeypatch, C, lambda: fp4.pack_fp4(c), native, error)
 
 
 @pytest.mark.gpu
@@ -135,30 +165,40 @@ def test_products_match_the_python_path(C, monkeypatch, M, N, K):
     odd = xs * 1.5   # scales that need the promotion
     wide = torch.zeros((M, K // 2 + 32), dtype=torch.uint8, device=dev)
     wide[:, :K // 2] = xp
-    forms = []
+    forms = []   # (call, taken by the native path, error)
     for dt in (torch.float32, torch.bfloat16, torch.float16):
-        for sa, sb in ((xk, wk), (xr, wr), (xs, ws), (xs.clone(), ws), (odd, ws), (xs.t().contiguous().t(), ws)):
-            forms.append(lambda sa=sa, sb=sb, dt=dt: mxfp4_gemm.mxfp4_gemm_packed(xp, wp, sa, sb, out_dtype=dt))
-        forms.append(lambda dt=dt: mxfp4_gemm.mxfp4_gemm_packed(wide[:, :K // 2], wp, xk, wk, out_dtype=dt))
+        # row-major E8M0 bytes and column-major fp32 scales are converted by the general path
+        for sa, sb, ok in ((xk, wk, True), (xr, wr, False), (xs, ws, True), (xs.clone(), ws, True), (odd, ws, True),
+                           (xs.t().contiguous().t(), ws, False)):
+            forms.append((lambda sa=sa, sb=sb, dt=dt: mxfp4_gemm.mxfp4_gemm_packed(xp, wp, sa, sb, out_dtype=dt), ok, None))
+        forms.append((lambda dt=dt: mxfp4_gemm.mxfp4_gemm_packed(wide[:, :K // 2], wp, xk, wk, out_dtype=dt), True, None))
         a, a1 = x.to(dt), x1.to(dt)
         pad = torch.zeros((M, K + 8), device=dev, dtype=dt)
         pad[:, :K] = a
-        for act in (a, pad[:, :K], a.t().contiguous().t()):
-            for sw in (wr, ws):
-                forms.append(lambda act=act, sw=sw: mxfp4_gemm.mxfp4_gemm_bf16(act, wp, sw))
-                forms.append(lambda act=act, sw=sw: mxfp4_gemm.mxfp4_linear_w(act, wp, sw))
-                forms.append(lambda act=act, sw=sw, a1=a1: dual_gemm.dual_mxfp4(act, a1, wp, sw, out_dtype=torch.float32))
+        for act, rows in ((a, True), (pad[:, :K], True), (a.t().contiguous().t(), False)):
+            for sw, e8m0 in ((wr, True), (ws, False)):
+                ok = rows and e8m0
+                forms.append((lambda act=act, sw=sw: mxfp4_gemm.mxfp4_gemm_bf16(act, wp, sw), ok, None))
+                forms.append((lambda act=act, sw=sw: mxfp4_gemm.mxfp4_linear_w(act, wp, sw), ok, None))
+                # both batches in one call: bf16 rows of one stride
+                forms.append((lambda act=act, sw=sw, a1=a1: dual_gemm.dual_mxfp4(act, a1, wp, sw, out_dtype=torch.float32),
+                              ok and dt == torch.bfloat16 and act.stride(0) == a1.stride(0), None))
         layer = MXFP4Linear(K, N).to(dev)
         layer.weight = torch.nn.Parameter(w.to(dt) if dt != torch.float16 else w)
         for t in (a, a.reshape(1, M, K)):
-            forms.append(lambda layer=layer, t=t: layer(t).detach())
+            forms.append((lambda layer=layer, t=t: layer(t).detach(), True, None))
+    forms.append((lambda: mxfp4_gemm.mxfp4_linear_w(x1.reshape(1, M, K), wp, wr), False, None))
+    forms.append((lambda: mxfp4_gemm.mxfp4_gemm_bf16(x1.double(), wp, wr), False, TypeError))
+    forms.append((lambda: dual_gemm.dual_mxfp4(x.bfloat16(), x1, wp, wr), False, TypeError))
     if N % 16 == 0:
         a8, b8 = fp4.codes_to_e4m3(xc), fp4.codes_to_e4m3(wc.t().contiguous())
         wst = ws.t().contiguous()
-        for sa, sb in ((xs, wst), (odd, wst), (xr, wr.t().contiguous())):
-            forms.append(lambda sa=sa, sb=sb: mxfp4_gemm.mxfp4_gemm_fp8(a8, b8, sa, sb))
-    for f in forms:
-        assert _same(_outcome(f), _general(monkeypatch, C, f))
+        for sa, sb, ok in ((xs, wst, True), (odd, wst, True), (xr, wr.t().contiguous(), False)):
+            forms.append((lambda sa=sa, sb=sb: mxfp4_gemm.mxfp4_gemm_fp8(a8, b8, sa, sb), ok, None))
+        forms.append((lambda: mxfp4_gemm.mxfp4_gemm_fp8(a8, fp4.codes_to_e4m3(wc).t(), xs, wst), False, None))
+    for f, native, error in forms:
+        # one row is dense in every layout: more forms are read in place
+        _check(monkeypatch, C, f, native or (None if min(M, N) == 1 else False), error)
 
 
 @pytest.mark.gpu
@@ -208,6 +248,11 @@ def test_calls_under_modes_and_transforms_take_the_python_path(C, monkeypatch):
         return torch.func.grad(lambda s: (call()[1].float() * s).sum())(torch.ones((), device=dev))
 
     for f in (fake, grad):
-        assert _same(_outcome(f), _general(monkeypatch, C, f))
+        errors = []
+        for fast in (C.fast, Declines()):
+            with pytest.raises(Exception) as e:
+                _run_with(monkeypatch, C, fast, f)
+            errors.append((e.type, str(e.value)))
+        assert errors[0] == errors[1]
     assert native and all(r is None for r in native)
     assert C.fast.quantize(x) is not None

@@ -12,16 +12,20 @@ pytestmark = pytest.mark.gpu
 Q = [0, 1, 2, 3, 4, 6, 8, 12, -1, -2, -3, -4, -6, -8, -12]
 
 
+# the tile of one product (gemm, packed); two products count twice the tiles
+SHAPES = [
+    (1, 8, 64), (64, 64, 128), (65, 72, 192), (500, 520, 640), (511, 2040, 320),     # 64 x 64
+    (1000, 1032, 1024),                                                              # 64 x 128
+    (2048, 2040, 512), (1500, 2000, 1024), (3000, 1000, 512),                        # 128 x 128
+    (2000, 2056, 256), (4095, 1032, 512), (4096, 4104, 192),                         # 192 x 128
+    (2048, 4096, 512),                                                               # 256 x 128
+    (4095, 4088, 320),                                                               # 256 x 256
+]
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("form", ["gemm", "packed", "separate"])
-@pytest.mark.parametrize("M,N,K", [
-    (1, 8, 64), (64, 64, 128), (65, 72, 192), (500, 520, 640),       # 64 x 64
-    (1000, 1032, 1024), (511, 2040, 320),                            # 64 x 128
-    (2048, 2040, 512), (2000, 2056, 256),                            # 128 x 128
-    (1500, 2000, 1024), (3000, 1000, 512),                           # 192 x 128
-    (4095, 1032, 512), (2048, 4096, 512),                            # 256 x 128
-    (4096, 4104, 192),                                               # 256 x 256
-])
+@pytest.mark.parametrize("M,N,K", SHAPES)
 def test_dense_tiles_bit_exact(M, N, K, form, dtype):
     from lockstep_amd import dual_gemm as D
     dev = torch.device("cuda", 0)

@@ -10,15 +10,18 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("M,N,K", [
+SHAPES = [
     (1, 16, 128), (64, 64, 256), (65, 80, 384), (300, 528, 1024), (131, 77, 256),   # 64 x 64
-    (256, 8176, 512), (700, 2064, 1024),                                            # 64 x 128
-    (700, 5008, 1024), (2048, 2032, 512),                                           # 128 x 128
-    (1500, 4096, 640), (1537, 4097, 256),                                           # 192 x 128
-    (1000, 8192, 1024), (4095, 2048, 512),                                          # 256 x 128
+    (256, 8176, 512), (700, 2064, 1024), (2048, 2032, 512),                         # 64 x 128
+    (700, 5008, 1024),                                                              # 128 x 128
+    (1500, 4096, 640),                                                              # 192 x 128
+    (1537, 4097, 256), (1000, 8192, 1024), (4095, 2048, 512),                       # 256 x 128
     (4096, 4080, 384),                                                              # 256 x 256
-])
+]
+
+
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", SHAPES)
 def test_fp8_tiles_bit_exact(M, N, K, out_dtype):
     from lockstep_amd import fp4, mxfp4_gemm
     dev = torch.device("cuda", 0)

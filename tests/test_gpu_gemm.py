@@ -145,12 +145,18 @@ def test_weight_only_bf16_x_fp4(dev, mods, oracle, out_dtype, M, N, K):
         assert oracle.max_rel(got.float().cpu().numpy(), ref) <= TOL[out_dtype]
 
 
-@pytest.mark.parametrize("M,N,K", [(2, 700, 512), (3, 300, 1536), (8, 1000, 4096), (16, 520, 8192),
-                                   (16, 260, 4608), (5, 14336, 4096)])
+# the decode kernel's shapes: one pass, and more than 16 weight rows per CU with
+# two passes (K = 8192; 4608: a second pass with one live slice)
+DECODE = [(2, 700, 512), (3, 300, 1536), (8, 1000, 4096), (5, 14336, 4096), (8, 14336, 8192), (16, 14331, 4608)]
+# few weight rows and K past one pass: K slices of the tile kernel
+DECODE_SLICED = [(16, 520, 8192), (16, 260, 4608)]
+
+
+@pytest.mark.parametrize("M,N,K", DECODE + DECODE_SLICED)
 def test_weight_only_decode_shapes(dev, mods, oracle, M, N, K):
-    """2 <= M <= 16 with K % 512 == 0 runs the decode kernel: 512-deep slices
-    per wave, 4096-deep passes (K = 8192: two; 4608: a second pass with one
-    live slice), ragged weight rows.  fp32 output vs the fp64 oracle; E8M0
+    """2 <= M <= 16 with K % 512 == 0 runs the decode kernel (512-deep slices
+    per wave, 4096-deep passes) unless a long K faces few weight rows; ragged
+    weight rows.  fp32 output vs the fp64 oracle; E8M0
     bytes and fp32 powers of two give the same bits; the dual form gives the
     single form's bits for both batches."""
     fp4, mg, dg, _ = mods
@@ -173,11 +179,8 @@ def test_weight_only_decode_shapes(dev, mods, oracle, M, N, K):
 @pytest.mark.parametrize("M,N,K", [(17, 4096, 512), (32, 5000, 4608), (48, 14336, 8192), (64, 14336, 4096),
                                    (40, 16384, 1024)])
 def test_weight_only_mid_m_shapes(dev, mods, oracle, M, N, K):
-    """17 <= M <= 64 against 16 .. 64 weight rows per CU with K % 512 == 0
-    runs the mid-M kernel (no split-K workspace is asked for): activation
-    groups of 64 rows (the dual forms of M = 48 and 64 have two; with
-    K = 8192 each group reloads its weight slices), a second pass with one
-    live slice (K = 4608), two live waves (K = 1024), ragged weight rows.
+    """17 <= M <= 64 against 16 .. 64 weight rows per CU: whole-K tiles of 32 or
+    64 rows (no workspace is asked for), ragged weight rows, long and short K.
     fp32 output vs the fp64 oracle; E8M0 bytes and fp32 powers of two give
     the same bits; the dual form gives the single form's bits for both
     batches; bf16 and fp16 outputs are the fp32 result rounded."""
@@ -203,7 +206,7 @@ def test_weight_only_mid_m_shapes(dev, mods, oracle, M, N, K):
 
 
 def test_weight_only_mid_m_special_scale_bytes(dev, mods, oracle):
-    """E8M0 bytes 0 (2^-127) and 255 (NaN) in the mid-M kernel: the NaN
+    """E8M0 bytes 0 (2^-127) and 255 (NaN) at 40 rows: the NaN
     byte's column is NaN, the others match the oracle."""
     fp4, mg, _, _ = mods
     M, N, K = 40, 14336, 4096
@@ -247,9 +250,8 @@ def test_weight_only_decode_nan_scale_byte(dev, mods, oracle):
 
 @pytest.mark.parametrize("M,N,K", [(4096, 4096, 512), (128, 14336, 512), (1000, 1000, 256), (1500, 4000, 512)])
 def test_weight_only_tile_paths(dev, mods, oracle, M, N, K):
-    """Large M runs 256 x 256 tiles, mid M (cfg3's M = 128) 128 x 128 tiles, and a single launch whose
-    256 x 256 tiles would leave CUs idle 128 x 256 tiles (1500 x 4000, ragged in both): all match the fp64
-    oracle on sampled rows, and give the same bits."""
+    """Large M runs 256 x 256 tiles, fewer output tiles smaller ones (128 x 14336: 64 x 128; 1500 x 4000,
+    ragged in both: 128 x 256): all match the fp64 oracle on sampled rows, and give the same bits."""
     fp4, mg, _, _ = mods
     g = torch.Generator(device=dev).manual_seed(M + N)
     a = torch.randn((M, K), device=dev, generator=g).to(torch.bfloat16)
@@ -334,18 +336,22 @@ def test_kmajor_scales_give_identical_gemm(dev, mods, oracle, M, N, K):
     assert oracle.max_rel(c_km.cpu().numpy(), ref) <= 1e-5
 
 
-@pytest.mark.parametrize("M,N,K", [(128, 14336, 4096), (200, 1000, 2048), (256, 4096, 1024), (64, 2304, 4096),
-                                   (256, 14336, 2048)])
-def test_weight_only_split_k(dev, mods, oracle, M, N, K):
-    """Mid-size M against a wide weight splits K (lsmx_gemm_bf16f4_ws): each
-    slice's fp32 partial tile goes to a workspace and a second kernel adds
-    the slices in slice order.  128 x 128 tiles in 2 or 4 slices at the
-    first four shapes, 128 x 256 tiles in 2 at the last.  vs fp64; repeated calls and the dual form
+@pytest.mark.parametrize("M,N,K,slices", [
+    (128, 14336, 4096, 1), (200, 1000, 2048, 1), (256, 4096, 1024, 1), (256, 14336, 2048, 1),
+    (64, 2304, 4096, 4), (20, 4096, 14336, 8), (162, 5000, 8192, 2), (240, 1024, 14336, 4), (100, 5000, 6144, 3)])
+def test_weight_only_split_k(dev, mods, oracle, M, N, K, slices):
+    """A workspace lets the GEMM cut K (lsmx_gemm_bf16f4_ws) where few output
+    tiles face a long K: each slice's fp32 partial tile goes to the workspace
+    and a second kernel adds the slices in slice order.  Sliced on 32 x 128
+    tiles (64 x 2304 and 20 x 4096), 64 x 128 (162, 240 and the dual form of
+    64 x 2304) and 128 x 128 ones (dual form of 100 x 5000), and shapes that
+    the plan leaves whole.  vs fp64; repeated calls and the dual form
     give the same bits; a call at another shape in between (sharing the
     cached workspace) does not disturb them."""
     fp4, mg, dg, _ = mods
     from lockstep_amd import _capi
-    assert _capi.load().lsmx_gemm_bf16f4_workspace(M, N, K, 0) > 0, "this shape must take the split-K path"
+    assert _capi.load().lsmx_gemm_bf16f4_workspace(M, N, K, 0) > 0
+    assert _capi.load().lsmx_gemm_bf16f4_slices(M, N, K) == slices
     g = torch.Generator(device=dev).manual_seed(M * 7 + K)
     a = torch.randn((M, K), device=dev, generator=g).to(torch.bfloat16)
     a1 = torch.randn((M, K), device=dev, generator=g).to(torch.bfloat16)
@@ -368,12 +374,14 @@ def test_weight_only_split_k(dev, mods, oracle, M, N, K):
     assert torch.equal(b16, c.to(torch.bfloat16))
 
 
-def test_weight_only_split_k_on_two_streams(dev, mods):
-    """Split-K calls running at once on two streams use one workspace per stream: the concurrent
+@pytest.mark.parametrize("M,N,K,slices", [(128, 14336, 4096, 1), (20, 4096, 14336, 8), (240, 1024, 14336, 4)])
+def test_weight_only_split_k_on_two_streams(dev, mods, M, N, K, slices):
+    """Sliced calls running at once on two streams use one workspace per stream: the concurrent
     results equal the sequential ones bit for bit, three rounds in a row."""
+    from lockstep_amd import _capi
     fp4, mg, _, _ = mods
+    assert _capi.load().lsmx_gemm_bf16f4_slices(M, N, K) == slices
     g = torch.Generator(device=dev).manual_seed(99)
-    M, N, K = 128, 14336, 4096
     a = [torch.randn((M, K), device=dev, generator=g).to(torch.bfloat16) for _ in range(2)]
     w = torch.randn((N, K), device=dev, generator=g) * 0.02
     wpk, we8 = fp4.quantize_pack_mxfp4(w)

@@ -9,15 +9,21 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("M,N,K", [
-    (2, 200, 4224), (4, 4096, 14336), (16, 1000, 8192), (15, 520, 1152),   # 32 x 128, sliced and not; skinny
-    (20, 4096, 14336), (20, 14330, 1024), (17, 5000, 640), (32, 130, 8192),
-    (33, 515, 1408), (64, 4096, 8320), (100, 4104, 4096), (128, 14336, 512),   # 64 x 128
-    (200, 14336, 640), (600, 4090, 1152), (1000, 2048, 2048),              # 128 x 128
-    (300, 14336, 1152), (1500, 4096, 640),                                 # 128 x 256
-    (600, 14336, 896), (577, 14330, 512),                                  # 192 x 256
-    (1000, 14336, 512), (4096, 4096, 640), (2048, 4090, 1536),             # 256 x 256 ring or 128 x 256
-])
+# the tile of the single form; the dual form counts twice the tiles
+SHAPES = [
+    (2, 200, 4224), (4, 4096, 14336), (16, 1000, 8192), (20, 4096, 14336), (32, 130, 8192), (64, 4096, 8320),  # 32 x 128, sliced
+    (20, 14330, 1024), (17, 5000, 640), (33, 515, 1408), (100, 4104, 4096),                                     # 32 x 128
+    (15, 520, 1152),                                                                                            # skinny
+    (162, 5000, 8192), (100, 5000, 6144),                          # 64 x 128, sliced (dual of 100: 128 x 128, sliced)
+    (128, 14336, 512), (1000, 2048, 2048),                         # 64 x 128
+    (200, 14336, 640), (600, 4090, 1152),                          # 128 x 128
+    (300, 14336, 1152), (1500, 4096, 640), (4096, 4096, 640), (2048, 4090, 1536),   # 128 x 256
+    (600, 14336, 896), (577, 14330, 512),                          # 192 x 256
+    (1000, 14336, 512),                                            # 256 x 256 ring
+]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
 def test_weight_tiles(M, N, K):
     from lockstep_amd import dual_gemm, fp4, mxfp4_gemm
     dev = torch.device("cuda", 0)

@@ -77,3 +77,67 @@ def test_slices_query_is_the_plan_that_runs(trace):
         assert grid * bm * bn * 4 <= r["workspace"]
         sliced += 1
     assert sliced > 100
+
+
+KMAJOR = C.SCALE_E8M0_KMAJOR
+
+
+def _launched(answers):
+    assert all(r["rc"] == 0 for r in answers)
+    return {name for r in answers for name, _ in r["launches"]}
+
+
+def _args(name):
+    return name[name.index("<") + 1:-1].split(", ")
+
+
+def test_gpu_tile_tests_reach_every_tile(trace):
+    """The shapes of the GPU tile tests launch every tile kernel of the library
+    (with fp32 outputs; bf16 operands for the dense ones) and the large-tile
+    kernel beside them."""
+    from tests import test_gpu_dense_tiles, test_gpu_f4_tiles, test_gpu_fp8_tiles, test_gpu_weight_tiles
+    kernels, = trace(["kernels 0 0 0"])
+
+    def instances(kernel, **fixed):
+        pos = {int(k[1:]): v for k, v in fixed.items()}
+        return {n for n in kernels if n.startswith(kernel + "<") and all(_args(n)[i] == v for i, v in pos.items())}
+
+    got = _launched(trace([f"f4 {m} {n} {k} {KMAJOR}" for m, n, k, _ in test_gpu_f4_tiles.SHAPES]))
+    want = instances("gemm_f4f4_tile_kernel", a3="0")
+    assert len(want) == 5 and got == want | {"gemm_f4f4_mx16_kernel<4, 0, false, false>"}
+
+    got = _launched(trace([f"f8 {m} {n} {k} {nc}" for m, n, k in test_gpu_fp8_tiles.SHAPES
+                           for nc in (0, 1) if not nc or n % 16 == 0]))
+    want = instances("gemm_f8f8_tile_kernel", a0="0")
+    assert len(want) == 10 and got == want | {"gemm_f8f8_kernel<0, true>", "gemm_f8f8_kernel<0, false>"}
+
+    got = _launched(trace([f"dense {m} {n} {k} 1 {mode} {nc}" for m, n, k in test_gpu_dense_tiles.SHAPES
+                           for mode in (0, 1, 2) for nc in (0, 1)]))
+    want = instances("gemm_dense_tile_kernel", a0="1") | instances("gemm_dense_ring_kernel", a0="1")
+    assert len(want) == 36 and got == want
+
+    # K slices on the tiles that the plan gives slices: 32, 64 and 128 rows x 128
+    got = _launched(trace([f"w4 {m} {n} {k} {dual} 1 0" for m, n, k in test_gpu_weight_tiles.SHAPES for dual in (0, 1)]))
+    whole = instances("gemm_bf16f4_tile_kernel", a0="0", a1="false")
+    sliced = {n for n in instances("gemm_bf16f4_tile_kernel", a1="true") if _args(n)[2:4] == ["1", "4"]}
+    assert len(whole) == 5 and len(sliced) == 3
+    assert got >= whole | sliced | {n for n in kernels if n.startswith("gemm_bf16f4_ring_kernel<") and _args(n)[1] == "0"}
+
+
+def test_decode_tests_run_the_decode_kernel(trace):
+    """More than 4096 K and more than 16 weight rows per CU: two passes of the
+    decode kernel; few weight rows: K slices."""
+    from tests import test_gpu_gemm
+    for shapes, kernel in ((test_gpu_gemm.DECODE, "gemm_bf16f4_decode_kernel"),
+                           (test_gpu_gemm.DECODE_SLICED, "gemm_bf16f4_tile_kernel")):
+        for r in trace([f"w4 {m} {n} {k} {dual} 1 0" for m, n, k in shapes for dual in (0, 1)]):
+            assert r["launches"][0][0].startswith(kernel + "<")
+    assert any(k > 4096 for _, _, k in test_gpu_gemm.DECODE)
+
+
+def test_long_rows_keep_off_the_24_bit_offsets(trace):
+    """K-major scales with rows of 2^19 bytes run the 32 x 32 x 64 kernel."""
+    for ld in ("524288 0", "0 524288"):
+        for k in (256, 384):
+            r, = trace([f"f4 70 50 {k} {KMAJOR} {ld}"])
+            assert r["launches"][0][0] == "gemm_f4f4_kernel<2, 4, 0>"

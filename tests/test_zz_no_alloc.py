@@ -3,9 +3,9 @@ tiles in the library's fixed device scratch instead of a caller workspace.
 
 Called through the C-ABI and checked bit for bit against lsmx_gemm_bf16f4_ws
 with a caller workspace (the same kernels in the same order), single and dual
-form, on two calls in a row, the second at a smaller shape (the scratch keeps
-the first call's partials; nothing in it has to start at zero), then a shape
-that takes the whole-K kernels (no scratch)."""
+form, on calls in a row at smaller and smaller shapes (the scratch keeps
+the earlier calls' partials; nothing in it has to start at zero), then shapes
+that take the whole-K kernels (no scratch)."""
 
 import pytest
 import torch
@@ -39,12 +39,14 @@ def test_noalloc_matches_workspace_form(dual):
     from lockstep_amd import fp4
     dev = torch.device("cuda", 0)
     L = C.load()
-    # 1: M = 128 against a 14336 x 4096 weight (4 K slices, the largest
-    # scratch use of this weight); 2: a smaller split shape; 3: whole K
-    for M, N, K, split in ((128, 14336, 4096, True), (64, 2304, 2048, True), (2048, 4096, 1024, False)):
+    # sliced shapes, each smaller in its partials than the one before it, two
+    # that have a workspace and run whole K, and one without a workspace
+    for M, N, K, slices, split in ((162, 5000, 8192, 2, True), (20, 4096, 14336, 8, True), (64, 2304, 4096, 4, True),
+                                   (128, 14336, 4096, 1, True), (64, 2304, 2048, 1, True),
+                                   (2048, 4096, 1024, 1, False)):
         print(f"[noalloc] dual={dual} M={M} N={N} K={K}", flush=True)
         need = L.lsmx_gemm_bf16f4_workspace(M, N, K, int(dual))
-        assert (need > 0) == split
+        assert (need > 0) == split and L.lsmx_gemm_bf16f4_slices(M, N, K) == slices
         a0, a1, wpk, we8 = _operands(dev, fp4, M, N, K, seed=M + N + K)
         a1 = a1 if dual else None
         ws = torch.empty(max(need, 16), dtype=torch.uint8, device=dev) if split else None
@@ -70,7 +72,8 @@ def test_noalloc_validates_like_the_workspace_form():
     assert "a1 and c1" in C.last_error()
 
 
-def test_noalloc_allocates_nothing_and_replays_under_graph_capture():
+@pytest.mark.parametrize("M,N,K,slices", [(20, 4096, 14336, 8), (128, 14336, 4096, 1)])
+def test_noalloc_allocates_nothing_and_replays_under_graph_capture(M, N, K, slices):
     """After a first call on the device (which looks up the scratch address),
     a call changes neither torch's allocator nor the device's free memory; and
     the call captured in a CUDA graph replays to the eager bits (the stated
@@ -78,9 +81,8 @@ def test_noalloc_allocates_nothing_and_replays_under_graph_capture():
     from lockstep_amd import _capi as C
     from lockstep_amd import fp4
     dev = torch.device("cuda", 0)
-    M, N, K = 128, 14336, 4096
     print(f"[noalloc] capture M={M} N={N} K={K}", flush=True)
-    assert C.load().lsmx_gemm_bf16f4_workspace(M, N, K, 0) > 0, "this shape must use the scratch"
+    assert C.load().lsmx_gemm_bf16f4_slices(M, N, K) == slices, "2 and more use the scratch"
     a0, _, wpk, we8 = _operands(dev, fp4, M, N, K, seed=5)
     c = torch.empty((M, N), device=dev, dtype=torch.float32)
 
