@@ -506,7 +506,7 @@ hipError_t launch_gemm_xf4(const GemmArgs &g, int a_dtype, hipStream_t s) {
 
 // ------------------------------------------------------------------ ring
 // The large-M form: 256 "A rows" x 256 weight columns per workgroup of 8 waves
-// (4 x 2, 64 x 128 per wave: two waves per SIMD, so one wave's MFMAs run
+// (2 x 4, 128 x 64 per wave: two waves per SIMD, so one wave's MFMAs run
 // while the other waits), a 3-slot LDS ring filled by direct-to-LDS loads
 // (no VGPR staging), one barrier per 64-deep K stage.
 //   - A stage is 128 bytes of every A row (64 bf16; 8 rows per load
@@ -531,55 +531,42 @@ hipError_t launch_gemm_xf4(const GemmArgs &g, int a_dtype, hipStream_t s) {
 namespace wr {
 constexpr int BK = 64;
 constexpr int NW = 8, NT = 64 * NW;
+constexpr int WGM = 2, WGN = NW / WGM;      // 2 x 4 waves, 128 x 64 each
+constexpr int NLW = 4;                      // loader waves
+constexpr int BR = 256, BN = 256;           // A rows (all batches) x weight columns
+constexpr int S = 3;                        // ring slots
 constexpr int A_ROW_B = BK * 2, W_ROW_B = BK / 2;
 constexpr int GROUP_M = 4;
 LSMX_DEV int swz(int row) { return (row >> 1) & 7; }
 }  // namespace wr
 
-// BR x BN tile (256 x 256 for large M; 128 x 64 and 128 x 128 for M of a few
-// hundred rows, where a 256-row tile would leave most CUs idle and every CU
-// streams all of A), S-slot ring.
-// WGM x (8 / WGM) waves: 4 x 2 (each wave a quarter of the rows and half of
-// the columns) or, for 128-row tiles, 1 x 8 (each wave all rows and a 32-
-// column strip, so every weight fragment is dequantized by one wave instead
-// of four: the dequantization is VALU work that does not shrink with the
-// tile's row count).
-// NLW loader waves issue the stage loads (all 8, or waves 0-3 only: the two
-// waves of a SIMD share its matrix core, the older one (0-3) wins issue
-// arbitration and reaches the barrier first, so the younger one's
-// instruction stream sets the stage's pace and is kept to LDS reads,
-// dequantization and MFMAs).
+// Only waves 0-3 issue the stage loads: the two waves of a SIMD share its
+// matrix core, the older one (0-3) wins issue arbitration and reaches the
+// barrier first, so the younger one's instruction stream sets the stage's
+// pace and is kept to LDS reads, dequantization and MFMAs.
 template <bool V>
 struct LoaderC {
     static constexpr bool value = V;
 };
-template <int NB, int CT, int BR, int BN, int S, int WGM = 4, int NLW = wr::NW>
+template <int NB, int CT>
 __global__ __launch_bounds__(wr::NT, 1) void gemm_bf16f4_ring_kernel(GemmArgs g) {
     using namespace wr;
     constexpr int RPB = BR / NB;        // A rows per batch per workgroup
-    constexpr int WGN = NW / WGM;
     constexpr int TM = BR / 32 / WGM, TN = BN / 32 / WGN;   // 32 x 32 tiles per wave
     static_assert(NB == 1 || TM * 32 <= RPB, "a wave's rows lie in one batch");
     constexpr int A_SLOT = BR * A_ROW_B, W_SLOT = BN * W_ROW_B;
     constexpr int XA = A_SLOT / 1024 / NLW;      // A load instructions per loader wave per stage
-    constexpr int WW = BN / 32;                  // W load instructions per stage (32 rows each)
-    constexpr int XWL = (WW + NLW - 1) / NLW;    // W loads per loader wave (some may be empty)
-    constexpr int L = XA + XWL;                  // (scales: one more every 8 stages)
-    constexpr int SWV = BN >= 64 ? BN / 64 : 1;  // distinct scale loads (64 rows each)
-    static_assert(TM >= 1 && TN >= 1 && XA >= 1 && S >= 3 && (A_SLOT / 1024) % NLW == 0 && NLW <= NW, "tile");
-    static_assert(NLW >= SWV, "every scale block needs a loader");
+    constexpr int XW = BN / 32 / NLW;            // W load instructions (32 rows each)
+    constexpr int L = XA + XW;                   // (scales: one more every 8 stages)
+    static_assert(NLW * 64 == BN, "one scale load per loader wave");
     // The scales of stages 8g+8 .. 8g+15 are issued first among stage 8g+6's
-    // loads and first read right after the barrier of stage 8g+7 (4 slots) or
-    // 8g+8 (3 slots); the wait at that barrier leaves (S - 3) L or (S - 2) L
-    // loads outstanding, which covers the scale load only for these depths.
-    static_assert(S == 3 || S == 4, "the scale prefetch distance assumes a 3- or 4-slot ring");
+    // loads and first read right after the barrier of stage 8g+8; the wait at
+    // that barrier leaves (S - 2) L loads outstanding, which covers the scale
+    // load only for this depth.
+    static_assert(S == 3, "the scale prefetch distance assumes a 3-slot ring");
     __shared__ __attribute__((aligned(16))) uint8_t sA[S][A_SLOT];
     __shared__ __attribute__((aligned(16))) uint8_t sW[S][W_SLOT];
     __shared__ __attribute__((aligned(16))) uint8_t sS[2][BN * 16];   // [group & 1][row][16 scale bytes]
-    // landing place of the loader waves' W loads past WW: they read nothing
-    // (an empty buffer descriptor: every lane out of range) and write zeros
-    // here, so that every loader counts the same loads
-    __shared__ __attribute__((aligned(16))) uint8_t sNull[XWL * NLW > WW ? 1024 : 16];
 
     const int tiles_m = (int)((g.M + RPB - 1) / RPB), tiles_n = (int)((g.N + BN - 1) / BN);
     const int tile = (int)blockIdx.x;
@@ -617,26 +604,20 @@ __global__ __launch_bounds__(wr::NT, 1) void gemm_bf16f4_ring_kernel(GemmArgs g)
         const int64_t left = g.M - (m0 + rb), rows = left < 8 ? (left > 0 ? left : 0) : 8;
         a_bytes[i] = rows > 0 ? (uint64_t)((rows - 1) * lda_b + g.K * 2) : 0;
     }
-    // W: load j of loader w covers slot rows (j*NLW + w)*32 .. +31 (when that
-    // is below BN), lane -> row lane%32, 16-byte half lane/32
+    // W: load j of loader w covers slot rows (j*NLW + w)*32 .. +31, lane -> row
+    // lane%32, 16-byte half lane/32
     const uint32_t w_off = (uint32_t)((lane & 31) * g.ldb + (lane >> 5) * 16);
-    const uint8_t *w_base[XWL];
-    uint64_t w_bytes[XWL];
-    uint32_t w_lds[XWL], w_slot[XWL];
+    const uint8_t *w_base[XW];
+    uint64_t w_bytes[XW];
 #pragma unroll
-    for (int j = 0; j < XWL; ++j) {
+    for (int j = 0; j < XW; ++j) {
         const int wi = j * NLW + wave;
-        const bool real = wi < WW;
-        w_base[j] = g.b + (n0 + (real ? wi : 0) * 32) * g.ldb;
-        const int64_t left = real ? g.N - (n0 + wi * 32) : 0, rows = left < 32 ? (left > 0 ? left : 0) : 32;
+        w_base[j] = g.b + (n0 + wi * 32) * g.ldb;
+        const int64_t left = g.N - (n0 + wi * 32), rows = left < 32 ? (left > 0 ? left : 0) : 32;
         w_bytes[j] = rows > 0 ? (uint64_t)((rows - 1) * g.ldb + g.K / 2) : 0;
-        w_lds[j] = real ? lds_u32(&sW[0][0]) + wi * 1024 : lds_u32(&sNull[0]);
-        w_slot[j] = real ? W_SLOT : 0;
     }
-    // scales: loader w loads 16 bytes of weight rows (w % SWV)*64 + lane
-    // (loaders w and w + SWV write the same bytes, so every loader counts the
-    // same loads)
-    const int s_w = wave % SWV;
+    // scales: loader w loads 16 bytes of weight rows 64 w + lane
+    const int s_w = wave % NLW;
     const int64_t s_rows = g.N - n0;
     const uint8_t *s_base = reinterpret_cast<const uint8_t *>(g.sb) + n0 * g.ld_sb;
     const uint32_t s_off = (uint32_t)(((s_w * 64) + lane) * g.ld_sb);
@@ -657,7 +638,8 @@ __global__ __launch_bounds__(wr::NT, 1) void gemm_bf16f4_ring_kernel(GemmArgs g)
             const int j = q - XA;
             const int64_t kw = (int64_t)kt * W_ROW_B;
             const uint64_t bytes = w_bytes[j] > 0 ? w_bytes[j] - (uint64_t)kw : 0;
-            dma_x4(w_off, buf_rsrc(w_base[j] + kw, bytes), w_lds[j] + slot * w_slot[j]);
+            dma_x4(w_off, buf_rsrc(w_base[j] + kw, bytes),
+                   lds_u32(&sW[0][0]) + slot * W_SLOT + (j * NLW + wave) * 1024);
         }
     };
 
@@ -684,14 +666,10 @@ __global__ __launch_bounds__(wr::NT, 1) void gemm_bf16f4_ring_kernel(GemmArgs g)
             for (int q = 0; q < L; ++q) issue(p < nk ? p : nk - 1, p, q);
     }
     // A stage's head: the W blocks and scales of this lane's columns and the
-    // A fragments of its first K-step; the rest of its A fragments are read
-    // one K-step ahead.  With 4 or more slots the head of stage u + 1 is read
-    // during the last K-step of stage u, so that a stage's MFMAs start right
-    // after its barrier; that needs stage u + 1 landed at the barrier of
-    // stage u, which a 3-slot ring cannot afford (measured: the wait for it
-    // costs more than the head read saves), so there the head is read after
-    // the barrier.
-    constexpr bool AHEAD = S >= 4;
+    // A fragments of its first K-step, read after its barrier; the rest of its
+    // A fragments are read one K-step ahead.  (Reading the head during the
+    // stage before needs that stage's loads one barrier earlier: the wait costs
+    // more than the head read saves.)
     u32x4 wblk[TN];
     uint32_t sraw[TN];
     v8bf fa0[TM];
@@ -709,24 +687,16 @@ __global__ __launch_bounds__(wr::NT, 1) void gemm_bf16f4_ring_kernel(GemmArgs g)
             fa0[i] = *reinterpret_cast<const v8bf *>(&sA[sl][r * A_ROW_B + (((4 * half) ^ swz(r)) << 4)]);
         }
     };
-    if constexpr (AHEAD) {
-        // stage 0 (and its scales) landed for every wave
-        if constexpr (LOADER) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 2) * L) : "memory");
-        else asm volatile("s_barrier" ::: "memory");
-        read_head(0);
-    }
     for (int u = 0; u < nk; ++u) {
         const int slot = u % S;
-        // this thread's loads of stage u + 1 (AHEAD) or u have landed (only
-        // the later stages up to u + S - 2 may be outstanding, and a scale
-        // load issued before the newest of them is waited for too); after
-        // the barrier everyone's have, and slot (u + S - 1) % S = (u - 1) % S
-        // is no longer read (a wave that issues no loads only meets the
-        // barrier)
-        constexpr int NOUT = (AHEAD ? S - 3 : S - 2) * L;
-        if constexpr (LOADER) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(NOUT) : "memory");
+        // this thread's loads of stage u have landed (only the later stages up
+        // to u + S - 2 may be outstanding, and a scale load issued before the
+        // newest of them is waited for too); after the barrier everyone's
+        // have, and slot (u + S - 1) % S = (u - 1) % S is no longer read (a
+        // wave that issues no loads only meets the barrier)
+        if constexpr (LOADER) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 2) * L) : "memory");
         else asm volatile("s_barrier" ::: "memory");
-        if constexpr (!AHEAD) read_head(u);
+        read_head(u);
         const int kn = u + S - 1 < nk ? u + S - 1 : nk - 1;
         const int sn = (u + S - 1) % S;
         // scales of the next group of 8 stages, first of this stage's loads
@@ -755,9 +725,7 @@ __global__ __launch_bounds__(wr::NT, 1) void gemm_bf16f4_ring_kernel(GemmArgs g)
                 const v2bf d3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(p, sc[j], 3);
                 fw[j] = v8bf{d0[0], d0[1], d1[0], d1[1], d2[0], d2[1], d3[0], d3[1]};
             }
-            // the next K-step's A fragments, or the next stage's head (its
-            // slot landed before this stage's barrier; past the last stage it
-            // holds a re-load of the last stage, read and discarded)
+            // the next K-step's A fragments
             if (st < 3) {
 #pragma unroll
                 for (int i = 0; i < TM; ++i) {
@@ -765,8 +733,6 @@ __global__ __launch_bounds__(wr::NT, 1) void gemm_bf16f4_ring_kernel(GemmArgs g)
                     fa[(st + 1) & 1][i] = *reinterpret_cast<const v8bf *>(
                         &sA[slot][r * A_ROW_B + (((4 * half + st + 1) ^ swz(r)) << 4)]);
                 }
-            } else if constexpr (AHEAD) {
-                read_head(u + 1);
             }
             // loads of stage u + S - 1, spread over the K-steps
             if constexpr (LOADER)
@@ -850,12 +816,12 @@ __global__ __launch_bounds__(wr::NT, 1) void gemm_bf16f4_ring_kernel(GemmArgs g)
         }
 }
 
-template <int NB, int BR, int BN, int S, int WGM = 4, int NLW = wr::NW>
+template <int NB>
 static hipError_t launch_ring(const GemmArgs &g, hipStream_t s) {
-    constexpr int RPB = BR / NB;
-    const int tiles = (int)(((g.M + RPB - 1) / RPB) * ((g.N + BN - 1) / BN));
+    constexpr int RPB = wr::BR / NB;
+    const int tiles = (int)(((g.M + RPB - 1) / RPB) * ((g.N + wr::BN - 1) / wr::BN));
     const dim3 grid(tiles), blk(wr::NT);
-#define LSMX_R(CT) hipLaunchKernelGGL((gemm_bf16f4_ring_kernel<NB, CT, BR, BN, S, WGM, NLW>), grid, blk, 0, s, g)
+#define LSMX_R(CT) hipLaunchKernelGGL((gemm_bf16f4_ring_kernel<NB, CT>), grid, blk, 0, s, g)
     if (g.c_dtype == LSMX_F32) LSMX_R(LSMX_F32);
     else if (g.c_dtype == LSMX_BF16) LSMX_R(LSMX_BF16);
     else LSMX_R(LSMX_F16);
@@ -1046,7 +1012,6 @@ constexpr int NW = 8, NT = 64 * NW;
 constexpr int SLICE_K = 512;          // K per wave per pass
 constexpr int PASS_K = NW * SLICE_K;  // 4096
 constexpr int ROW_B = SLICE_K / 2;    // code bytes of one row per slice
-constexpr int SC_ROW = PASS_K / 32;   // scale bytes of one row per pass
 }  // namespace dk
 
 // 16-byte global load from inline asm: its completion is waited for with an
@@ -1286,9 +1251,10 @@ static hipError_t launch_decode(const GemmArgs &g, hipStream_t s) {
     return vm <= 16 ? launch_decode_r<64, 1>(g, s) : launch_decode_r<32, 2>(g, s);
 }
 
-// The decode kernel's scale loads: 16-byte aligned rows of either format
-// (the same test for both, so that E8M0 bytes and fp32 powers of two of the
-// same scales pick the same kernel and give the same bits).
+// The decode kernel's scale loads: 16-byte aligned rows of either format.  Up
+// to one pass of K (PASS_K) E8M0 bytes and fp32 powers of two of the same
+// scales run this kernel and give the same bits; past it, E8M0 calls with a
+// workspace run K slices where gemm_bf16f4_slices says so.
 static bool decode_ok(const GemmArgs &g) {
     return g.K % dk::SLICE_K == 0 && (reinterpret_cast<uintptr_t>(g.sb) & 15) == 0 && g.ld_sb % 16 == 0;
 }
@@ -1859,7 +1825,8 @@ void gemm_bf16f4_tile_kernel(GemmArgs g) {
 //   4096x4096x4096                    121.3   111.9           107.4
 // K slices: partials and their reduction add ~1.2 us and, per slice, 0.45 us +
 // 0.6 us per MB, which pays where few tiles face a long K: 20x4096x14336 whole
-// K 38 us, 7 slices 13.6; 64x4096x14336 45 and 17; 200x1024x4096 16 and 12.3.
+// K 38 us, 7 or 8 slices 13.6 (8 is the plan's); 64x4096x14336 45 and 17;
+// 200x1024x4096 16 and 12.3.
 static const TileCost kTiles[] = {
     {32, 128, 2, 3.5f, 0.33f, 0.55f},  {64, 128, 2, 4.0f, 0.42f, 0.95f},  {128, 128, 1, 4.5f, 0.64f, 0.86f},
     {128, 256, 1, 4.5f, 1.20f, 1.66f}, {192, 256, 1, 5.5f, 1.80f, 2.05f}, {256, 256, 1, 8.0f, 2.20f, 3.05f},
@@ -2040,7 +2007,7 @@ hipError_t launch_gemm_bf16f4(const GemmArgs &g, hipStream_t s) {
     case 2: return launch_tile<1, 4, 4, 1, 3, 2>(g, p.splits, s);
     case 3: return launch_tile<2, 4, 2, 2, 3, 2>(g, p.splits, s);
     case 4: return launch_tile<2, 4, 3, 2, 2, 1>(g, p.splits, s);
-    default: return g.a1 ? launch_ring<2, 256, 256, 3, 2, 4>(g, s) : launch_ring<1, 256, 256, 3, 2, 4>(g, s);
+    default: return g.a1 ? launch_ring<2>(g, s) : launch_ring<1>(g, s);
     }
 }
 

@@ -15,6 +15,7 @@ SHAPES = [
     (20, 14330, 1024), (17, 5000, 640), (33, 515, 1408), (100, 4104, 4096),                                     # 32 x 128
     (15, 520, 1152),                                                                                            # skinny
     (162, 5000, 8192), (100, 5000, 6144),                          # 64 x 128, sliced (dual of 100: 128 x 128, sliced)
+    (117, 8255, 8832), (267, 3601, 12160),                         # dual: 128 x 256 and 192 x 256, sliced
     (128, 14336, 512), (1000, 2048, 2048),                         # 64 x 128
     (200, 14336, 640), (600, 4090, 1152),                          # 128 x 128
     (300, 14336, 1152), (1500, 4096, 640), (4096, 4096, 640), (2048, 4090, 1536),   # 128 x 256
