@@ -1489,13 +1489,15 @@ static int num_cus_w() {
     return cus;
 }
 
+// 16-row weight tiles per workgroup: two (the activation loads then serve
+// twice the weight bytes) while that still gives every CU a workgroup and the
+// activation tiles are at most 4; two workgroups are resident per CU either
+// way with up to 2 of them
+static int skinny_ct(int64_t vm, int64_t N) { return vm <= 64 && (N + 31) / 32 >= num_cus_w() ? 2 : 1; }
 static hipError_t launch_skinny(const GemmArgs &g, hipStream_t s) {
     const int64_t vm = g.a1 ? 2 * g.M : g.M;
     const int mt = vm <= 16 ? 1 : vm <= 32 ? 2 : vm <= 64 ? 4 : 8;
-    // two 16-row weight tiles per workgroup (the activation loads then serve
-    // twice the weight bytes) while that still gives every CU a workgroup;
-    // MT <= 2 keeps two workgroups resident per CU either way
-    const int ct = (mt <= 4 && (g.N + 31) / 32 >= num_cus_w()) ? 2 : 1;
+    const int ct = skinny_ct(vm, g.N);
     const dim3 grid((unsigned)((g.N + 16 * ct - 1) / (16 * ct))), blk(64 * sk::WK);
 #define LSMX_S(MT, CT) hipLaunchKernelGGL((gemm_bf16f4_skinny_kernel<MT, CT>), grid, blk, 0, s, g)
     switch (mt * 10 + ct) {
@@ -1884,25 +1886,55 @@ static Plan best_plan(int64_t M, int64_t N, int64_t K, int nb, int splits, int64
     return best;
 }
 
-// up to 32 rows against a small weight: the skinny kernel (launch_gemm_bf16f4)
-static bool small_weight(int64_t N, int64_t K) { return N <= 16 * (int64_t)num_cus_w() && K <= 2048; }
+// Time (us) of the skinny kernel at vm activation rows, a fit of 370 shapes,
+// M 1 .. 32, N 64 .. 65536, K 128 .. 28672, within 10%: a launch, then per 1024 K
+// one pass of 16 (32) weight rows per workgroup, and each further workgroup of
+// a CU.
+static float skinny_time(int64_t vm, int64_t N, int64_t K) {
+    const int64_t cus = num_cus_w();
+    const int ct = skinny_ct(vm, N);
+    const float more = (float)((N + 16 * ct * cus - 1) / (16 * ct * cus) - 1), v = (float)vm;
+    return 2.5f + 0.5f * more + (float)K / 1024.0f * (0.42f + 0.05f * v + more * (0.62f + 0.045f * v)) * (ct == 2 ? 1.32f : 1.0f);
+}
+
+// Route of a shape whose scales the tile kernel reads.
+struct Route {
+    bool skinny;
+    int splits;   // K slices, given a workspace
+};
+static Route find_route(int64_t M, int64_t N, int64_t K) {
+    // up to 32 rows against a small weight: the skinny kernel's 16-row tiles
+    // spread it over more CUs (M = 32, 2048 x 2048: 7.3 us against 7.9)
+    if (M <= kSkinnyMaxM && N <= 16 * (int64_t)num_cus_w() && K <= 2048) return Route{true, 1};
+    const int64_t budget = split_budget(M, N, K);
+    const bool few = M <= kDecodeMaxM && K % dk::SLICE_K != 0;
+    const Plan one = budget > 0 || few ? best_plan(M, N, K, 1, 0, budget, K % 512 == 0) : Plan{0, 1, 0.0f};
+    // up to 16 rows that the decode kernel does not take: the skinny kernel
+    // where its time is less than the tiles', both forms weighed alike (M = 2,
+    // 64 x 2944: 4.2 us against 9.7; M = 12, 2752 x 3328 6.9 and 12.0; M = 1,
+    // 320 x 21888 12.8 and 56; M = 10, 59200 x 6784 61 and 40)
+    if (few) {
+        const Plan two = best_plan(M, N, K, 2, one.splits, budget, false);
+        if (skinny_time(M, N, K) * skinny_time(2 * M, N, K) <= one.us * two.us) return Route{true, 1};
+    }
+    return Route{false, one.splits};
+}
+// A call asks twice, before it allocates a workspace and at its launch; the
+// search (up to 1 us) runs once.
+static Route route_of(int64_t M, int64_t N, int64_t K) {
+    static thread_local int64_t last[3] = {0, 0, 0};
+    static thread_local Route route;
+    if (M != last[0] || N != last[1] || K != last[2]) {
+        route = find_route(M, N, K);
+        last[0] = M, last[1] = N, last[2] = K;
+    }
+    return route;
+}
 
 // The slices depend on M, N and K only, so the single and the dual launch of
 // one M add the same partial sums and give identical bits; the tile of the
 // dual form is chosen for its own number of tiles.
-int gemm_bf16f4_slices(int64_t M, int64_t N, int64_t K) {
-    const int64_t budget = split_budget(M, N, K);
-    if (budget == 0 || (M <= kSkinnyMaxM && small_weight(N, K))) return 1;
-    // a call asks twice, before it allocates a workspace and at its launch: the
-    // search (0.4 us) runs once
-    static thread_local int64_t last[3] = {0, 0, 0};
-    static thread_local int slices = 1;
-    if (M != last[0] || N != last[1] || K != last[2]) {
-        slices = best_plan(M, N, K, 1, 0, budget, K % 512 == 0).splits;
-        last[0] = M, last[1] = N, last[2] = K;
-    }
-    return slices;
-}
+int gemm_bf16f4_slices(int64_t M, int64_t N, int64_t K) { return route_of(M, N, K).splits; }
 
 // Workspace bytes to give: the budget, for each batch.
 int64_t gemm_bf16f4_workspace(int64_t M, int64_t N, int64_t K, bool dual) {
@@ -1996,9 +2028,7 @@ hipError_t launch_gemm_bf16f4(const GemmArgs &g, hipStream_t s) {
     // against 12.4), past that K slices (M = 4, 4096 x 14336: 23.1 against 12.7)
     const int splits = tiles && g.ws ? g.splits : 1;
     if (g.M <= kDecodeMaxM && decode_ok(g) && (g.K <= dk::PASS_K || splits == 1)) return launch_decode(g, s);
-    // few rows against a small weight: the skinny kernel's 16-row tiles spread
-    // it over more CUs (M = 32, 2048 x 2048: 7.3 us against 7.9)
-    if (g.M <= kSkinnyMaxM && (small_weight(g.N, g.K) || !tiles)) return launch_skinny(g, s);
+    if (tiles ? route_of(g.M, g.N, g.K).skinny : g.M <= kSkinnyMaxM) return launch_skinny(g, s);
     if (!tiles) return g.a1 ? launch_w4_any<2>(g, s) : launch_w4_any<1>(g, s);
     const Plan p = best_plan(g.M, g.N, g.K, g.a1 ? 2 : 1, splits, splits > 1 ? split_budget(g.M, g.N, g.K) : 0, ring_ok(g));
     switch (p.tile) {

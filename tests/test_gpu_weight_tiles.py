@@ -11,9 +11,9 @@ pytestmark = pytest.mark.gpu
 
 # the tile of the single form; the dual form counts twice the tiles
 SHAPES = [
-    (2, 200, 4224), (4, 4096, 14336), (16, 1000, 8192), (20, 4096, 14336), (32, 130, 8192), (64, 4096, 8320),  # 32 x 128, sliced
+    (4, 4096, 14336), (16, 1000, 8192), (20, 4096, 14336), (32, 130, 8192), (64, 4096, 8320),  # 32 x 128, sliced
     (20, 14330, 1024), (17, 5000, 640), (33, 515, 1408), (100, 4104, 4096),                                     # 32 x 128
-    (15, 520, 1152),                                                                                            # skinny
+    (15, 520, 1152), (2, 200, 4224), (12, 2752, 3328), (1, 320, 17536),                                         # skinny
     (162, 5000, 8192), (100, 5000, 6144),                          # 64 x 128, sliced (dual of 100: 128 x 128, sliced)
     (117, 8255, 8832), (267, 3601, 12160),                         # dual: 128 x 256 and 192 x 256, sliced
     (128, 14336, 512), (1000, 2048, 2048),                         # 64 x 128

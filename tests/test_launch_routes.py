@@ -140,3 +140,20 @@ def test_long_rows_keep_off_the_24_bit_offsets(trace):
         for k in (256, 384):
             r, = trace([f"f4 70 50 {k} {KMAJOR} {ld}"])
             assert r["launches"][0][0] == "gemm_f4f4_kernel<2, 4, 0>"
+
+
+# us on the kernel named, and on the one that took the shape in between
+@pytest.mark.parametrize("M,N,K,dual", [
+    (1, 320, 21888, 0),     # 13.4, 55.5
+    (2, 64, 2944, 0),       # 4.3, 10.4
+    (12, 2752, 3328, 0),    # 6.5, 11.8
+    (2, 9152, 14208, 0),    # 25.8, 38.5
+    (6, 512, 2816, 1),      # 5.9, 10.2
+])
+def test_few_rows_of_any_depth_run_the_skinny_kernel(trace, M, N, K, dual):
+    """Up to 16 rows that the decode kernel does not take (K % 512 != 0)."""
+    r, r1 = trace([f"w4 {M} {N} {K} {dual} 1 0", f"w4 {M} {N} {K} {1 - dual} 1 0"])
+    for x in (r, r1):   # the single and the dual form alike
+        assert x["slices"] == 1 and x["launches"][0][0].startswith("gemm_bf16f4_skinny_kernel<")
+    wide, = trace(["w4 10 59200 6784 0 1 0"])   # 60 us on the skinny kernel, 40 here
+    assert wide["launches"][0][0].startswith("gemm_bf16f4_tile_kernel<")
