@@ -1573,7 +1573,9 @@ constexpr int lds(int bm, int bn, int s) { return s * (bm * A_ROW_B + bn * W_ROW
 // two workgroups per CU where the LDS holds both rings
 constexpr int waves_per_simd(int bm, int bn, int s, int waves) { return waves / 4 * (2 * lds(bm, bn, s) <= 160 * 1024 ? 2 : 1); }
 }  // namespace wt
-template <int CT, bool SPLITK, int WM, int WN, int TM, int TN, int S, int LA>
+// VEC: C rows start at multiples of 16 bytes and their length is a multiple of
+// 4 elements.
+template <int CT, bool SPLITK, int WM, int WN, int TM, int TN, int S, int LA, bool VEC>
 __global__ __launch_bounds__(64 * (WM * WN + wt::NLW), wt::waves_per_simd(32 * TM * WM, 32 * TN * WN, S, WM * WN + wt::NLW))
 void gemm_bf16f4_tile_kernel(GemmArgs g) {
     using namespace wt;
@@ -1788,24 +1790,35 @@ void gemm_bf16f4_tile_kernel(GemmArgs g) {
             }
     } else {
         void *c = batch ? g.c1 : g.c;
-        const bool vec_c = (reinterpret_cast<uintptr_t>(c) & 15) == 0 && g.ldc % 8 == 0;
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int gr = 0; gr < 4; ++gr) {
-                const int64_t row = m0 + (wm * TM + i) * 32 + 8 * gr + 4 * half + q;
+                const int64_t row = m0 + (wm * TM + i) * 32 + 8 * gr + 4 * half;
 #pragma unroll
                 for (int j = 0; j < TN; ++j) {
-                    float x[4] = {acc[i][j][4 * gr], acc[i][j][4 * gr + 1], acc[i][j][4 * gr + 2], acc[i][j][4 * gr + 3]};
-                    // all four lanes of a quad take part in the exchanges
-                    quad_transpose(x, q);
-                    const int64_t col = n0 + (wn * TN + j) * 32 + (frow & ~3);
-                    if (row < g.M && col < g.N) {
-                        if (vec_c && col + 4 <= g.N) store_c4<CT>(c, row * g.ldc + col, x[0], x[1], x[2], x[3]);
-                        else
+                    const int64_t col = n0 + (wn * TN + j) * 32;
+                    if constexpr (VEC) {
+                        float x[4] = {acc[i][j][4 * gr], acc[i][j][4 * gr + 1], acc[i][j][4 * gr + 2], acc[i][j][4 * gr + 3]};
+                        // all four lanes of a quad take part in the exchanges
+                        quad_transpose(x, q);
+                        const int64_t cq = col + (frow & ~3);
+                        if (row + q < g.M && cq < g.N) {
+                            if (cq + 4 <= g.N) store_c4<CT>(c, (row + q) * g.ldc + cq, x[0], x[1], x[2], x[3]);
+                            else
 #pragma unroll
-                            for (int k = 0; k < 4; ++k)
-                                if (col + k < g.N) store_c<CT>(c, row * g.ldc + col + k, x[k]);
+                                for (int k = 0; k < 4; ++k)
+                                    if (cq + k < g.N) store_c<CT>(c, (row + q) * g.ldc + cq + k, x[k]);
+                        }
+                    } else {
+                        // rows at any alignment: one element per lane, 32
+                        // columns of 2 rows per store (as quads of 4
+                        // columns each store touched 16 rows: 252 x 33771 x
+                        // 384 21.7 us on this tile, 19.1 so)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            if (row + e < g.M && col + frow < g.N)
+                                store_c<CT>(c, (row + e) * g.ldc + col + frow, acc[i][j][4 * gr + e]);
                     }
                 }
             }
@@ -1834,6 +1847,20 @@ static const TileCost kTiles[] = {
     {128, 256, 1, 4.5f, 1.20f, 1.66f}, {192, 256, 1, 5.5f, 1.80f, 2.05f}, {256, 256, 1, 8.0f, 2.20f, 3.05f},
 };
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]), kRingTile = kNumTiles - 1;
+// The same tiles at K <= 512 (kShortStages), where ramp and stores of a round
+// outweigh its stages and the fits above put the 256-column tiles 20 to 40% too
+// low: fits of 590 shapes, M 33 .. 32768, N 64 .. 65536, that pick the fastest
+// tile or one within 0.4% of it on average, 14% at worst.
+//   M x N x K              64x128  192x256  ring (256 x 256)
+//   30508x384x256            18.0     23.8             us
+//   2309x48000x512 (dual)   332.5    320.9    247.6
+//   12189x29056x512                    507      436
+constexpr int kShortStages = 4;
+static const TileCost kShortTiles[] = {
+    {32, 128, 2, 4.10f, 0.13f, 0.634f, -0.41f}, {64, 128, 2, 4.41f, 0.27f, 0.94f, -1.18f},
+    {128, 128, 1, 5.75f, 0.40f, 0.915f, -1.45f}, {128, 256, 1, 6.93f, 0.81f, 1.84f, -1.10f},
+    {192, 256, 1, 8.27f, 1.14f, 2.72f, -0.62f},  {256, 256, 1, 9.67f, 2.35f, 3.21f, -3.00f},
+};
 
 // Bytes of fp32 partials a shape may use (one batch): what fills the CUs once
 // with 128-row tiles of 256 or 128 columns in 2 or 4 slices.  0 where whole-K
@@ -1872,7 +1899,7 @@ static Plan best_plan(int64_t M, int64_t N, int64_t K, int nb, int splits, int64
     Plan best{0, 1, 1e30f};
     for (int i = 0; i < kNumTiles; ++i) {
         if (i == kRingTile && (splits > 1 || !ring)) continue;
-        const TileCost &c = kTiles[i];
+        const TileCost &c = nk <= kShortStages ? kShortTiles[i] : kTiles[i];
         const int64_t bm = i == kRingTile ? c.bm / nb : c.bm;
         const int64_t tiles = ((M + bm - 1) / bm) * ((N + c.bn - 1) / c.bn) * (i == kRingTile ? 1 : nb);
         const int64_t slice = partial_bytes(c, M, N, 2) / 2;
@@ -1981,26 +2008,29 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
 // still be there when its reduction runs.
 static std::mutex g_slices_mu;
 
-// LAS: LA of the K-slice form, whose epilogue holds two registers more: 64 x 128
-// tiles have 128 per lane (two workgroups per CU), and with LA = 4 spilled two
-template <int WM, int WN, int TM, int TN, int S, int LA, int LAS = LA>
+// LA: 64 x 128 tiles have 128 registers per lane (two workgroups per CU), which
+// LA = 4 overruns by two
+template <int WM, int WN, int TM, int TN, int S, int LA>
 static hipError_t launch_tile(GemmArgs g, int splits, hipStream_t s) {
     constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
     const int64_t tm = (g.M + BM - 1) / BM, tn = (g.N + BN - 1) / BN;
     const int nb = g.a1 ? 2 : 1;
     const dim3 grid((unsigned)(tm * tn * nb * splits)), blk(64 * (WM * WN + wt::NLW));
     g.splits = splits;
+    const bool vec = ((reinterpret_cast<uintptr_t>(g.c) | reinterpret_cast<uintptr_t>(g.c1)) & 15) == 0 && g.ldc % 4 == 0;
     const int64_t Mp = tm * BM, Np = tn * BN;
     const dim3 rgrid((unsigned)(nb * g.M * ((Np / 4 + 255) / 256))), rblk(256);
 #define LSMX_T(CT)                                                                                                 \
     do {                                                                                                           \
-        if (splits == 1) {                                                                                         \
-            hipLaunchKernelGGL((gemm_bf16f4_tile_kernel<CT, false, WM, WN, TM, TN, S, LA>), grid, blk, 0, s, g);        \
-        } else {                                                                                                   \
+        if (splits > 1) {                                                                                          \
             std::lock_guard<std::mutex> lk(g_slices_mu);                                                           \
-            hipLaunchKernelGGL((gemm_bf16f4_tile_kernel<LSMX_F32, true, WM, WN, TM, TN, S, LAS>), grid, blk, 0, s, g);  \
+            hipLaunchKernelGGL((gemm_bf16f4_tile_kernel<LSMX_F32, true, WM, WN, TM, TN, S, LA, true>), grid, blk, 0, s, g); \
             hipLaunchKernelGGL((splitk_reduce_kernel<CT>), rgrid, rblk, 0, s, g.ws, splits, nb, Mp, Np, g.c, g.c1, \
                                g.ldc, g.M, g.N);                                                                   \
+        } else if (vec) {                                                                                          \
+            hipLaunchKernelGGL((gemm_bf16f4_tile_kernel<CT, false, WM, WN, TM, TN, S, LA, true>), grid, blk, 0, s, g);  \
+        } else {                                                                                                   \
+            hipLaunchKernelGGL((gemm_bf16f4_tile_kernel<CT, false, WM, WN, TM, TN, S, LA, false>), grid, blk, 0, s, g); \
         }                                                                                                          \
     } while (0)
     if (g.c_dtype == LSMX_F32) LSMX_T(LSMX_F32);
@@ -2033,7 +2063,7 @@ hipError_t launch_gemm_bf16f4(const GemmArgs &g, hipStream_t s) {
     const Plan p = best_plan(g.M, g.N, g.K, g.a1 ? 2 : 1, splits, splits > 1 ? split_budget(g.M, g.N, g.K) : 0, ring_ok(g));
     switch (p.tile) {
     case 0: return launch_tile<1, 4, 1, 1, 4, 4>(g, p.splits, s);
-    case 1: return launch_tile<1, 4, 2, 1, 3, 4, 2>(g, p.splits, s);
+    case 1: return launch_tile<1, 4, 2, 1, 3, 2>(g, p.splits, s);
     case 2: return launch_tile<1, 4, 4, 1, 3, 2>(g, p.splits, s);
     case 3: return launch_tile<2, 4, 2, 2, 3, 2>(g, p.splits, s);
     case 4: return launch_tile<2, 4, 3, 2, 2, 1>(g, p.splits, s);

@@ -87,19 +87,22 @@ LSMX_HD int stage_tile_iter(int u, int nk, int my_tiles) { return imin(u / nk, m
 // Cost model for the output tile of a GEMM launch (host).  A launch of
 // `tiles` tiles on `cus` CUs with per_cu workgroups on each runs in rounds of
 // cap = cus * per_cu tiles and costs, in us,
-//   rounds * fix + stages * (hi per full round + the last round's time),
+//   rounds * fix + full rounds * more + stages * (hi per full round + the
+//   last round's time),
 // where the last round's stages take from lo (few tiles: the loads have the
 // L2s and the fabric to themselves) to hi (every CU loads): in proportion to
 // its tiles with one workgroup per CU; with two, lo until CUs get a second
-// one.  fix, lo and hi are measured per kernel and tile, see the tables.
+// one.  fix, lo, hi and more (what a round that another follows costs beside
+// its fix: stores that the next tile's loads wait behind, or less than fix
+// where the rounds overlap) are measured per kernel and tile, see the tables.
 struct TileCost {
     int bm, bn, per_cu;
-    float fix, lo, hi;
+    float fix, lo, hi, more = 0.0f;
 };
 inline float tile_time(const TileCost &c, int64_t tiles, int64_t stages, int cus) {
     const int64_t cap = (int64_t)cus * c.per_cu, full = (tiles - 1) / cap, last = tiles - full * cap;
     const float tl = c.per_cu == 1 ? c.lo + (c.hi - c.lo) * (float)last / (float)cap : last <= cus ? c.lo : c.hi;
-    return (float)(full + 1) * c.fix + (float)stages * ((float)full * c.hi + tl);
+    return (float)(full + 1) * c.fix + (float)full * c.more + (float)stages * ((float)full * c.hi + tl);
 }
 template <int NT>
 inline int pick_tile(const TileCost (&table)[NT], int64_t M, int64_t N, int64_t problems, int64_t stages, int cus) {

@@ -119,7 +119,7 @@ def test_gpu_tile_tests_reach_every_tile(trace):
     got = _launched(trace([f"w4 {m} {n} {k} {dual} 1 0" for m, n, k in test_gpu_weight_tiles.SHAPES for dual in (0, 1)]))
     whole = instances("gemm_bf16f4_tile_kernel", a0="0", a1="false")
     sliced = instances("gemm_bf16f4_tile_kernel", a1="true")
-    assert len(whole) == 5 and len(sliced) == 5
+    assert len(whole) == 10 and len(sliced) == 5
     assert got >= whole | sliced | {n for n in kernels if n.startswith("gemm_bf16f4_ring_kernel<") and _args(n)[1] == "0"}
 
 
@@ -157,3 +157,15 @@ def test_few_rows_of_any_depth_run_the_skinny_kernel(trace, M, N, K, dual):
         assert x["slices"] == 1 and x["launches"][0][0].startswith("gemm_bf16f4_skinny_kernel<")
     wide, = trace(["w4 10 59200 6784 0 1 0"])   # 60 us on the skinny kernel, 40 here
     assert wide["launches"][0][0].startswith("gemm_bf16f4_tile_kernel<")
+
+
+@pytest.mark.parametrize("M,N,K,dual,kernel", [
+    # us on the kernel named, and on the one that took the shape in between
+    (12189, 29056, 512, 0, "gemm_bf16f4_ring_kernel<1, 0>"),                               # 419, 504
+    (4829, 12864, 512, 1, "gemm_bf16f4_ring_kernel<2, 0>"),                                # 156, 197
+    (30508, 384, 256, 0, "gemm_bf16f4_tile_kernel<0, false, 1, 4, 2, 1, 3, 2, true>"),     # 18.4, 24.0
+    (252, 33771, 384, 0, "gemm_bf16f4_tile_kernel<0, false, 1, 4, 2, 1, 3, 2, false>"),    # 18.3, 27.8
+])
+def test_short_k_has_tiles_of_its_own(trace, M, N, K, dual, kernel):
+    r, = trace([f"w4 {M} {N} {K} {dual} 1 0"])
+    assert [x[0] for x in r["launches"]] == [kernel]

@@ -7,6 +7,8 @@ form, on calls in a row at smaller and smaller shapes (the scratch keeps
 the earlier calls' partials; nothing in it has to start at zero), then shapes
 that take the whole-K kernels (no scratch)."""
 
+import gc
+
 import pytest
 import torch
 
@@ -94,6 +96,7 @@ def test_noalloc_allocates_nothing_and_replays_under_graph_capture(M, N, K, slic
     torch.cuda.synchronize()
     ref = c.clone()
     torch.cuda.synchronize()
+    gc.collect()   # tensors of earlier tests that only reference cycles hold
     free0, _ = torch.cuda.mem_get_info()
     alloc0, reserved0 = torch.cuda.memory_allocated(), torch.cuda.memory_reserved()
     call()
