@@ -1021,14 +1021,11 @@ __global__ __launch_bounds__(512, 1) void gemm_f4f4_mx16_kernel(GemmArgs g) {
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j) {
-                    float x[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
-                    quad_transpose(x, q);
-                    const int64_t row = m0 + wm * 64 + 16 * i + 4 * egrp + q;
-                    const int64_t col = n0 + wn * 128 + 16 * j + (er16 & ~3);
-                    if (row < g.M)
+                    // one element per lane: 16 columns of 4 rows per store
+                    const int64_t row = m0 + wm * 64 + 16 * i + 4 * egrp, col = n0 + wn * 128 + 16 * j + er16;
 #pragma unroll
-                        for (int c = 0; c < 4; ++c)
-                            if (col + c < g.N) store_c<CT>(g.c, row * g.ldc + col + c, x[c]);
+                    for (int e = 0; e < 4; ++e)
+                        if (row + e < g.M && col < g.N) store_c<CT>(g.c, (row + e) * g.ldc + col, acc[i][j][e]);
                 }
         }
     }
@@ -1067,7 +1064,9 @@ __global__ __launch_bounds__(512, 1) void gemm_f4f4_mx16_kernel(GemmArgs g) {
 constexpr int f4_tile_lds(int tm, int tn, int s) {
     return s * ((tm + tn) * 32 * 128 + 2 * (((tm + 1) / 2) * 256 + 64 + ((tn + 1) / 2) * 256 + 64));
 }
-template <int TM, int TN, int S, int CT>
+// VEC: C rows start at multiples of 16 bytes and their length is a multiple of
+// 4 elements.
+template <int TM, int TN, int S, int CT, bool VEC>
 __global__ __launch_bounds__(512, 2) void gemm_f4f4_tile_kernel(GemmArgs g) {
     using namespace f4;
     constexpr int BM_ = 32 * TM, BN_ = 32 * TN;      // tile: 2 x 2 waves of 16 TM x 16 TN
@@ -1245,11 +1244,11 @@ __global__ __launch_bounds__(512, 2) void gemm_f4f4_tile_kernel(GemmArgs g) {
 
     // ---- epilogue: as in gemm_f4f4_mx16_kernel, whole 16-byte stores where
     // the rows are aligned and the columns inside C
-    const bool vec_c = ((reinterpret_cast<uintptr_t>(g.c) & 15) == 0) && (g.ldc % 8 == 0);
     const int q = lane & 3;
     const int64_t rb = m0 + wm * 16 * TM, cb = n0 + wn * 16 * TN;
-    if constexpr (CT != LSMX_F32 && TN % 2 == 0) {
-        if (vec_c) {
+    static_assert(TN % 2 == 0, "pairs of column blocks");
+    if constexpr (VEC) {
+        if constexpr (CT != LSMX_F32) {
             const bool odd = (lane & 4) != 0;
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
@@ -1271,23 +1270,39 @@ __global__ __launch_bounds__(512, 2) void gemm_f4f4_tile_kernel(GemmArgs g) {
                     }
                 }
             }
-            return;
+        } else {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    float x[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+                    quad_transpose(x, q);
+                    const int64_t row = rb + 16 * i + 4 * grp + q, col = cb + 16 * j + (r16 & ~3);
+                    if (row < g.M) {
+                        if (col + 4 <= g.N) store_c4<CT>(g.c, row * g.ldc + col, x[0], x[1], x[2], x[3]);
+                        else
+#pragma unroll
+                            for (int c = 0; c < 4; ++c)
+                                if (col + c < g.N) store_c<CT>(g.c, row * g.ldc + col + c, x[c]);
+                    }
+                }
         }
+        return;
     }
+    // rows at any alignment: one element per lane, 16 columns of 4 rows per
+    // store (as quads of 4 columns each store touched 16 rows: 4892 x 4660 x
+    // 896 on 256 x 128 tiles 60.9 us, 34.0 so)
+    const int64_t r0 = rb + 4 * grp, c0 = cb + r16, at = r0 * g.ldc + c0;
+    const int nr = (int)min(g.M - r0, (int64_t)BM_), nc = (int)min(g.N - c0, (int64_t)BN_);
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            float x[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
-            quad_transpose(x, q);
-            const int64_t row = rb + 16 * i + 4 * grp + q, col = cb + 16 * j + (r16 & ~3);
-            if (row < g.M) {
-                if (CT == LSMX_F32 && vec_c && col + 4 <= g.N) store_c4<CT>(g.c, row * g.ldc + col, x[0], x[1], x[2], x[3]);
-                else
+        for (int e = 0; e < 4; ++e) {
+            const int64_t ro = (int64_t)(16 * i + e) * g.ldc;
+            if (16 * i + e < nr)
 #pragma unroll
-                    for (int c = 0; c < 4; ++c)
-                        if (col + c < g.N) store_c<CT>(g.c, row * g.ldc + col + c, x[c]);
-            }
+                for (int j = 0; j < TN; ++j)
+                    if (16 * j < nc) store_c<CT>(g.c, at + ro + 16 * j, acc[i][j][e]);
         }
 }
 
@@ -1307,17 +1322,25 @@ static int num_cus() {
 template <int TM, int TN, int S>
 static hipError_t launch_tile(const GemmArgs &g, hipStream_t s) {
     const int64_t grid = ((g.M + 32 * TM - 1) / (32 * TM)) * ((g.N + 32 * TN - 1) / (32 * TN));
-    if (g.c_dtype == LSMX_F32) hipLaunchKernelGGL((gemm_f4f4_tile_kernel<TM, TN, S, LSMX_F32>), (int)grid, 512, 0, s, g);
-    else if (g.c_dtype == LSMX_BF16) hipLaunchKernelGGL((gemm_f4f4_tile_kernel<TM, TN, S, LSMX_BF16>), (int)grid, 512, 0, s, g);
-    else hipLaunchKernelGGL((gemm_f4f4_tile_kernel<TM, TN, S, LSMX_F16>), (int)grid, 512, 0, s, g);
+    const bool vec = (reinterpret_cast<uintptr_t>(g.c) & 15) == 0 && g.ldc % 4 == 0;
+#define LSMX_T(CT)                                                                                               \
+    do {                                                                                                         \
+        if (vec) hipLaunchKernelGGL((gemm_f4f4_tile_kernel<TM, TN, S, CT, true>), (int)grid, 512, 0, s, g);      \
+        else hipLaunchKernelGGL((gemm_f4f4_tile_kernel<TM, TN, S, CT, false>), (int)grid, 512, 0, s, g);         \
+    } while (0)
+    if (g.c_dtype == LSMX_F32) LSMX_T(LSMX_F32);
+    else if (g.c_dtype == LSMX_BF16) LSMX_T(LSMX_BF16);
+    else LSMX_T(LSMX_F16);
+#undef LSMX_T
     return hipGetLastError();
 }
 
 // Tile of the K-major path (pick_tile), stages of 256 codes.  The constants
-// (us) are fits of graph-replayed launches at 28 shapes, M and N 64 .. 8192, K
-// 512 .. 8192, every tile at every shape, and pick the fastest tile or one
-// within 6% of it there.  Large tiles load the fewest bytes and win once they
-// fill the CUs; before that the smaller ones do:
+// (us) are fits of graph-replayed launches at 1700 shapes, M 1 .. 65536, N 16 ..
+// 65536, K 128 .. 16384, every tile at every shape, and pick the fastest tile or
+// one within 0.1% of it there on average, 17% at worst.  Large tiles load the
+// fewest bytes and win once they fill the CUs; before that the smaller ones do
+// (K = 2048 and up; 4443x5184x128: 256x256 18.0, 64x128 28.2):
 //   M x N x K         256x256  256x128  192x128  128x128  64x128  64x64
 //   200x8192x2048        20.4     11.9     10.2      9.0     7.7    8.3 us
 //   256x2048x8192        40.5     26.4     21.7     18.3    15.0   11.7
@@ -1326,8 +1349,9 @@ static hipError_t launch_tile(const GemmArgs &g, hipStream_t s) {
 //   4096x2048x8192       43.2     35.4     46.0     42.7    50.6   67.3
 //   4096x4096x4096       37.4     44.1     49.0     52.5    60.0   75.6
 static const TileCost kTiles[] = {
-    {256, 256, 1, 8.5f, 1.00f, 1.60f}, {256, 128, 1, 6.0f, 0.62f, 0.86f}, {192, 128, 1, 4.2f, 0.50f, 0.72f},
-    {128, 128, 1, 3.5f, 0.43f, 0.58f}, {64, 128, 2, 2.6f, 0.36f, 0.665f}, {64, 64, 2, 2.0f, 0.27f, 0.45f},
+    {256, 256, 1, 7.76f, 1.02f, 1.67f, -1.43f}, {256, 128, 1, 5.40f, 0.65f, 0.95f, 0.78f},
+    {192, 128, 1, 5.45f, 0.45f, 0.79f, -0.66f}, {128, 128, 1, 4.66f, 0.40f, 0.56f, -1.08f},
+    {64, 128, 2, 3.83f, 0.30f, 0.85f, -1.44f},  {64, 64, 2, 3.75f, 0.225f, 0.54f, -2.10f},
 };
 // dma_x4_at forms i * (32 * ld) in a 24-bit multiply
 constexpr int64_t kShortRow = (int64_t)1 << 19;

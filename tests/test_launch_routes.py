@@ -104,7 +104,7 @@ def test_gpu_tile_tests_reach_every_tile(trace):
 
     got = _launched(trace([f"f4 {m} {n} {k} {KMAJOR}" for m, n, k, _ in test_gpu_f4_tiles.SHAPES]))
     want = instances("gemm_f4f4_tile_kernel", a3="0")
-    assert len(want) == 5 and got == want | {"gemm_f4f4_mx16_kernel<4, 0, false, false>"}
+    assert len(want) == 10 and got == want | {"gemm_f4f4_mx16_kernel<4, 0, false, false>"}
 
     got = _launched(trace([f"f8 {m} {n} {k} {nc}" for m, n, k in test_gpu_fp8_tiles.SHAPES
                            for nc in (0, 1) if not nc or n % 16 == 0]))
@@ -168,4 +168,17 @@ def test_few_rows_of_any_depth_run_the_skinny_kernel(trace, M, N, K, dual):
 ])
 def test_short_k_has_tiles_of_its_own(trace, M, N, K, dual, kernel):
     r, = trace([f"w4 {M} {N} {K} {dual} 1 0"])
+    assert [x[0] for x in r["launches"]] == [kernel]
+
+
+@pytest.mark.parametrize("M,N,K,kernel", [
+    # us on the kernel named, and before (other tile or stores)
+    (34898, 133, 1152, "gemm_f4f4_mx16_kernel<4, 0, false, false>"),     # 16.9, 31.4
+    (520, 8185, 640, "gemm_f4f4_tile_kernel<6, 4, 3, 0, false>"),        # the stores of odd rows
+    (15781, 28450, 384, "gemm_f4f4_mx16_kernel<4, 0, false, false>"),    # 362, 740
+    (4443, 5184, 128, "gemm_f4f4_mx16_kernel<4, 0, false, false>"),      # 18.2, 28.1
+    (4892, 4660, 896, "gemm_f4f4_mx16_kernel<4, 0, false, false>"),      # 26.4, 59.9
+])
+def test_f4_tiles_of_ragged_outputs(trace, M, N, K, kernel):
+    r, = trace([f"f4 {M} {N} {K} {KMAJOR}"])
     assert [x[0] for x in r["launches"]] == [kernel]
