@@ -594,8 +594,9 @@ bool dense_ring_ok(const DenseArgs &g, int dtype) {
 }
 
 // Output tile (pick_tile), stages of 64 elements.  The constants (us) are fits
-// of graph-replayed launches of every tile at 17 shapes, M and N 64 .. 4096,
-// K 1024 .. 8192, one and two problems:
+// of graph-replayed launches of every tile at 1300 shapes, M 1 .. 32768, N 8 ..
+// 32768, K 64 .. 16384, one and two problems, and pick the fastest tile or one
+// within 0.9% of it on average:
 //   M x N x K (products)   256x256  256x128  192x128  128x128  64x128  64x64
 //   512x512x4096     (1)      68.9     38.8     33.0     26.7    21.5   18.0 us
 //   1024x1024x4096   (2)      70.1     42.2     36.1     29.1    25.7   34.4
@@ -604,8 +605,9 @@ bool dense_ring_ok(const DenseArgs &g, int dtype) {
 //   2048x2048x8192   (2)     185.3    127.4    160.6    163.8   216.2  264.1
 //   4096x4096x4096   (1)     116.8    124.9    140.8    163.1   183.2  226.8
 static const TileCost kTiles[] = {
-    {256, 256, 1, 8.5f, 0.95f, 1.68f}, {256, 128, 1, 5.5f, 0.55f, 0.93f}, {192, 128, 1, 4.2f, 0.46f, 0.80f},
-    {128, 128, 1, 3.5f, 0.33f, 0.61f}, {64, 128, 2, 3.0f, 0.32f, 0.74f},  {64, 64, 2, 2.5f, 0.26f, 0.48f},
+    {256, 256, 1, 8.56f, 0.90f, 1.68f}, {256, 128, 1, 5.28f, 0.535f, 0.92f, 0.63f},
+    {192, 128, 1, 4.20f, 0.41f, 0.79f}, {128, 128, 1, 3.71f, 0.27f, 0.54f},
+    {64, 128, 2, 3.00f, 0.315f, 0.76f, -0.10f}, {64, 64, 2, 2.88f, 0.26f, 0.49f, -1.03f},
 };
 
 template <int TM, int TN, int S>

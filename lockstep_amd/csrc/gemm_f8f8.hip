@@ -561,8 +561,9 @@ static int num_cus_f8() {
 }
 
 // Output tile (pick_tile), stages of 128 elements.  The constants (us) are fits
-// of graph-replayed launches of every tile at 18 shapes, M and N 64 .. 8192,
-// K 1024 .. 8192, B N-contiguous:
+// of graph-replayed launches of every tile at 900 shapes, M 1 .. 32768, N 16 ..
+// 32768, K 128 .. 12288, B N-contiguous, and pick the fastest tile or one within
+// 0.8% of it on average:
 //   M x N x K         256x256  256x128  192x128  128x128  64x128  64x64
 //   64x4096x2048         32.1     15.3     12.9     10.4     8.2    7.2 us
 //   1024x1024x4096       55.0     26.8     22.1     18.0    14.1   13.8
@@ -571,8 +572,9 @@ static int num_cus_f8() {
 //   4096x2048x4096       54.2     35.6     45.4     42.1    48.8   72.2
 //   4096x4096x4096       61.9     66.4     75.9     77.3    90.8  135.3
 static const TileCost kTiles[] = {
-    {256, 256, 1, 11.0f, 1.30f, 1.58f}, {256, 128, 1, 6.0f, 0.60f, 0.93f}, {192, 128, 1, 5.0f, 0.48f, 0.78f},
-    {128, 128, 1, 4.0f, 0.40f, 0.56f},  {64, 128, 2, 3.0f, 0.34f, 0.72f},  {64, 64, 2, 2.5f, 0.31f, 0.55f},
+    {256, 256, 1, 13.6f, 1.21f, 1.78f, -3.26f}, {256, 128, 1, 6.12f, 0.56f, 0.99f, 0.88f},
+    {192, 128, 1, 5.45f, 0.44f, 0.80f, 0.92f},  {128, 128, 1, 4.47f, 0.315f, 0.67f, -0.30f},
+    {64, 128, 2, 3.57f, 0.28f, 0.85f, -0.28f},  {64, 64, 2, 3.26f, 0.23f, 0.595f, -0.73f},
 };
 
 template <int TM, int TN, int S>

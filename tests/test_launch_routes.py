@@ -182,3 +182,15 @@ def test_short_k_has_tiles_of_its_own(trace, M, N, K, dual, kernel):
 def test_f4_tiles_of_ragged_outputs(trace, M, N, K, kernel):
     r, = trace([f"f4 {M} {N} {K} {KMAJOR}"])
     assert [x[0] for x in r["launches"]] == [kernel]
+
+
+@pytest.mark.parametrize("cmd,kernel", [
+    # us on the kernel named, and on the one that took the shape in between
+    ("dense 940 4256 960 1 2 1", "gemm_dense_tile_kernel<1, 2, true, 3, 2, 4>"),   # 32.3, 39.3
+    ("dense 22565 1312 448 1 2 1", "gemm_dense_ring_kernel<1, 2, true>"),          # 96.8, 110
+    ("f8 290 25088 4096 1", "gemm_f8f8_tile_kernel<0, true, 3, 2, 3>"),            # 46.2, 79.2
+    ("f8 3618 14688 768 1", "gemm_f8f8_kernel<0, true>"),                          # 80.2, 92.4
+])
+def test_dense_and_e4m3_tiles_past_one_round(trace, cmd, kernel):
+    r, = trace([cmd])
+    assert [x[0] for x in r["launches"]] == [kernel]
