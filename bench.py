@@ -578,9 +578,7 @@ def run_configs(torch, dev, deferred=None):
         fl = 2.0 * M * 14336 * 4096
         by = 14336 * 4096 * (0.5 + 1 / 32) + 2 * M * 4096 + 2 * M * 14336
         kern = ("gemv_bf16f4_kernel" if M <= 1 else "gemm_bf16f4_decode_kernel" if M <= 16 else
-                "gemm_bf16f4_skinny_kernel" if M <= 32 else
-                "gemm_bf16f4_ring_kernel (split-K) + splitk_reduce_kernel" if M <= 256 else
-                "gemm_bf16f4_ring_kernel")
+                "gemm_bf16f4_ring_kernel" if M == 1024 else "gemm_bf16f4_tile_kernel")
         if M <= 16:
             rl = roofline("hbm", kern, by / ms / 1e6, PEAK_HBM_GBS, "GB/s")
         else:
