@@ -188,7 +188,7 @@ _captured: list = []
 
 
 def workspace(device: torch.device, nbytes: int) -> torch.Tensor:
-    """A device workspace of at least nbytes for the split-K GEMMs.
+    """A device workspace of at least nbytes for the K slices of a GEMM.
 
     Eager calls share one per (device, stream): calls on one stream are
     ordered, those of several host threads included (the library enqueues the

@@ -19,10 +19,12 @@
 // stage: the A operand for step s reads A[row][32h + 8s .. +8].  A and W use
 // the same assignment, so the sum is unchanged.
 //
-// Tiling: 256 "A rows" x 256 weight columns per workgroup of 4 waves (2 x 2),
-// 128 x 128 per wave (4 x 4 MFMA tiles).  In dual mode the 256 A rows are
-// 128 rows of A0 followed by the same 128 rows of A1: one weight tile in LDS
-// feeds both batches and is read from memory once per stage.
+// Kernels, by the rules at launch_gemm_bf16f4: GEMV (1 row), decode and skinny
+// (up to 32), tile and ring (E8M0 scales), gemm_bf16f4_kernel (what is left),
+// gemm_xf4_kernel (fp32 / fp16 activations).  In the dual form of the ring
+// kernel and gemm_bf16f4_kernel half of a tile's A rows are rows of A0 and half
+// the same rows of A1: one weight tile in LDS feeds both batches and is read
+// from memory once per stage.
 #include <mutex>
 
 #include "lsmx_dma.h"

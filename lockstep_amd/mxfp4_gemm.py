@@ -205,7 +205,7 @@ def _wscales(s: torch.Tensor, rows: int, nkb: int) -> torch.Tensor:
     with 16-byte aligned rows: fp32 powers of two are converted on the device
     (a non-power of two becomes E8M0 NaN, as the kernels' own fp32 path
     treats it), so that fp32 and E8M0 forms of one weight run the same
-    kernels -- the ring and split-K kernels read E8M0 rows -- and give the
+    kernels -- the tile and ring kernels read E8M0 rows -- and give the
     same bits."""
     s = _scales(s, rows, nkb)
     if s.dtype == torch.float32:
