@@ -1575,8 +1575,8 @@ constexpr int lds(int bm, int bn, int s) { return s * (bm * A_ROW_B + bn * W_ROW
 // two workgroups per CU where the LDS holds both rings
 constexpr int waves_per_simd(int bm, int bn, int s, int waves) { return waves / 4 * (2 * lds(bm, bn, s) <= 160 * 1024 ? 2 : 1); }
 }  // namespace wt
-// VEC: C rows start at multiples of 16 bytes and their length is a multiple of
-// 4 elements.
+// VEC: C starts at a multiple of 16 bytes, its rows at multiples of 4 elements
+// (8 bytes of a 16-bit output, the width of its stores).
 template <int CT, bool SPLITK, int WM, int WN, int TM, int TN, int S, int LA, bool VEC>
 __global__ __launch_bounds__(64 * (WM * WN + wt::NLW), wt::waves_per_simd(32 * TM * WM, 32 * TN * WN, S, WM * WN + wt::NLW))
 void gemm_bf16f4_tile_kernel(GemmArgs g) {

@@ -1064,8 +1064,8 @@ __global__ __launch_bounds__(512, 1) void gemm_f4f4_mx16_kernel(GemmArgs g) {
 constexpr int f4_tile_lds(int tm, int tn, int s) {
     return s * ((tm + tn) * 32 * 128 + 2 * (((tm + 1) / 2) * 256 + 64 + ((tn + 1) / 2) * 256 + 64));
 }
-// VEC: C rows start at multiples of 16 bytes and their length is a multiple of
-// 4 elements.
+// VEC: C starts at a multiple of 16 bytes, its rows at multiples of 4 elements
+// (rows of 16-bit outputs at 8 bytes, where a 16-byte store may start too).
 template <int TM, int TN, int S, int CT, bool VEC>
 __global__ __launch_bounds__(512, 2) void gemm_f4f4_tile_kernel(GemmArgs g) {
     using namespace f4;
